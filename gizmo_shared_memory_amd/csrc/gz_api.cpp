@@ -106,7 +106,7 @@ gz_status walk(gz_ctx* ctx, const gz_tree* tree, const gz_particles* p, const ui
                  o_gseg = c.add<int>(ex.nseg > 1 ? n_t : 1), o_mflag = c.add<uint32_t>(n_t),
                  o_mid = c.add<uint32_t>(n_t), o_gstart2 = c.add<int>(n_t + 1),
                  o_scale = c.add<float>(ex.model ? n_t : 1), o_tslot = c.add<int>(n_t),
-                 o_misc = c.add<long long>(16),
+                 o_misc = c.add<long long>(16 + gz::kQueueInts / 2),
                  o_lgroup = c.add<int>(group_size > 0 ? (size_t)std::max(tree->nnodes, 1) : 1),
                  o_tmp = c.add<uint8_t>(gz::scan_tmp_bytes(n_t));
     gz::DevMem& s = ctx->scratch[5];
@@ -118,13 +118,13 @@ gz_status walk(gz_ctx* ctx, const gz_tree* tree, const gz_particles* p, const ui
     int* gstart = reinterpret_cast<int*>(b + o_gstart);
     long long* misc = reinterpret_cast<long long*>(b + o_misc);
     uint32_t* ngroups_dev = reinterpret_cast<uint32_t*>(misc + 4);
-    int* queue = reinterpret_cast<int*>(misc + 9); // eight ints: misc[9..12]
+    int* queue = reinterpret_cast<int*>(misc + 16); // kQueueInts ints
     int* status = reinterpret_cast<int*>(misc + 6);
     int* n_retry = reinterpret_cast<int*>(misc + 7);
     int* retry_list = reinterpret_cast<int*>(b + o_retry);
 
     GZ_HIP(hipEventRecord(ev[8], st));
-    GZ_TRY(gz::fill_zero_u32(reinterpret_cast<uint32_t*>(misc), 32, st));
+    GZ_TRY(gz::fill_zero_u32(reinterpret_cast<uint32_t*>(misc), 32 + gz::kQueueInts, st));
     int* gseg = ex.nseg > 1 ? reinterpret_cast<int*>(b + o_gseg) : nullptr;
     int* tslot = reinterpret_cast<int*>(b + o_tslot);
     GZ_TRY(gz::launch_group_prep(targets, n_t, tree->rank, tree->orderbuf, tree->n_live,
@@ -165,8 +165,9 @@ gz_status walk(gz_ctx* ctx, const gz_tree* tree, const gz_particles* p, const ui
         gstart = gstart2;
     }
 
-    // counters, queue and status start at zero (a fill kernel rather than a memset node, so the
-    // sequence stays valid under stream capture); misc[14], the packed group count, is kept
+    // counters and status start at zero, as the queue does already (a fill kernel rather than a
+    // memset node, so the sequence stays valid under stream capture); misc[14], the packed group
+    // count, is kept
     GZ_TRY(gz::fill_zero_u32(reinterpret_cast<uint32_t*>(misc), 28, st));
     int* nfb = nullptr;
     if (groups_only) {
@@ -1021,12 +1022,12 @@ gz_status gz_walk_plan_create(gz_ctx* ctx, const gz_tree* tree, const gz_particl
     P->model = model;
     P->stack_limit = opts ? opts->stack_limit : 0;
     P->waves_per_cu = opts ? opts->waves_per_cu : 0;
-    // device memory: group starts (n_t + 1), counters (16 x i64), retry list (n_t), segment
+    // device memory: group starts (n_t + 1), counters (16 x i64) and queue, retry list (n_t), segment
     // offsets, and the global stacks of the re-walk
     P->gstack_cap = std::max(1024, std::min(tree->nnodes, 1 << 18));
     P->retry_waves = 64;
     Carver c;
-    const size_t o_gs = c.add<int>(n_t + 1), o_misc = c.add<long long>(16),
+    const size_t o_gs = c.add<int>(n_t + 1), o_misc = c.add<long long>(16 + gz::kQueueInts / 2),
                  o_rl = c.add<int>(n_t + 1), o_seg = c.add<uint32_t>(n_seg + 2),
                  o_sc = c.add<float>(model ? n_t : 1), o_ts = c.add<int>(n_t),
                  o_stk = c.add<int>((size_t)P->retry_waves * P->gstack_cap);
@@ -1096,7 +1097,7 @@ gz_status gz_walk_plan_launch(gz_ctx* ctx, gz_walk_plan* P, double theta, double
     if (P->n_t == 0) return GZ_OK;
     hipStream_t st = ctx->stream;
     const gz_tree* tree = P->tree;
-    GZ_TRY(gz::fill_zero_u32(reinterpret_cast<uint32_t*>(P->misc), 32, st));
+    GZ_TRY(gz::fill_zero_u32(reinterpret_cast<uint32_t*>(P->misc), 32 + gz::kQueueInts, st));
     gz::WalkArgs a{};
     a.wn = tree->wn;
     a.src = tree->src;
@@ -1118,7 +1119,7 @@ gz_status gz_walk_plan_launch(gz_ctx* ctx, gz_walk_plan* P, double theta, double
     a.persistent = P->persistent;
     a.stack_limit = P->stack_limit;
     a.waves_per_cu = P->waves_per_cu;
-    a.queue = reinterpret_cast<int*>(P->misc + 9); // eight ints: misc[9..12]
+    a.queue = reinterpret_cast<int*>(P->misc + 16);
     a.status = reinterpret_cast<int*>(P->misc + 6);
     a.counts = P->misc;
     a.n_retry = reinterpret_cast<int*>(P->misc + 7);

@@ -43,6 +43,10 @@ struct GroupInfo {
     int tlo, thi;        // target slots [tlo, thi)
 };
 
+// The walk's work counters lie a cache line apart: each is claimed from by the waves of one XCD.
+constexpr int kQueueStride = 32;
+constexpr int kQueueInts = 8 * kQueueStride;
+
 // Everything the walk kernel reads. Passed by value.
 // Per-node reuse state written by the build (tree.h:250-317); vectors are SoA with stride nn.
 struct NodeVel {
@@ -83,7 +87,8 @@ struct WalkArgs {
     const double* nvel;
     const uint32_t* orderbuf;
     int nnodes;
-    int* queue;             // persistent launch: eight work counters, one per XCD (zeroed)
+    int* queue;             // persistent launch: eight work counters, one per XCD, kQueueStride
+                            // apart (zeroed)
     int* status;            // bit 0: a group's global node stack overflowed too
     long long* counts;      // nodes visited, multipole, pairs, max stack depth (COUNT builds)
     int* n_retry;           // groups whose LDS node stack overflowed ...
