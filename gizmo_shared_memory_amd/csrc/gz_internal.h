@@ -168,9 +168,9 @@ size_t scan_tmp_bytes(size_t n);
 gz_status exclusive_scan_u32(const uint32_t* in, uint32_t* out, size_t n, uint32_t* total_dev,
                              void* tmp, hipStream_t st, int* starts = nullptr);
 
-// Stable LSD radix sort of (key, value) pairs by the low `bits` bits of the key, 8 bits per pass,
-// skipping passes whose digit is the same for every key. The *_alt buffers are scratch of the
-// same size; the pointers are swapped so that on return keys/vals hold the sorted pairs.
+// Stable LSD radix sort of (key, value) pairs by the low `bits` bits of the key, 8 bits per pass.
+// The *_alt buffers are scratch of the same size; the pointers are swapped so that on return
+// keys/vals hold the sorted pairs. Enqueues only.
 gz_status radix_sort_pairs(uint64_t*& keys, uint32_t*& vals, uint64_t*& keys_alt,
                            uint32_t*& vals_alt, size_t n, int bits, DevMem& scratch,
                            hipStream_t st);

@@ -1,6 +1,6 @@
 // Device-wide primitives used by the tree build: an exclusive scan and a stable LSD radix sort of
-// (64-bit key, 32-bit value) pairs. Both are memory-bound; tiles are 2048 elements per 256-thread
-// workgroup so one launch has thousands of workgroups at the sizes the tree sees (>= 1M keys).
+// (64-bit key, 32-bit value) pairs. Both are memory-bound at the sizes of large trees (>= 1M
+// keys), where one launch has a thousand workgroups, and bound by their launches below that.
 #include <algorithm>
 #include <cstdarg>
 #include <cstdio>
@@ -179,6 +179,48 @@ __global__ __launch_bounds__(kScanThreads) void k_scan_apply(const uint32_t* in,
     }
 }
 
+// One workgroup scans the whole array: below kScanSmall elements two more launches cost more than
+// the chip's width gains (a level of the tree build, a pass of a small sort).
+constexpr size_t kScanSmall = 16384;
+__global__ __launch_bounds__(1024) void k_scan_small(const uint32_t* in, uint32_t* out, int n,
+                                                     uint32_t* __restrict__ total_out,
+                                                     int* __restrict__ starts) {
+    __shared__ uint32_t s16[16];
+    const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    uint32_t carry = 0;
+    for (int base = 0; base < n; base += 1024 * kScanIpt) {
+        const int i0 = base + threadIdx.x * kScanIpt;
+        uint32_t v[kScanIpt], sum = 0;
+#pragma unroll
+        for (int j = 0; j < kScanIpt; ++j) {
+            v[j] = (i0 + j < n) ? in[i0 + j] : 0u;
+            sum += v[j];
+        }
+        const uint32_t inc = wave_inclusive_scan(sum);
+        if (lane == 63) s16[w] = inc;
+        __syncthreads();
+        uint32_t off = 0, tot = 0;
+#pragma unroll
+        for (int k = 0; k < 16; ++k) {
+            const uint32_t s = s16[k];
+            off += (k < w) ? s : 0u;
+            tot += s;
+        }
+        uint32_t run = carry + off + inc - sum;
+#pragma unroll
+        for (int j = 0; j < kScanIpt; ++j) {
+            if (i0 + j < n) {
+                out[i0 + j] = run;
+                if (starts && v[j]) starts[run] = i0 + j;
+            }
+            run += v[j];
+        }
+        carry += tot;
+        __syncthreads();
+    }
+    if (threadIdx.x == 0 && total_out) *total_out = carry;
+}
+
 size_t scan_tmp_bytes(size_t n) {
     const size_t nb = (n + kScanTile - 1) / kScanTile;
     return (nb + 64) * sizeof(uint32_t);
@@ -188,6 +230,11 @@ gz_status exclusive_scan_u32(const uint32_t* in, uint32_t* out, size_t n, uint32
                              void* tmp, hipStream_t st, int* starts) {
     if (n == 0) {
         if (total_dev) GZ_HIP(hipMemsetAsync(total_dev, 0, sizeof(uint32_t), st));
+        return GZ_OK;
+    }
+    if (n <= kScanSmall) {
+        k_scan_small<<<1, 1024, 0, st>>>(in, out, (int)n, total_dev, starts);
+        GZ_HIP(hipGetLastError());
         return GZ_OK;
     }
     const size_t nb = (n + kScanTile - 1) / kScanTile;
@@ -213,93 +260,138 @@ gz_status fill_zero_u32(uint32_t* a, size_t n, hipStream_t st) {
 }
 
 // ---- radix sort ------------------------------------------------------------------------------
+// Stable LSD passes of 8 bits, each a count of every tile's digits and a scatter. A tile's wave
+// ranks its own contiguous elements against counters of its own (no barrier between them), the
+// tile is put in digit order in LDS, and the runs of equal digits are then written out by
+// neighbouring lanes.
 constexpr int kRsThreads = 256;
-constexpr int kRsIpt = 8;
-constexpr int kRsTile = kRsThreads * kRsIpt;
 constexpr int kRsRadix = 256;
-constexpr int kRsMaxPasses = 8;
+// Tiles: 4096 elements make runs of 16 (128 B of keys) on average; below kRsBig elements smaller
+// tiles keep more of the chip busy, and up to kRsDirect tiles each scatter workgroup adds up the
+// counts of the tiles before it instead of waiting for a scan.
+constexpr size_t kRsBig = size_t(1) << 20;
+constexpr uint32_t kRsDirect = 128;
 
-// Histograms of every 8-bit digit in one read of the keys, so passes whose digit is the same for
-// every key can be skipped.
-__global__ __launch_bounds__(kRsThreads) void k_rs_digit_hist(const uint64_t* __restrict__ keys,
-                                                              size_t n, int npasses,
-                                                              uint32_t* __restrict__ ghist) {
-    __shared__ uint32_t h[kRsMaxPasses * kRsRadix];
-    for (int k = threadIdx.x; k < kRsMaxPasses * kRsRadix; k += kRsThreads) h[k] = 0;
-    __syncthreads();
-    for (size_t i = (size_t)blockIdx.x * kRsThreads + threadIdx.x; i < n;
-         i += (size_t)gridDim.x * kRsThreads) {
-        const uint64_t k = keys[i];
-        for (int p = 0; p < npasses; ++p) atomicAdd(&h[p * kRsRadix + ((k >> (8 * p)) & 255u)], 1u);
-    }
-    __syncthreads();
-    for (int k = threadIdx.x; k < npasses * kRsRadix; k += kRsThreads)
-        if (h[k]) atomicAdd(&ghist[k], h[k]);
-}
-
-// Per-tile digit counts, digit-major: hist[d * nb + b].
+// Digit counts of every tile: hist[d * nb + b], or hist[b * 256 + d] for the direct scatter.
+template <int IPT>
 __global__ __launch_bounds__(kRsThreads) void k_rs_count(const uint64_t* __restrict__ keys,
                                                          size_t n, int shift, uint32_t nb,
+                                                         int direct,
                                                          uint32_t* __restrict__ hist) {
     __shared__ uint32_t c[kRsRadix];
     c[threadIdx.x] = 0;
     __syncthreads();
-    const size_t base = (size_t)blockIdx.x * kRsTile;
+    const size_t base = (size_t)blockIdx.x * (kRsThreads * IPT);
+    uint32_t d[IPT];
 #pragma unroll
-    for (int j = 0; j < kRsIpt; ++j) {
+    for (int j = 0; j < IPT; ++j) {
         const size_t i = base + (size_t)j * kRsThreads + threadIdx.x;
-        if (i < n) atomicAdd(&c[(uint32_t)(keys[i] >> shift) & 255u], 1u);
+        d[j] = (i < n) ? (uint32_t)(keys[i] >> shift) & 255u : 256u;
     }
+#pragma unroll
+    for (int j = 0; j < IPT; ++j)
+        if (d[j] < 256u) atomicAdd(&c[d[j]], 1u);
     __syncthreads();
-    hist[(size_t)threadIdx.x * nb + blockIdx.x] = c[threadIdx.x];
+    const size_t at = direct ? (size_t)blockIdx.x * kRsRadix + threadIdx.x
+                             : (size_t)threadIdx.x * nb + blockIdx.x;
+    hist[at] = c[threadIdx.x];
 }
 
-// Stable scatter. Within a tile, an element's rank among equal digits is the number of equal
-// digits at smaller indices: earlier rounds (s_run), earlier waves of this round (s_wcnt) and
-// earlier lanes of this wave (match by 8 ballots).
+template <int IPT>
 __global__ __launch_bounds__(kRsThreads) void k_rs_scatter(
     const uint64_t* __restrict__ kin, const uint32_t* __restrict__ vin,
     uint64_t* __restrict__ kout, uint32_t* __restrict__ vout, size_t n, int shift, uint32_t nb,
-    const uint32_t* __restrict__ offs) {
-    __shared__ uint32_t s_off[kRsRadix];
-    __shared__ uint32_t s_run[kRsRadix];
-    __shared__ uint32_t s_wcnt[4][kRsRadix];
+    int direct, const uint32_t* __restrict__ offs) {
+    constexpr int kTile = kRsThreads * IPT;
+    __shared__ uint64_t s_key[kTile];
+    __shared__ uint32_t s_val[kTile];
+    __shared__ uint32_t s_cnt[4][kRsRadix]; // a wave's count so far, then its first place
+    __shared__ uint32_t s_goff[kRsRadix];   // output place of a digit's run, less its place here
+    __shared__ uint32_t s4[4];
     const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63;
-    s_off[tid] = offs[(size_t)tid * nb + blockIdx.x];
-    s_run[tid] = 0;
-    const uint64_t below_mask = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
-    const size_t base = (size_t)blockIdx.x * kRsTile;
-    for (int j = 0; j < kRsIpt; ++j) {
-        const size_t i = base + (size_t)j * kRsThreads + tid;
-        const bool valid = i < n;
-        uint64_t key = 0;
-        uint32_t val = 0, d = 0;
-        if (valid) {
-            key = kin[i];
-            val = vin[i];
-            d = (uint32_t)(key >> shift) & 255u;
+    const size_t base = (size_t)blockIdx.x * kTile;
+    const int count = (int)((n - base < (size_t)kTile) ? n - base : (size_t)kTile);
+    // element (w, j, lane) of the tile: the input order is w, then j, then lane
+    uint64_t key[IPT];
+    uint32_t val[IPT], rank[IPT];
+#pragma unroll
+    for (int j = 0; j < IPT; ++j) {
+        const int e = (w * IPT + j) * kWave + lane;
+        key[j] = 0;
+        val[j] = 0;
+        if (e < count) {
+            key[j] = kin[base + e];
+            val[j] = vin[base + e];
         }
+    }
+    // where this tile's digits go: thread d's digit, after the lower digits of all tiles and its
+    // own digit of the tiles before
+    uint32_t gplace, total;
+    if (direct) {
+        uint32_t before = 0, all = 0;
+        for (uint32_t b = 0; b < nb; ++b) {
+            const uint32_t c = offs[(size_t)b * kRsRadix + tid];
+            before += (b < blockIdx.x) ? c : 0u;
+            all += c;
+        }
+        gplace = block256_exclusive_scan(all, s4, total) + before;
+    } else {
+        gplace = offs[(size_t)tid * nb + blockIdx.x];
+    }
+    for (int k = lane; k < kRsRadix; k += kWave) s_cnt[w][k] = 0;
+    __syncthreads();
+    const uint64_t below_mask = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
+#pragma unroll
+    for (int j = 0; j < IPT; ++j) {
+        const bool valid = (w * IPT + j) * kWave + lane < count;
+        const uint32_t d = (uint32_t)(key[j] >> shift) & 255u;
         uint64_t peers = __ballot(valid);
 #pragma unroll
         for (int bit = 0; bit < 8; ++bit) {
             const bool set = (d >> bit) & 1u;
-            const uint64_t b = __ballot(set);
-            peers &= set ? b : ~b;
+            const uint64_t m = __ballot(set);
+            peers &= set ? m : ~m;
         }
-        for (int k = lane; k < kRsRadix; k += kWave) s_wcnt[w][k] = 0;
-        __syncthreads();
         const uint32_t below = (uint32_t)__popcll(peers & below_mask);
-        if (valid && below == 0) s_wcnt[w][d] = (uint32_t)__popcll(peers);
-        __syncthreads();
-        if (valid) {
-            uint32_t pos = s_off[d] + s_run[d] + below;
-            for (int k = 0; k < w; ++k) pos += s_wcnt[k][d];
-            kout[pos] = key;
-            vout[pos] = val;
+        // the wave's own counter: read by every peer, then advanced by the first of them (LDS
+        // accesses of one wave stay in order)
+        volatile uint32_t* c = &s_cnt[w][d];
+        const uint32_t old = *c;
+        __builtin_amdgcn_wave_barrier();
+        if (valid && below == 0) *c = old + (uint32_t)__popcll(peers);
+        __builtin_amdgcn_wave_barrier();
+        rank[j] = old + below;
+    }
+    __syncthreads();
+    uint32_t c[4], mine = 0;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        c[k] = s_cnt[k][tid];
+        mine += c[k];
+    }
+    uint32_t place = block256_exclusive_scan(mine, s4, total);
+    s_goff[tid] = gplace - place;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        s_cnt[k][tid] = place;
+        place += c[k];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < IPT; ++j) {
+        if ((w * IPT + j) * kWave + lane < count) {
+            const uint32_t d = (uint32_t)(key[j] >> shift) & 255u;
+            const uint32_t at = s_cnt[w][d] + rank[j];
+            s_key[at] = key[j];
+            s_val[at] = val[j];
         }
-        __syncthreads();
-        s_run[tid] += s_wcnt[0][tid] + s_wcnt[1][tid] + s_wcnt[2][tid] + s_wcnt[3][tid];
-        __syncthreads();
+    }
+    __syncthreads();
+    for (int e = tid; e < count; e += kRsThreads) {
+        const uint64_t k = s_key[e];
+        const uint32_t pos = s_goff[(uint32_t)(k >> shift) & 255u] + (uint32_t)e;
+        kout[pos] = k;
+        vout[pos] = s_val[e];
     }
 }
 
@@ -308,34 +400,28 @@ gz_status radix_sort_pairs(uint64_t*& keys, uint32_t*& vals, uint64_t*& keys_alt
                            hipStream_t st) {
     if (n <= 1) return GZ_OK;
     if (n >= 0xFFFFFFFFull) return fail(GZ_ERR_INVALID, "radix sort: %zu keys exceed 2^32-1", n);
-    const int npasses = std::min(kRsMaxPasses, (bits + 7) / 8);
-    const uint32_t nb = (uint32_t)((n + kRsTile - 1) / kRsTile);
+    const int npasses = std::min(8, (bits + 7) / 8);
+    const bool big = n >= kRsBig;
+    const size_t tile = (size_t)kRsThreads * (big ? 16 : 8);
+    const uint32_t nb = (uint32_t)((n + tile - 1) / tile);
+    const int direct = nb <= kRsDirect;
     const size_t hist_n = (size_t)kRsRadix * nb;
-    const size_t ghist_bytes = kRsMaxPasses * kRsRadix * sizeof(uint32_t);
-    const size_t need = ghist_bytes + hist_n * sizeof(uint32_t) + scan_tmp_bytes(hist_n) + 256;
-    GZ_TRY(scratch.reserve(need));
-    uint8_t* base = scratch.as<uint8_t>();
-    uint32_t* ghist = reinterpret_cast<uint32_t*>(base);
-    uint32_t* hist = reinterpret_cast<uint32_t*>(base + ghist_bytes);
-    void* scan_tmp = base + ghist_bytes + hist_n * sizeof(uint32_t);
-
-    GZ_HIP(hipMemsetAsync(ghist, 0, ghist_bytes, st));
-    const unsigned hgrid = (unsigned)std::min<size_t>((n + kRsThreads - 1) / kRsThreads, 1024);
-    k_rs_digit_hist<<<hgrid, kRsThreads, 0, st>>>(keys, n, npasses, ghist);
-    GZ_HIP(hipGetLastError());
-    std::vector<uint32_t> h(kRsMaxPasses * kRsRadix);
-    GZ_HIP(hipMemcpyAsync(h.data(), ghist, ghist_bytes, hipMemcpyDeviceToHost, st));
-    GZ_HIP(hipStreamSynchronize(st));
-
+    const size_t hist_bytes = (hist_n * sizeof(uint32_t) + 255) & ~size_t(255);
+    GZ_TRY(scratch.reserve(hist_bytes + scan_tmp_bytes(hist_n) + 256));
+    uint32_t* hist = scratch.as<uint32_t>();
+    void* scan_tmp = scratch.as<uint8_t>() + hist_bytes;
     for (int p = 0; p < npasses; ++p) {
-        const uint32_t* hp = h.data() + p * kRsRadix;
-        if (*std::max_element(hp, hp + kRsRadix) == (uint32_t)n) continue; // one digit: no-op
         const int shift = 8 * p;
-        k_rs_count<<<nb, kRsThreads, 0, st>>>(keys, n, shift, nb, hist);
+        if (big) k_rs_count<16><<<nb, kRsThreads, 0, st>>>(keys, n, shift, nb, direct, hist);
+        else k_rs_count<8><<<nb, kRsThreads, 0, st>>>(keys, n, shift, nb, direct, hist);
         GZ_HIP(hipGetLastError());
-        GZ_TRY(exclusive_scan_u32(hist, hist, hist_n, nullptr, scan_tmp, st));
-        k_rs_scatter<<<nb, kRsThreads, 0, st>>>(keys, vals, keys_alt, vals_alt, n, shift, nb,
-                                                hist);
+        if (!direct) GZ_TRY(exclusive_scan_u32(hist, hist, hist_n, nullptr, scan_tmp, st));
+        if (big)
+            k_rs_scatter<16><<<nb, kRsThreads, 0, st>>>(keys, vals, keys_alt, vals_alt, n, shift,
+                                                        nb, direct, hist);
+        else
+            k_rs_scatter<8><<<nb, kRsThreads, 0, st>>>(keys, vals, keys_alt, vals_alt, n, shift,
+                                                       nb, direct, hist);
         GZ_HIP(hipGetLastError());
         std::swap(keys, keys_alt);
         std::swap(vals, vals_alt);
