@@ -16,10 +16,15 @@
 #include <cstring>
 
 #include "gz_internal.h"
+#include "gz_wave.h"
 
 namespace gz {
 
 constexpr int kThreads = 256;
+// The level table on the device: first nodes of levels 0..kMaxLevel + 2, then the nodes that a
+// level which outgrew the arena would have needed.
+constexpr int kLevNeed = kMaxLevel + 3;
+constexpr int kLevInts = kMaxLevel + 4;
 
 static inline unsigned grid_for(size_t n, int threads = kThreads) {
     return (unsigned)((n + threads - 1) / threads);
@@ -44,11 +49,14 @@ __global__ __launch_bounds__(kThreads) void k_bbox_partial(const double* __restr
                                                            const double* __restrict__ y,
                                                            const double* __restrict__ z,
                                                            const double* __restrict__ m, size_t n,
-                                                           double* __restrict__ partial) {
+                                                           double* __restrict__ partial,
+                                                           uint32_t* __restrict__ live) {
     double lo0 = 1e300, lo1 = 1e300, lo2 = 1e300, hi0 = -1e300, hi1 = -1e300, hi2 = -1e300;
+    uint32_t cnt = 0;
     for (size_t i = (size_t)blockIdx.x * kThreads + threadIdx.x; i < n;
          i += (size_t)gridDim.x * kThreads) {
         if (!(m[i] > 0)) continue;
+        ++cnt;
         const double a = x[i], b = y[i], c = z[i];
         lo0 = dmin_(lo0, a); hi0 = dmax_(hi0, a);
         lo1 = dmin_(lo1, b); hi1 = dmax_(hi1, b);
@@ -68,6 +76,8 @@ __global__ __launch_bounds__(kThreads) void k_bbox_partial(const double* __restr
         for (int j = 1; j < 4; ++j) v = (k < 3) ? dmin_(v, s[j][k]) : dmax_(v, s[j][k]);
         partial[(size_t)blockIdx.x * 6 + k] = v;
     }
+    for (int d = 32; d >= 1; d >>= 1) cnt += __shfl_xor(cnt, d);
+    if (lane == 0) live[(size_t)blockIdx.x * 4 + w] = cnt;
 }
 
 // splitmix64 draw in [0,1) for RANDOMIZE_GRAVTREE (tree.cc:381-393)
@@ -78,16 +88,45 @@ __device__ double splitmix_unit(uint64_t& s) {
     return (double)((z ^ (z >> 31)) >> 11) * (1.0 / 9007199254740992.0);
 }
 
-// root[0..3] = centre x, y, z and side; root[4..9] = live bounding box lo, hi.
-__global__ void k_root_cell(const double* __restrict__ partial, int nb, long long seed, double fx,
-                            double fy, double fz, double* __restrict__ root) {
-    if (threadIdx.x != 0 || blockIdx.x != 0) return;
+// root[0..3] = centre x, y, z and side; root[4..9] = live bounding box lo, hi; root[10] = the live
+// particles. One workgroup (one thread took 270 us over the 1024 partial boxes of a 4M build).
+__global__ __launch_bounds__(kThreads) void k_root_cell(const double* __restrict__ partial,
+                                                        const uint32_t* __restrict__ live, int nb,
+                                                        long long seed, double fx, double fy,
+                                                        double fz, double* __restrict__ root) {
     double lo[3] = {1e300, 1e300, 1e300}, hi[3] = {-1e300, -1e300, -1e300};
-    for (int b = 0; b < nb; ++b)
+    uint32_t cnt = 0;
+    for (int b = threadIdx.x; b < nb; b += kThreads)
         for (int k = 0; k < 3; ++k) {
             lo[k] = dmin_(lo[k], partial[(size_t)b * 6 + k]);
             hi[k] = dmax_(hi[k], partial[(size_t)b * 6 + 3 + k]);
         }
+    for (int b = threadIdx.x; b < 4 * nb; b += kThreads) cnt += live[b];
+    __shared__ double s[4][6];
+    __shared__ uint32_t sc[4];
+    const int w = threadIdx.x >> 6;
+    for (int d = 32; d >= 1; d >>= 1) cnt += __shfl_xor(cnt, d);
+    for (int k = 0; k < 3; ++k) {
+        lo[k] = wave_min(lo[k]);
+        hi[k] = wave_max(hi[k]);
+    }
+    if ((threadIdx.x & 63) == 0) {
+        for (int k = 0; k < 3; ++k) {
+            s[w][k] = lo[k];
+            s[w][3 + k] = hi[k];
+        }
+        sc[w] = cnt;
+    }
+    __syncthreads();
+    if (threadIdx.x != 0) return;
+    for (int j = 1; j < 4; ++j) {
+        for (int k = 0; k < 3; ++k) {
+            lo[k] = dmin_(lo[k], s[j][k]);
+            hi[k] = dmax_(hi[k], s[j][3 + k]);
+        }
+        cnt += sc[j];
+    }
+    root[10] = (double)cnt;
     double cx = 0.5 * (lo[0] + hi[0]), cy = 0.5 * (lo[1] + hi[1]), cz = 0.5 * (lo[2] + hi[2]);
     double side = dmax_(hi[0] - lo[0], dmax_(hi[1] - lo[1], hi[2] - lo[2])) * 1.0000001;
     if (side <= 0) side = 1.0;
@@ -180,9 +219,14 @@ __global__ __launch_bounds__(kThreads) void k_init_roots(int nc, const double* _
                                                          const int* __restrict__ rstart, int* nlo,
                                                          int* nhi, double* gcx, double* gcy,
                                                          double* gcz, double* size, int* parent,
-                                                         int* next) {
+                                                         int* next, int* lev) {
     const int c = blockIdx.x * kThreads + threadIdx.x;
     if (c >= nc) return;
+    if (c == 0) {
+        lev[0] = 0;
+        lev[1] = nc;
+        lev[kLevNeed] = 0;
+    }
     nlo[c] = rstart[c];
     nhi[c] = rstart[c + 1];
     gcx[c] = roots[4 * c];
@@ -223,32 +267,102 @@ __global__ __launch_bounds__(kThreads) void k_keys(const uint32_t* __restrict__ 
                                                    const double* __restrict__ z,
                                                    const double* __restrict__ roots,
                                                    const uint32_t* __restrict__ cstart, int nc,
-                                                   uint64_t* __restrict__ keys) {
+                                                   uint64_t* __restrict__ keys,
+                                                   uint32_t* __restrict__ vals) {
     const size_t r = (size_t)blockIdx.x * kThreads + threadIdx.x;
     if (r >= nl) return;
-    const double* root = roots + (nc > 1 ? (size_t)cluster_of(order[r], cstart, nc) * 4 : 0);
+    const uint32_t i = order ? order[r] : (uint32_t)r;
+    if (!order) vals[r] = i;
+    const double* root = roots + (nc > 1 ? (size_t)cluster_of(i, cstart, nc) * 4 : 0);
     const double side = root[3];
     const double scale = (double)((1u << kMaxLevel) - 1) / side;
     const double bx = root[0] - 0.5 * side, by = root[1] - 0.5 * side, bz = root[2] - 0.5 * side;
-    const uint32_t i = order[r];
     const uint32_t a = (uint32_t)((x[i] - bx) * scale);
     const uint32_t b = (uint32_t)((y[i] - by) * scale);
     const uint32_t c = (uint32_t)((z[i] - bz) * scale);
     keys[r] = spread3(a) | (spread3(b) << 1) | (spread3(c) << 2);
 }
 
-// Sorted copy of the source data, and the inverse permutation (tree.cc:483-485).
+// One particle's sources in a line of their own.
+struct alignas(64) PRec {
+    double x, y, z, m, soft, pad[3];
+};
+
+// Sorted copy of the source data (tree.cc:483-485). The particles are read in random order: from
+// the caller's arrays that is five partly used lines each, 470 us for 4M particles and bound by
+// them. Large sets are therefore first packed to a line per particle (k_pack_rec, a streaming
+// pass), which the gather then reads whole: 4M together 235 us. Below kPackRec particles the
+// arrays stay in cache and the direct gather is as fast with a launch less.
+constexpr size_t kPackRec = size_t(1) << 19;
+__global__ __launch_bounds__(kThreads) void k_pack_rec(size_t n, const double* __restrict__ x,
+                                                       const double* __restrict__ y,
+                                                       const double* __restrict__ z,
+                                                       const double* __restrict__ m,
+                                                       const double* __restrict__ soft,
+                                                       PRec* __restrict__ rec) {
+    const size_t i = (size_t)blockIdx.x * kThreads + threadIdx.x;
+    if (i >= n) return;
+    double4* o = reinterpret_cast<double4*>(rec + i);
+    o[0] = make_double4(x[i], y[i], z[i], m[i]);
+    o[1] = make_double4(soft ? soft[i] : 0.0, 0.0, 0.0, 0.0);
+}
+
+__global__ __launch_bounds__(kThreads) void k_gather_rec(const uint32_t* __restrict__ orderbuf,
+                                                         size_t nl, const PRec* __restrict__ rec,
+                                                         double4* __restrict__ src,
+                                                         double* __restrict__ src_soft) {
+    const size_t r = (size_t)blockIdx.x * kThreads + threadIdx.x;
+    if (r >= nl) return;
+    const double4* p = reinterpret_cast<const double4*>(rec + orderbuf[r]);
+    const double4 q = p[0];
+    const double s = p[1].x;
+    src[r] = q;
+    src_soft[r] = s;
+}
+
 __global__ __launch_bounds__(kThreads) void k_gather_sorted(
     const uint32_t* __restrict__ orderbuf, size_t nl, const double* __restrict__ x,
     const double* __restrict__ y, const double* __restrict__ z, const double* __restrict__ m,
-    const double* __restrict__ soft, double4* __restrict__ src, double* __restrict__ src_soft,
-    uint32_t* __restrict__ rank) {
+    const double* __restrict__ soft, double4* __restrict__ src, double* __restrict__ src_soft) {
     const size_t r = (size_t)blockIdx.x * kThreads + threadIdx.x;
     if (r >= nl) return;
     const uint32_t p = orderbuf[r];
     src[r] = make_double4(x[p], y[p], z[p], m[p]);
     src_soft[r] = soft ? soft[p] : 0.0;
+}
+
+// grow: the records' memory may be allocated (else they are used only if there is room already).
+static gz_status gather_sources(const gz_particles* p, const uint32_t* orderbuf, size_t nl,
+                                double4* src, double* src_soft, DevMem& mem, bool grow,
+                                hipStream_t st) {
+    if (nl == 0) return GZ_OK;
+    const size_t rec_bytes = p->n * sizeof(PRec);
+    // (packing the dead particles of a set that is mostly dead would cost more than it saves)
+    if (nl >= kPackRec && nl >= p->n / 2 && (grow || mem.bytes >= rec_bytes)) {
+        GZ_TRY(mem.reserve(rec_bytes));
+        k_pack_rec<<<grid_for(p->n), kThreads, 0, st>>>(p->n, p->x, p->y, p->z, p->m, p->soft,
+                                                        mem.as<PRec>());
+        k_gather_rec<<<grid_for(nl), kThreads, 0, st>>>(orderbuf, nl, mem.as<PRec>(), src,
+                                                        src_soft);
+    } else {
+        k_gather_sorted<<<grid_for(nl), kThreads, 0, st>>>(orderbuf, nl, p->x, p->y, p->z, p->m,
+                                                           p->soft, src, src_soft);
+    }
+    GZ_HIP(hipGetLastError());
+    return GZ_OK;
+}
+
+// The inverse permutation and each particle's leaf, from the sorted side.
+__global__ __launch_bounds__(kThreads) void k_particle_links(const uint32_t* __restrict__ orderbuf,
+                                                             const int* __restrict__ slot_leaf,
+                                                             size_t nl,
+                                                             uint32_t* __restrict__ rank,
+                                                             int* __restrict__ leaf_of) {
+    const size_t r = (size_t)blockIdx.x * kThreads + threadIdx.x;
+    if (r >= nl) return;
+    const uint32_t p = orderbuf[r];
     rank[p] = (uint32_t)r;
+    leaf_of[p] = slot_leaf[r];
 }
 
 // Sorted copy of the build-time velocities.
@@ -271,7 +385,10 @@ __global__ __launch_bounds__(kThreads) void k_fill_u32(uint32_t* __restrict__ a,
 
 __global__ void k_init_root(const double* __restrict__ root, int nl, int* nlo, int* nhi,
                             double* gcx, double* gcy, double* gcz, double* size, int* parent,
-                            int* next) {
+                            int* next, int* lev) {
+    lev[0] = 0;
+    lev[1] = 1;
+    lev[kLevNeed] = 0;
     nlo[0] = 0;
     nhi[0] = nl;
     gcx[0] = root[0];
@@ -282,87 +399,181 @@ __global__ void k_init_root(const double* __restrict__ root, int nl, int* nlo, i
     next[0] = -1;
 }
 
-// ---- topology, one level per launch (tree.cc:86-143) -------------------------------------------
-// For each node of the level: leaf test, then the start of each octant's run of keys by binary
-// search on the 3-bit digit (keys in a node share every higher digit, so the digit is sorted).
-__global__ __launch_bounds__(kThreads) void k_split(int lb, int count, int level,
+// ---- topology, two launches per level (tree.cc:86-143) ------------------------------------------
+// The level table lev (node ids [lev[L], lev[L+1]) are level L) is kept on the device, so levels
+// are enqueued without the host reading a count back in between (16 read-backs of 20 us in a 4M
+// build); launches are sized by an upper bound and step over the nodes there are.
+constexpr int kLevelChunk = 64; // nodes whose children k_split counts together
+
+// Each node of the level: leaf test, then the start of each octant's run of keys (keys in a node
+// share every higher digit, so the 3-bit digit is sorted). Eight lanes take one node, lane o
+// finding octant o by binary search; with WIDE a wave takes one node, eight lanes to an octant,
+// each step probing eight places at once, for the few nodes of the top levels, whose searches
+// would otherwise be 22 dependent loads long (65 us a level at 4M particles by one thread a node).
+template <bool WIDE>
+__global__ __launch_bounds__(kThreads) void k_split(int level, const int* __restrict__ lev,
                                                     const int* __restrict__ nlo,
                                                     const int* __restrict__ nhi,
                                                     const uint64_t* __restrict__ skey,
                                                     int* __restrict__ oct_start,
-                                                    uint32_t* __restrict__ nkids) {
-    const int i = blockIdx.x * kThreads + threadIdx.x;
-    if (i >= count) return;
-    const int node = lb + i;
-    const int lo = nlo[node], hi = nhi[node];
-    if ((hi - lo <= kLeafMax) || (level >= kMaxLevel)) {
-        nkids[i] = 0;
-        return;
-    }
-    const int shift = 3 * (kMaxLevel - level - 1);
-    int* os = oct_start + (size_t)i * 8;
-    os[0] = lo;
-    int a = lo;
-    for (int o = 1; o < 8; ++o) {
-        int b = hi;
-        while (a < b) { // first index in [a, hi) with digit >= o
-            const int mid = a + ((b - a) >> 1);
-            if ((int)((skey[mid] >> shift) & 7ull) < o) a = mid + 1;
-            else b = mid;
+                                                    uint32_t* __restrict__ nkids,
+                                                    uint32_t* __restrict__ chunk_sum) {
+    constexpr int kLanes = WIDE ? 64 : 8;
+    constexpr int kPer = kThreads / kLanes; // nodes a workgroup holds at once
+    __shared__ uint32_t s_sum[kThreads / kWave];
+    const int lb = lev[level], count = lev[level + 1] - lb;
+    const int lane = threadIdx.x & 63;
+    const int o = WIDE ? (lane >> 3) : (threadIdx.x & 7), probe = lane & 7;
+    for (int c0 = blockIdx.x * kLevelChunk; c0 < count; c0 += gridDim.x * kLevelChunk) {
+        uint32_t sum = 0; // children of this wave's nodes
+        for (int k = 0; k < kLevelChunk; k += kPer) {
+            const int i = c0 + k + (int)threadIdx.x / kLanes;
+            const bool live = i < count;
+            int lo = 0, hi = 0;
+            if (live) {
+                lo = nlo[lb + i];
+                hi = nhi[lb + i];
+            }
+            const bool split = hi - lo > kLeafMax && level < kMaxLevel;
+            const int shift = 3 * (kMaxLevel - level - 1);
+            int a = lo, b = hi; // the first index in [lo, hi) with digit >= o, or hi, is in [a, b]
+            if (!split || o == 0) b = a;
+            if (WIDE) {
+                while (__ballot(a < b)) {
+                    // probes cut [a, b) into nine parts; digits ascend, so those below o come first
+                    const int len = b - a;
+                    const int at = a + (int)(((long long)len * (probe + 1)) / 9);
+                    const bool below = a < b && (int)((skey[at] >> shift) & 7ull) < o;
+                    const uint64_t m = (__ballot(below) >> (lane & 56)) & 0xffull;
+                    const int nbelow = __popcll(m);
+                    if (a < b) {
+                        const int na = nbelow ? a + (int)(((long long)len * nbelow) / 9) + 1 : a;
+                        const int nb = nbelow < 8 ? a + (int)(((long long)len * (nbelow + 1)) / 9)
+                                                  : b;
+                        a = na;
+                        b = nb;
+                    }
+                }
+            } else {
+                while (a < b) {
+                    const int mid = a + ((b - a) >> 1);
+                    if ((int)((skey[mid] >> shift) & 7ull) < o) a = mid + 1;
+                    else b = mid;
+                }
+            }
+            int e = __shfl_down(a, WIDE ? 8 : 1); // the next octant's start
+            if (o == 7) e = hi;
+            const uint64_t m = __ballot(split && e > a && (!WIDE || probe == 0));
+            if (split && (!WIDE || probe == 0)) oct_start[(size_t)i * 8 + o] = a;
+            const uint32_t nk = WIDE ? (uint32_t)__popcll(m)
+                                     : (uint32_t)__popcll((m >> (lane & 56)) & 0xffull);
+            if (live && (WIDE ? lane == 0 : o == 0)) nkids[i] = nk;
+            sum += (uint32_t)__popcll(m);
         }
-        os[o] = a;
+        if (lane == 0) s_sum[threadIdx.x >> 6] = sum;
+        __syncthreads();
+        if (threadIdx.x == 0)
+            chunk_sum[c0 / kLevelChunk] = s_sum[0] + s_sum[1] + s_sum[2] + s_sum[3];
+        __syncthreads();
     }
-    uint32_t nk = 0;
-    for (int o = 0; o < 8; ++o) {
-        const int e = (o < 7) ? os[o + 1] : hi;
-        nk += (e > os[o]) ? 1u : 0u;
-    }
-    nkids[i] = nk;
 }
 
-// Allocate each node's children at next_lb + off[i] in octant order, with the child cell from
-// halving the parent's (tree.cc:101, 116-118) and the threaded successor (tree.cc:340-348): the
-// next sibling, or the parent's successor for the last child.
+// Allocate each node's children after the level's own nodes, by the prefix sum of the counts, in
+// octant order, with the child cell from halving the parent's (tree.cc:101, 116-118) and the
+// threaded successor (tree.cc:340-348): the next sibling, or the parent's successor for the last
+// child. A workgroup adds up the chunk counts before its own. Eight lanes write one node's
+// children, so neighbouring lanes write neighbouring nodes. When the children would outgrow the
+// arena, nothing is emitted, the next level stays empty and lev[kLevNeed] tells the nodes needed.
+constexpr int kEmitChunks = 4; // chunks a workgroup emits at a time
 __global__ __launch_bounds__(kThreads) void k_emit(
-    int lb, int count, int next_lb, const uint32_t* __restrict__ nkids,
-    const uint32_t* __restrict__ off, const int* __restrict__ oct_start, int* __restrict__ nlo,
-    int* __restrict__ nhi, double* __restrict__ gcx, double* __restrict__ gcy,
-    double* __restrict__ gcz, double* __restrict__ size, int* __restrict__ parent,
-    int* __restrict__ next, WNode* __restrict__ wn) {
-    const int i = blockIdx.x * kThreads + threadIdx.x;
-    if (i >= count) return;
-    const int node = lb + i;
-    const int nk = (int)nkids[i];
-    if (nk == 0) {
-        wn[node].first = -1;
-        wn[node].nchild = 0;
-        return;
+    int level, int cap, int* __restrict__ lev, const uint32_t* __restrict__ nkids,
+    const uint32_t* __restrict__ chunk_sum, const int* __restrict__ oct_start,
+    int* __restrict__ nlo, int* __restrict__ nhi, double* __restrict__ gcx,
+    double* __restrict__ gcy, double* __restrict__ gcz, double* __restrict__ size,
+    int* __restrict__ parent, int* __restrict__ next, WNode* __restrict__ wn) {
+    constexpr int kNodes = kEmitChunks * kLevelChunk; // one per thread
+    static_assert(kNodes == kThreads, "the prefix of a step is one value per thread");
+    __shared__ uint32_t s_red[8];
+    __shared__ int s_off[kNodes];
+    const int lb = lev[level], le = lev[level + 1], count = le - lb;
+    const int nchunk = (count + kLevelChunk - 1) / kLevelChunk;
+    const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    for (int n0 = blockIdx.x * kNodes; n0 < count || (blockIdx.x == 0 && n0 == 0);
+         n0 += gridDim.x * kNodes) {
+        // children of the chunks before this step's first, and of all of them
+        uint32_t before = 0, all = 0;
+        for (int c = threadIdx.x; c < nchunk; c += kThreads) {
+            const uint32_t v = chunk_sum[c];
+            before += (c < n0 / kLevelChunk) ? v : 0u;
+            all += v;
+        }
+        for (int d = 32; d >= 1; d >>= 1) {
+            before += __shfl_xor(before, d);
+            all += __shfl_xor(all, d);
+        }
+        if (lane == 0) {
+            s_red[w] = before;
+            s_red[4 + w] = all;
+        }
+        __syncthreads();
+        before = s_red[0] + s_red[1] + s_red[2] + s_red[3];
+        all = s_red[4] + s_red[5] + s_red[6] + s_red[7];
+        const bool fits = (long long)le + (long long)all <= (long long)cap;
+        if (blockIdx.x == 0 && n0 == 0 && threadIdx.x == 0) {
+            lev[level + 2] = fits ? le + (int)all : le;
+            if (!fits) atomicMax(&lev[kLevNeed], (int)min((long long)le + all, 0x7fffffffll));
+        }
+        if (!fits) return;
+        // first child of each node of this step
+        const int i = n0 + (int)threadIdx.x;
+        const uint32_t nk = (i < count) ? nkids[i] : 0u;
+        uint32_t inc = wave_incl_scan_dpp(nk);
+        __syncthreads();
+        if (lane == 63) s_red[w] = inc;
+        __syncthreads();
+        for (int k = 0; k < w; ++k) inc += s_red[k];
+        s_off[threadIdx.x] = le + (int)(before + inc - nk);
+        if (i < count) {
+            wn[lb + i].first = nk ? s_off[threadIdx.x] : -1;
+            wn[lb + i].nchild = (int)nk;
+        }
+        __syncthreads();
+        const int o = threadIdx.x & 7;
+        for (int k = 0; k < kNodes; k += kThreads / 8) {
+            const int j = k + (int)threadIdx.x / 8, ij = n0 + j, node = lb + ij;
+            const bool live = ij < count;
+            const int kids = live ? (int)nkids[ij] : 0;
+            int s = 0, hi = 0;
+            if (kids) {
+                s = oct_start[(size_t)ij * 8 + o];
+                hi = nhi[node];
+            }
+            int e = __shfl_down(s, 1);
+            if (o == 7) e = hi;
+            const bool child = kids && e > s;
+            const uint32_t m = (uint32_t)(__ballot(child) >> (lane & 56)) & 0xffu;
+            if (!child) continue;
+            const int r = __popc(m & ((1u << o) - 1u));
+            const int c = s_off[j] + r;
+            const double sz = size[node];
+            const double h = sz * 0.5, q = sz * 0.25;
+            nlo[c] = s;
+            nhi[c] = e;
+            gcx[c] = gcx[node] + ((o & 1) ? q : -q);
+            gcy[c] = gcy[node] + ((o & 2) ? q : -q);
+            gcz[c] = gcz[node] + ((o & 4) ? q : -q);
+            size[c] = h;
+            parent[c] = node;
+            next[c] = (r < kids - 1) ? c + 1 : next[node];
+        }
+        __syncthreads();
     }
-    const int base = next_lb + (int)off[i];
-    wn[node].first = base;
-    wn[node].nchild = nk;
-    const int hi = nhi[node];
-    const double sz = size[node];
-    const double h = sz * 0.5, q = sz * 0.25;
-    const double cx = gcx[node], cy = gcy[node], cz = gcz[node];
-    const int succ = next[node];
-    const int* os = oct_start + (size_t)i * 8;
-    int k = 0;
-    for (int o = 0; o < 8; ++o) {
-        const int s = os[o];
-        const int e = (o < 7) ? os[o + 1] : hi;
-        if (e <= s) continue;
-        const int c = base + k;
-        nlo[c] = s;
-        nhi[c] = e;
-        gcx[c] = cx + ((o & 1) ? q : -q);
-        gcy[c] = cy + ((o & 2) ? q : -q);
-        gcz[c] = cz + ((o & 4) ? q : -q);
-        size[c] = h;
-        parent[c] = node;
-        next[c] = (k < nk - 1) ? c + 1 : succ;
-        ++k;
-    }
+}
+
+// Levels below the deepest start (and end) at the node count.
+__global__ void k_pad_levels(int* __restrict__ lev, int from, int nnodes) {
+    const int L = from + (int)threadIdx.x;
+    if (L < kLevNeed) lev[L] = nnodes; // (the table's own entries are as they should be)
 }
 
 // ---- moments, deepest level first (tree.cc:153-196) + walk-node pack (tree.cc:507-523) ---------
@@ -371,8 +582,7 @@ __global__ __launch_bounds__(kThreads) void k_moments(
     const int* __restrict__ nhi, const double* __restrict__ gcx, const double* __restrict__ gcy,
     const double* __restrict__ gcz, const double* __restrict__ size,
     const double4* __restrict__ src, const double* __restrict__ src_soft,
-    const uint32_t* __restrict__ orderbuf, int* __restrict__ leaf_of,
-    int* __restrict__ slot_leaf, NodeVel nv, double* __restrict__ delta_out,
+    const uint32_t* __restrict__ orderbuf, int* __restrict__ slot_leaf, NodeVel nv, double* __restrict__ delta_out,
     double* __restrict__ soft_out, int* __restrict__ nleaf) {
     const int i = blockIdx.x * kThreads + threadIdx.x;
     const bool live = i < count;
@@ -404,7 +614,6 @@ __global__ __launch_bounds__(kThreads) void k_moments(
                 pvy += mm * uy;
                 pvz += mm * uz;
             }
-            leaf_of[orderbuf[k]] = node;
             slot_leaf[k] = node;
         }
     } else {
@@ -578,12 +787,14 @@ gz_status build_tree(gz_ctx* ctx, const gz_particles* p, const gz_build_opts* op
     // --- bbox + root cell (one per cluster for a forest)
     DevMem& s0 = ctx->scratch[0];
     const unsigned nbb = (unsigned)std::max<size_t>(1, std::min<size_t>(grid_for(n), 1024));
-    GZ_TRY(s0.reserve(nbb * 6 * sizeof(double) + 16 * sizeof(double) +
-                      (nc > 1 ? (size_t)nc * (4 * sizeof(double) + 2 * sizeof(int)) + 512 : 0)));
+    const size_t s0_live = nbb * 6 * sizeof(double) + 16 * sizeof(double) +
+                           (size_t)nc * (4 * sizeof(double) + 2 * sizeof(int)) + 512;
+    GZ_TRY(s0.reserve(s0_live + nbb * 4 * sizeof(uint32_t)));
     double* partial = s0.as<double>();
     double* droot = partial + (size_t)nbb * 6;
     double* croots = droot + 16;                                     // nc x 4 (forest)
     int* ccount = reinterpret_cast<int*>(croots + (size_t)4 * nc);   // nc + 1 (forest)
+    uint32_t* live = reinterpret_cast<uint32_t*>(s0.as<uint8_t>() + s0_live);
     uint32_t* cstart_dev = nullptr;
     if (nc > 1) {
         GZ_TRY(dalloc(reinterpret_cast<void**>(&t->cluster_start_dev), (nc + 1) * sizeof(uint32_t)));
@@ -596,11 +807,11 @@ gz_status build_tree(gz_ctx* ctx, const gz_particles* p, const gz_build_opts* op
         // droot keeps the first cluster's cell for the tree's info
         GZ_HIP(hipMemcpyAsync(droot, croots, 4 * sizeof(double), hipMemcpyDeviceToDevice, st));
     } else {
-        k_bbox_partial<<<nbb, kThreads, 0, st>>>(p->x, p->y, p->z, p->m, n, partial);
-        k_root_cell<<<1, 64, 0, st>>>(partial, (int)nbb, seed, fx, fy, fz, droot);
+        k_bbox_partial<<<nbb, kThreads, 0, st>>>(p->x, p->y, p->z, p->m, n, partial, live);
+        k_root_cell<<<1, kThreads, 0, st>>>(partial, live, (int)nbb, seed, fx, fy, fz, droot);
     }
     GZ_HIP(hipGetLastError());
-    double hroot[10];
+    double hroot[11];
     GZ_HIP(hipMemcpyAsync(hroot, droot, sizeof hroot, hipMemcpyDeviceToHost, st));
     GZ_HIP(hipEventRecord(ev[1], st));
 
@@ -608,13 +819,7 @@ gz_status build_tree(gz_ctx* ctx, const gz_particles* p, const gz_build_opts* op
     GZ_TRY(dalloc(reinterpret_cast<void**>(&t->rank), n * sizeof(uint32_t)));
     GZ_TRY(dalloc(reinterpret_cast<void**>(&t->leaf_of), n * sizeof(int)));
     GZ_TRY(dalloc(reinterpret_cast<void**>(&t->slot_leaf), n * sizeof(int)));
-    DevMem& s1 = ctx->scratch[1];
     const size_t nalloc = std::max<size_t>(n, 1);
-    const size_t flag_bytes = (nalloc + 64) * sizeof(uint32_t);
-    GZ_TRY(s1.reserve(flag_bytes + scan_tmp_bytes(nalloc) + 64));
-    uint32_t* flags = s1.as<uint32_t>();
-    uint32_t* dcount = flags + nalloc;
-    void* stmp = reinterpret_cast<uint8_t*>(s1.p) + flag_bytes;
     // order / keys ping-pong buffers
     DevMem& s2 = ctx->scratch[2];
     GZ_TRY(s2.reserve(nalloc * (2 * sizeof(uint64_t) + 2 * sizeof(uint32_t)) + 256));
@@ -622,22 +827,33 @@ gz_status build_tree(gz_ctx* ctx, const gz_particles* p, const gz_build_opts* op
     uint64_t* k1 = k0 + nalloc;
     uint32_t* v0 = reinterpret_cast<uint32_t*>(k1 + nalloc);
     uint32_t* v1 = v0 + nalloc;
-    uint32_t n_live32 = 0;
-    if (n > 0) {
+    GZ_HIP(hipStreamSynchronize(st));
+    for (int k = 0; k < 4; ++k) t->root_box[k] = hroot[k];
+    size_t nl = n;
+    // one tree whose particles are all live (the usual case): slot r is particle r before the
+    // sort. Otherwise the live ones are compacted first.
+    const bool all_live = nc == 1 && hroot[10] == (double)n;
+    if (n > 0 && !all_live) {
+        DevMem& s1 = ctx->scratch[1];
+        const size_t flag_bytes = (nalloc + 64) * sizeof(uint32_t);
+        GZ_TRY(s1.reserve(flag_bytes + scan_tmp_bytes(nalloc) + 64));
+        uint32_t* flags = s1.as<uint32_t>();
+        uint32_t* dcount = flags + nalloc;
+        void* stmp = reinterpret_cast<uint8_t*>(s1.p) + flag_bytes;
         k_live_flags<<<grid_for(n), kThreads, 0, st>>>(p->m, n, flags);
         GZ_TRY(exclusive_scan_u32(flags, flags, n, dcount, stmp, st));
         k_live_compact<<<grid_for(n), kThreads, 0, st>>>(p->m, n, flags, v0);
         GZ_HIP(hipGetLastError());
+        uint32_t n_live32 = 0;
         GZ_HIP(hipMemcpyAsync(&n_live32, dcount, sizeof(uint32_t), hipMemcpyDeviceToHost, st));
+        GZ_HIP(hipStreamSynchronize(st));
+        nl = n_live32;
     }
-    GZ_HIP(hipStreamSynchronize(st));
-    for (int k = 0; k < 4; ++k) t->root_box[k] = hroot[k];
-    const size_t nl = n_live32;
     t->n_live = nl;
     const double* key_roots = nc > 1 ? croots : droot;
     if (nl > 0) {
-        k_keys<<<grid_for(nl), kThreads, 0, st>>>(v0, nl, p->x, p->y, p->z, key_roots, cstart_dev,
-                                                  nc, k0);
+        k_keys<<<grid_for(nl), kThreads, 0, st>>>(all_live ? nullptr : v0, nl, p->x, p->y, p->z,
+                                                  key_roots, cstart_dev, nc, k0, v0);
         GZ_HIP(hipGetLastError());
     }
     GZ_HIP(hipEventRecord(ev[2], st));
@@ -654,7 +870,7 @@ gz_status build_tree(gz_ctx* ctx, const gz_particles* p, const gz_build_opts* op
         while ((1 << bits) < nc) ++bits;
         GZ_TRY(radix_sort_pairs(k1, v0, k0, v1, nl, bits, ctx->scratch[3], st));
         k_keys<<<grid_for(nl), kThreads, 0, st>>>(v0, nl, p->x, p->y, p->z, key_roots,
-                                                  cstart_dev, nc, t->skey);
+                                                  cstart_dev, nc, t->skey, nullptr);
         GZ_TRY(fill_zero_u32(reinterpret_cast<uint32_t*>(ccount), nc, st));
         k_cluster_counts<<<grid_for(nl), kThreads, 0, st>>>(v0, nl, cstart_dev, nc, ccount);
         GZ_HIP(hipGetLastError());
@@ -669,19 +885,16 @@ gz_status build_tree(gz_ctx* ctx, const gz_particles* p, const gz_build_opts* op
         GZ_HIP(hipMemcpyAsync(t->orderbuf, v0, nl * sizeof(uint32_t), hipMemcpyDeviceToDevice, st));
     GZ_HIP(hipEventRecord(ev[3], st));
 
-    // --- sorted source copy, rank, leaf_of reset
+    // --- sorted source copy
     GZ_TRY(dalloc(reinterpret_cast<void**>(&t->src), nl * sizeof(double4)));
     GZ_TRY(dalloc(reinterpret_cast<void**>(&t->src_soft), nl * sizeof(double)));
-    if (n) {
+    if (n > nl) { // particles outside the tree (the others are written below)
         k_fill_u32<<<grid_for(n), kThreads, 0, st>>>(t->rank, n, 0xFFFFFFFFu);
         k_fill_u32<<<grid_for(n), kThreads, 0, st>>>(reinterpret_cast<uint32_t*>(t->leaf_of), n,
                                                      0xFFFFFFFFu);
+        GZ_HIP(hipGetLastError());
     }
-    if (nl)
-        k_gather_sorted<<<grid_for(nl), kThreads, 0, st>>>(t->orderbuf, nl, p->x, p->y, p->z,
-                                                           p->m, p->soft, t->src, t->src_soft,
-                                                           t->rank);
-    GZ_HIP(hipGetLastError());
+    GZ_TRY(gather_sources(p, t->orderbuf, nl, t->src, t->src_soft, ctx->scratch[2], true, st));
     GZ_HIP(hipEventRecord(ev[4], st));
 
     // --- topology, level by level
@@ -690,8 +903,10 @@ gz_status build_tree(gz_ctx* ctx, const gz_particles* p, const gz_build_opts* op
     GZ_TRY(grow_nodes(t, 0, cap, st));
     t->level_begin.clear();
     t->level_begin.push_back(0);
+    t->level_begin.push_back(nc);
     t->arena_grows = 0;
-    int nnodes = 0;
+    GZ_TRY(dalloc(reinterpret_cast<void**>(&t->level_begin_dev), kLevInts * sizeof(int)));
+    int* lev = t->level_begin_dev;
     {
         // root: range [0, nl), the root cell, no parent, no successor. An empty particle set
         // still gets a root (a leaf of mass 0), as the reference's build_node does for [0, 0).
@@ -706,65 +921,82 @@ gz_status build_tree(gz_ctx* ctx, const gz_particles* p, const gz_build_opts* op
             }
             k_init_roots<<<grid_for(nc), kThreads, 0, st>>>(nc, croots, rstart_d, t->nlo, t->nhi,
                                                             t->gcx, t->gcy, t->gcz, t->size,
-                                                            t->parent, t->next);
+                                                            t->parent, t->next, lev);
             GZ_HIP(hipStreamSynchronize(st)); // rstart_h is a host vector read by the copy
         } else {
             k_init_root<<<1, 1, 0, st>>>(droot, (int)nl, t->nlo, t->nhi, t->gcx, t->gcy, t->gcz,
-                                         t->size, t->parent, t->next);
+                                         t->size, t->parent, t->next, lev);
         }
         GZ_HIP(hipGetLastError());
-        nnodes = nc;
-        t->level_begin.push_back(nc);
-        DevMem& s4 = ctx->scratch[4];
-        for (int level = 0;; ++level) {
-            const int lb = t->level_begin[level], le = t->level_begin[level + 1];
-            const int count = le - lb;
-            if (count == 0) break;
-            const size_t per = (size_t)count;
-            const size_t ob = per * 8 * sizeof(int), cb = (per + 64) * sizeof(uint32_t);
-            GZ_TRY(s4.reserve(ob + 2 * cb + scan_tmp_bytes(per) + 256));
-            int* oct = s4.as<int>();
-            uint32_t* nk = reinterpret_cast<uint32_t*>(reinterpret_cast<uint8_t*>(s4.p) + ob);
-            uint32_t* off = reinterpret_cast<uint32_t*>(reinterpret_cast<uint8_t*>(nk) + cb);
-            uint32_t* tot = off + per;
-            void* tmp = reinterpret_cast<uint8_t*>(off) + cb;
-            k_split<<<grid_for(per), kThreads, 0, st>>>(lb, count, level, t->nlo, t->nhi, t->skey,
-                                                        oct, nk);
-            GZ_HIP(hipGetLastError());
-            GZ_TRY(exclusive_scan_u32(nk, off, per, tot, tmp, st));
-            uint32_t total = 0;
-            GZ_HIP(hipMemcpyAsync(&total, tot, sizeof(uint32_t), hipMemcpyDeviceToHost, st));
-            GZ_HIP(hipStreamSynchronize(st));
-            const long long need = (long long)le + (long long)total;
-            if (need > 0x7FFFFFF0ll) return fail(GZ_ERR_NOMEM, "gz_tree_build: node count overflow");
-            if (need > cap) {
-                if (max_nodes > 0)
-                    return fail(GZ_ERR_ARENA,
-                                "gz_tree_build: tree needs more than max_nodes=%d nodes", max_nodes);
-                const long long want = std::min<long long>(2 * need + 1024, 0x7FFFFFF0ll);
-                GZ_TRY(grow_nodes(t, le, (int)want, st));
-                cap = (int)want;
-                ++t->arena_grows;
-            }
-            k_emit<<<grid_for(per), kThreads, 0, st>>>(lb, count, le, nk, off, oct, t->nlo, t->nhi,
-                                                       t->gcx, t->gcy, t->gcz, t->size, t->parent,
-                                                       t->next, t->wn);
-            GZ_HIP(hipGetLastError());
-            t->level_begin.push_back(le + (int)total);
-            nnodes = le + (int)total;
-            if (total == 0) break;
-        }
     }
+    DevMem& s4 = ctx->scratch[4];
+    // Levels are enqueued in batches, a read-back of the table after each: as many as a tree of nl
+    // particles has unless it is deeply clustered, then four at a time.
+    int level = 0, batch = 5;
+    for (size_t k = nl / (size_t)nc; k > 8; k >>= 3) ++batch;
+    for (bool done = false; !done;) {
+        // a level holds at most cap nodes
+        const size_t per = (size_t)cap, chunks = (per + kLevelChunk - 1) / kLevelChunk;
+        GZ_TRY(s4.reserve((per * 9 + chunks) * sizeof(int) + 768));
+        int* oct = s4.as<int>();
+        uint32_t* nk = reinterpret_cast<uint32_t*>(oct + 8 * per);
+        uint32_t* csum = nk + per;
+        const int end = std::min(level + batch, kMaxLevel + 1);
+        for (int L = level; L < end; ++L) {
+            // nodes of the level: at most 8 children of each node above; and every node but the
+            // roots has a parent of more than kLeafMax particles
+            long long most = (L < 12) ? ((long long)nc << (3 * L)) : (long long)cap;
+            most = std::max<long long>(1, std::min<long long>(most, cap));
+            if (L > 0) most = std::min<long long>(most, 8 * ((long long)nl / (kLeafMax + 1)) + 8);
+            const unsigned gs = (unsigned)std::min<long long>((most + kLevelChunk - 1) / kLevelChunk,
+                                                              4096);
+            if (L <= 3)
+                k_split<true><<<gs, kThreads, 0, st>>>(L, lev, t->nlo, t->nhi, t->skey, oct, nk,
+                                                       csum);
+            else
+                k_split<false><<<gs, kThreads, 0, st>>>(L, lev, t->nlo, t->nhi, t->skey, oct, nk,
+                                                        csum);
+            const unsigned ge = (unsigned)std::min<long long>((most + kThreads - 1) / kThreads,
+                                                              1024);
+            k_emit<<<ge, kThreads, 0, st>>>(L, cap, lev, nk, csum, oct, t->nlo, t->nhi, t->gcx,
+                                            t->gcy, t->gcz, t->size, t->parent, t->next, t->wn);
+            GZ_HIP(hipGetLastError());
+        }
+        int h[kLevInts];
+        GZ_HIP(hipMemcpyAsync(h, lev, sizeof h, hipMemcpyDeviceToHost, st));
+        GZ_HIP(hipStreamSynchronize(st));
+        for (; level < end; ++level) {
+            if (h[level + 2] > h[level + 1]) {
+                t->level_begin.push_back(h[level + 2]);
+                continue;
+            }
+            if (h[kLevNeed] == 0) { // no children: the deepest level (an empty one follows it)
+                t->level_begin.push_back(h[level + 1]);
+                done = true;
+                break;
+            }
+            // the children of this level outgrew the arena
+            const long long need = h[kLevNeed];
+            if (need > 0x7FFFFFF0ll)
+                return fail(GZ_ERR_NOMEM, "gz_tree_build: node count overflow");
+            if (max_nodes > 0)
+                return fail(GZ_ERR_ARENA, "gz_tree_build: tree needs more than max_nodes=%d nodes",
+                            max_nodes);
+            const long long want = std::min<long long>(2 * need + 1024, 0x7FFFFFF0ll);
+            GZ_TRY(grow_nodes(t, h[level + 1], (int)want, st));
+            cap = (int)want;
+            ++t->arena_grows;
+            GZ_TRY(fill_zero_u32(reinterpret_cast<uint32_t*>(lev + kLevNeed), 1, st));
+            break;
+        }
+        batch = 4;
+    }
+    const int nnodes = t->level_begin.back();
     t->nnodes = nnodes;
     t->depth = (int)t->level_begin.size() - 2;
-    {
-        // the level table on the device, padded with nnodes so any level index is valid
-        int lb[kMaxLevel + 2];
-        for (int L = 0; L < kMaxLevel + 2; ++L)
-            lb[L] = (L < (int)t->level_begin.size()) ? t->level_begin[L] : nnodes;
-        GZ_TRY(dalloc(reinterpret_cast<void**>(&t->level_begin_dev), sizeof lb));
-        GZ_HIP(hipMemcpy(t->level_begin_dev, lb, sizeof lb, hipMemcpyHostToDevice));
-    }
+    // any level index up to kMaxLevel + 1 is valid
+    k_pad_levels<<<1, 64, 0, st>>>(lev, (int)t->level_begin.size(), nnodes);
+    GZ_HIP(hipGetLastError());
     GZ_HIP(hipEventRecord(ev[5], st));
 
     // --- reuse state (tree.h:250-317): vmax and xpad always, the velocity moments with velocities
@@ -803,11 +1035,15 @@ gz_status build_tree(gz_ctx* ctx, const gz_particles* p, const gz_build_opts* op
         if (le <= lb) continue;
         k_moments<<<grid_for(le - lb), kThreads, 0, st>>>(lb, le - lb, t->wn, t->nlo, t->nhi,
                                                           t->gcx, t->gcy, t->gcz, t->size, t->src,
-                                                          t->src_soft, t->orderbuf, t->leaf_of,
+                                                          t->src_soft, t->orderbuf,
                                                           t->slot_leaf, nv, t->delta, t->soft,
                                                           dleaf);
         GZ_HIP(hipGetLastError());
     }
+    if (nl)
+        k_particle_links<<<grid_for(nl), kThreads, 0, st>>>(t->orderbuf, t->slot_leaf, nl, t->rank,
+                                                            t->leaf_of);
+    GZ_HIP(hipGetLastError());
     GZ_HIP(hipEventRecord(ev[6], st));
     int nleaf = 0;
     GZ_HIP(hipMemcpyAsync(&nleaf, dleaf, sizeof(int), hipMemcpyDeviceToHost, st));
@@ -838,12 +1074,13 @@ gz_status build_tree(gz_ctx* ctx, const gz_particles* p, const gz_build_opts* op
 gz_status regather_sources(gz_ctx* ctx, const gz_particles* p, gz_tree* t) {
     if (p->n != t->n) return fail(GZ_ERR_INVALID, "particle count %zu differs from the tree's %zu",
                                   p->n, t->n);
-    if (t->n_live)
-        k_gather_sorted<<<grid_for(t->n_live), kThreads, 0, ctx->stream>>>(
-            t->orderbuf, t->n_live, p->x, p->y, p->z, p->m, p->soft, t->src, t->src_soft,
-            t->rank);
-    GZ_HIP(hipGetLastError());
-    return GZ_OK;
+    // a captured call must not keep the scratch's address, which a later build may replace
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    GZ_HIP(hipStreamIsCapturing(ctx->stream, &cap));
+    DevMem none;
+    return gather_sources(p, t->orderbuf, t->n_live, t->src, t->src_soft,
+                          cap == hipStreamCaptureStatusNone ? ctx->scratch[2] : none, false,
+                          ctx->stream);
 }
 
 } // namespace gz
