@@ -440,18 +440,16 @@ __global__ __launch_bounds__(kThreads) void k_split(int level, const int* __rest
             if (!split || o == 0) b = a;
             if (WIDE) {
                 while (__ballot(a < b)) {
-                    // probes cut [a, b) into nine parts; digits ascend, so those below o come first
-                    const int len = b - a;
-                    const int at = a + (int)(((long long)len * (probe + 1)) / 9);
+                    // eight probes from a on cut [a, b) into eight parts; digits ascend, so the
+                    // probes below o come first
+                    const long long len = b - a;
+                    const int at = a + (int)((len * probe) >> 3);
                     const bool below = a < b && (int)((skey[at] >> shift) & 7ull) < o;
                     const uint64_t m = (__ballot(below) >> (lane & 56)) & 0xffull;
                     const int nbelow = __popcll(m);
                     if (a < b) {
-                        const int na = nbelow ? a + (int)(((long long)len * nbelow) / 9) + 1 : a;
-                        const int nb = nbelow < 8 ? a + (int)(((long long)len * (nbelow + 1)) / 9)
-                                                  : b;
-                        a = na;
-                        b = nb;
+                        if (nbelow < 8) b = a + (int)((len * nbelow) >> 3);
+                        if (nbelow > 0) a = a + (int)((len * (nbelow - 1)) >> 3) + 1;
                     }
                 }
             } else {
@@ -576,98 +574,65 @@ __global__ void k_pad_levels(int* __restrict__ lev, int from, int nnodes) {
     if (L < kLevNeed) lev[L] = nnodes; // (the table's own entries are as they should be)
 }
 
-// ---- moments, deepest level first (tree.cc:153-196) + walk-node pack (tree.cc:507-523) ---------
-__global__ __launch_bounds__(kThreads) void k_moments(
-    int lb, int count, WNode* __restrict__ wn, const int* __restrict__ nlo,
-    const int* __restrict__ nhi, const double* __restrict__ gcx, const double* __restrict__ gcy,
-    const double* __restrict__ gcz, const double* __restrict__ size,
-    const double4* __restrict__ src, const double* __restrict__ src_soft,
-    const uint32_t* __restrict__ orderbuf, int* __restrict__ slot_leaf, NodeVel nv, double* __restrict__ delta_out,
-    double* __restrict__ soft_out, int* __restrict__ nleaf) {
-    const int i = blockIdx.x * kThreads + threadIdx.x;
-    const bool live = i < count;
-    const int node = lb + (live ? i : 0);
-    const int nk = live ? wn[node].nchild : 1;
-    const uint64_t leaves = __ballot(live && nk == 0);
-    if (__lane_id() == 0 && leaves) atomicAdd(nleaf, (int)__popcll(leaves));
-    if (!live) return;
-    const int first = wn[node].first;
-    const int lo = nlo[node], hi = nhi[node];
+// ---- moments (tree.cc:153-196) + walk-node pack (tree.cc:507-523) --------------------------------
+// All leaves in one launch, then the interior nodes level by level from the deepest. The sums
+// are added in particle or child order, as the reference's are; only their loads are batched.
+struct MomentArgs {
+    WNode* wn;
+    const int *nlo, *nhi;
+    const double *gcx, *gcy, *gcz, *size;
+    const double4* src;
+    const double* src_soft;
+    const uint32_t* orderbuf;
+    int* slot_leaf;
+    NodeVel nv;
+    double *delta_out, *soft_out;
+};
+
+// Sums over a node's particles or children.
+struct NodeSums {
     double M = 0, sx = 0, sy = 0, sz = 0, smax = 0;
     double vmax = 0, pvx = 0, pvy = 0, pvz = 0; // with velocities: max |v| and momentum
-    if (nk == 0) {
-        for (int k = lo; k < hi; ++k) {
-            const double4 p = src[k];
-            const double mm = p.w;
-            M += mm;
-            sx += mm * p.x;
-            sy += mm * p.y;
-            sz += mm * p.z;
-            const double s = src_soft[k];
-            if (s > smax) smax = s;
-            if (nv.vx) { // tree.cc:161-166
-                const uint32_t q = orderbuf[k];
-                const double ux = nv.vx[q], uy = nv.vy[q], uz = nv.vz[q];
-                const double v = sqrt(ux * ux + uy * uy + uz * uz);
-                if (v > vmax) vmax = v;
-                pvx += mm * ux;
-                pvy += mm * uy;
-                pvz += mm * uz;
-            }
-            slot_leaf[k] = node;
-        }
-    } else {
-        for (int c = first; c < first + nk; ++c) {
-            const double mm = wn[c].mass;
-            M += mm;
-            sx += mm * wn[c].cx;
-            sy += mm * wn[c].cy;
-            sz += mm * wn[c].cz;
-            const double s = soft_out[c];
-            if (s > smax) smax = s;
-            if (nv.vx) { // tree.cc:177-181
-                if (nv.vmax[c] > vmax) vmax = nv.vmax[c];
-                pvx += mm * nv.vcom[c];
-                pvy += mm * nv.vcom[nv.nn + c];
-                pvz += mm * nv.vcom[2 * (size_t)nv.nn + c];
-            }
-        }
+};
+
+__device__ __forceinline__ void put_node(const MomentArgs& a, int node, NodeSums S, int first,
+                                         int nk, int lo, int hi) {
+    if (S.M > 0) {
+        S.sx /= S.M;
+        S.sy /= S.M;
+        S.sz /= S.M;
     }
-    if (M > 0) {
-        sx /= M;
-        sy /= M;
-        sz /= M;
-    }
-    const double dx = sx - gcx[node], dy = sy - gcy[node], dz = sz - gcz[node];
+    const double dx = S.sx - a.gcx[node], dy = S.sy - a.gcy[node], dz = S.sz - a.gcz[node];
     const double delta = sqrt(dx * dx + dy * dy + dz * dz);
-    const double side = size[node];
+    const double side = a.size[node];
     WNode w;
-    w.cx = sx;
-    w.cy = sy;
-    w.cz = sz;
+    w.cx = S.sx;
+    w.cy = S.sy;
+    w.cz = S.sz;
     w.s = side + delta;
-    w.mass = M;
-    w.soft = (float)smax;
+    w.mass = S.M;
+    w.soft = (float)S.smax;
     w.len = (float)side;
     w.first = first;
     w.nchild = nk;
     w.plo = lo;
     w.phi = hi;
-    wn[node] = w;
-    delta_out[node] = delta;
-    soft_out[node] = smax;
-    nv.vmax[node] = (float)vmax; // 0 without velocities
+    a.wn[node] = w;
+    a.delta_out[node] = delta;
+    a.soft_out[node] = S.smax;
+    const NodeVel& nv = a.nv;
+    nv.vmax[node] = (float)S.vmax; // 0 without velocities
     if (nv.vx) {
         // centre-of-mass velocity (tree.cc:188-190), the build moments that refreshes start
         // from, and zeroed incremental moments
         const size_t nn = (size_t)nv.nn;
-        nv.vcom[node] = (M > 0) ? pvx / M : 0.0;
-        nv.vcom[nn + node] = (M > 0) ? pvy / M : 0.0;
-        nv.vcom[2 * nn + node] = (M > 0) ? pvz / M : 0.0;
-        nv.m0[node] = M;
-        nv.m0[nn + node] = sx;
-        nv.m0[2 * nn + node] = sy;
-        nv.m0[3 * nn + node] = sz;
+        nv.vcom[node] = (S.M > 0) ? S.pvx / S.M : 0.0;
+        nv.vcom[nn + node] = (S.M > 0) ? S.pvy / S.M : 0.0;
+        nv.vcom[2 * nn + node] = (S.M > 0) ? S.pvz / S.M : 0.0;
+        nv.m0[node] = S.M;
+        nv.m0[nn + node] = S.sx;
+        nv.m0[2 * nn + node] = S.sy;
+        nv.m0[3 * nn + node] = S.sz;
         for (int d = 0; d < 3; ++d) {
             nv.dp[d * nn + node] = 0.0;
             nv.dq[d * nn + node] = 0.0;
@@ -675,6 +640,104 @@ __global__ __launch_bounds__(kThreads) void k_moments(
         nv.dmass[node] = 0.0;
     }
     nv.xpad[node] = 0.0f;
+}
+
+// The leaves, one thread each, four particles loaded together; nleaf (their number) is added to
+// once a workgroup (once a wave, it had 18,000 additions in turn at 4M particles).
+__global__ __launch_bounds__(kThreads) void k_leaf_moments(int nnodes, MomentArgs a,
+                                                           int* __restrict__ nleaf) {
+    __shared__ int s_n[kThreads / kWave];
+    int mine = 0;
+    for (int node = blockIdx.x * kThreads + threadIdx.x; node < nnodes;
+         node += gridDim.x * kThreads) {
+        if (a.wn[node].nchild != 0) continue;
+        ++mine;
+        const int lo = a.nlo[node], hi = a.nhi[node];
+        NodeSums S;
+        for (int k0 = lo; k0 < hi; k0 += 4) {
+            double4 p[4];
+            double e[4], ux[4], uy[4], uz[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const int k = min(k0 + j, hi - 1);
+                p[j] = a.src[k];
+                e[j] = a.src_soft[k];
+                if (a.nv.vx) {
+                    const uint32_t q = a.orderbuf[k];
+                    ux[j] = a.nv.vx[q];
+                    uy[j] = a.nv.vy[q];
+                    uz[j] = a.nv.vz[q];
+                }
+            }
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                if (k0 + j >= hi) break;
+                const double mm = p[j].w;
+                S.M += mm;
+                S.sx += mm * p[j].x;
+                S.sy += mm * p[j].y;
+                S.sz += mm * p[j].z;
+                if (e[j] > S.smax) S.smax = e[j];
+                if (a.nv.vx) { // tree.cc:161-166
+                    const double v = sqrt(ux[j] * ux[j] + uy[j] * uy[j] + uz[j] * uz[j]);
+                    if (v > S.vmax) S.vmax = v;
+                    S.pvx += mm * ux[j];
+                    S.pvy += mm * uy[j];
+                    S.pvz += mm * uz[j];
+                }
+                a.slot_leaf[k0 + j] = node;
+            }
+        }
+        put_node(a, node, S, -1, 0, lo, hi);
+    }
+    for (int d = 32; d >= 1; d >>= 1) mine += __shfl_xor(mine, d);
+    if ((threadIdx.x & 63) == 0) s_n[threadIdx.x >> 6] = mine;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        const int n = s_n[0] + s_n[1] + s_n[2] + s_n[3];
+        if (n) atomicAdd(nleaf, n);
+    }
+}
+
+// The interior nodes of one level, one thread each, all children loaded together.
+__global__ __launch_bounds__(kThreads) void k_inner_moments(int lb, int count, MomentArgs a) {
+    const int i = blockIdx.x * kThreads + threadIdx.x;
+    if (i >= count) return;
+    const int node = lb + i;
+    const int nk = a.wn[node].nchild;
+    if (nk == 0) return;
+    const int first = a.wn[node].first;
+    const NodeVel& nv = a.nv;
+    double cm[8], cx[8], cy[8], cz[8], cs[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+        const int c = first + min(j, nk - 1);
+        cm[j] = a.wn[c].mass;
+        cx[j] = a.wn[c].cx;
+        cy[j] = a.wn[c].cy;
+        cz[j] = a.wn[c].cz;
+        cs[j] = a.soft_out[c];
+    }
+    NodeSums S;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+        if (j >= nk) break;
+        S.M += cm[j];
+        S.sx += cm[j] * cx[j];
+        S.sy += cm[j] * cy[j];
+        S.sz += cm[j] * cz[j];
+        if (cs[j] > S.smax) S.smax = cs[j];
+    }
+    if (nv.vx) { // tree.cc:177-181
+        for (int c = first; c < first + nk; ++c) {
+            const double mm = a.wn[c].mass;
+            if (nv.vmax[c] > S.vmax) S.vmax = nv.vmax[c];
+            S.pvx += mm * nv.vcom[c];
+            S.pvy += mm * nv.vcom[nv.nn + c];
+            S.pvz += mm * nv.vcom[2 * (size_t)nv.nn + c];
+        }
+    }
+    put_node(a, node, S, first, nk, a.nlo[node], a.nhi[node]);
 }
 
 // ---- host driver ---------------------------------------------------------------------------------
@@ -1030,14 +1093,14 @@ gz_status build_tree(gz_ctx* ctx, const gz_particles* p, const gz_build_opts* op
     // --- moments + pack, deepest level first
     int* dleaf = reinterpret_cast<int*>(droot + 12);
     k_fill_u32<<<1, kThreads, 0, st>>>(reinterpret_cast<uint32_t*>(dleaf), 1, 0u);
-    for (int level = (int)t->level_begin.size() - 2; level >= 0; --level) {
+    const MomentArgs ma{t->wn, t->nlo, t->nhi, t->gcx, t->gcy, t->gcz, t->size, t->src,
+                        t->src_soft, t->orderbuf, t->slot_leaf, nv, t->delta, t->soft};
+    k_leaf_moments<<<std::min(grid_for(nnodes), 4096u), kThreads, 0, st>>>(nnodes, ma, dleaf);
+    GZ_HIP(hipGetLastError());
+    // (the deepest level is all leaves)
+    for (int level = (int)t->level_begin.size() - 4; level >= 0; --level) {
         const int lb = t->level_begin[level], le = t->level_begin[level + 1];
-        if (le <= lb) continue;
-        k_moments<<<grid_for(le - lb), kThreads, 0, st>>>(lb, le - lb, t->wn, t->nlo, t->nhi,
-                                                          t->gcx, t->gcy, t->gcz, t->size, t->src,
-                                                          t->src_soft, t->orderbuf,
-                                                          t->slot_leaf, nv, t->delta, t->soft,
-                                                          dleaf);
+        k_inner_moments<<<grid_for(le - lb), kThreads, 0, st>>>(lb, le - lb, ma);
         GZ_HIP(hipGetLastError());
     }
     if (nl)
@@ -1046,13 +1109,13 @@ gz_status build_tree(gz_ctx* ctx, const gz_particles* p, const gz_build_opts* op
     GZ_HIP(hipGetLastError());
     GZ_HIP(hipEventRecord(ev[6], st));
     int nleaf = 0;
+    WNode r;
     GZ_HIP(hipMemcpyAsync(&nleaf, dleaf, sizeof(int), hipMemcpyDeviceToHost, st));
+    GZ_HIP(hipMemcpyAsync(&r, t->wn, sizeof r, hipMemcpyDeviceToHost, st));
     GZ_HIP(hipStreamSynchronize(st));
     t->nleaves = nleaf;
     t->root = 0;
     {
-        WNode r;
-        GZ_HIP(hipMemcpy(&r, t->wn, sizeof r, hipMemcpyDeviceToHost));
         t->root_com[0] = r.cx;
         t->root_com[1] = r.cy;
         t->root_com[2] = r.cz;
