@@ -409,6 +409,12 @@ gz_status gz_ctx_create(int device, void* stream, gz_ctx** out) {
     gz_ctx* c = new (std::nothrow) gz_ctx();
     if (!c) return fail(GZ_ERR_NOMEM, "gz_ctx_create: out of host memory");
     c->device = device;
+    try {
+        c->blocks = std::make_shared<gz::BlockCache>();
+    } catch (const std::bad_alloc&) {
+        delete c;
+        return fail(GZ_ERR_NOMEM, "gz_ctx_create: out of host memory");
+    }
     if (stream) {
         c->stream = static_cast<hipStream_t>(stream);
     } else {
@@ -435,6 +441,7 @@ gz_status gz_ctx_destroy(gz_ctx* ctx) {
     (void)hipSetDevice(ctx->device);
     if (ctx->stream) (void)hipStreamSynchronize(ctx->stream);
     for (auto& m : ctx->scratch) m.release();
+    if (ctx->blocks) ctx->blocks->close();
     if (ctx->spill) (void)hipFree(ctx->spill);
     for (auto& e : ctx->ev)
         if (e) (void)hipEventDestroy(e);
@@ -459,9 +466,11 @@ gz_status gz_tree_build(gz_ctx* ctx, const gz_particles* p, const gz_build_opts*
     gz_tree* t = new (std::nothrow) gz_tree();
     if (!t) return fail(GZ_ERR_NOMEM, "gz_tree_build: out of host memory");
     t->ctx = ctx;
+    t->device = ctx->device;
+    t->blocks = ctx->blocks;
     gz_status s = gz::build_tree(ctx, p, opts, t);
     if (s != GZ_OK) {
-        (void)hipStreamSynchronize(ctx->stream);
+        (void)hipDeviceSynchronize();
         gz::tree_release(t);
         delete t;
         return s;
@@ -472,10 +481,9 @@ gz_status gz_tree_build(gz_ctx* ctx, const gz_particles* p, const gz_build_opts*
 
 gz_status gz_tree_free(gz_tree* tree) {
     if (!tree) return GZ_OK;
-    if (tree->ctx) {
-        (void)hipSetDevice(tree->ctx->device);
-        (void)hipStreamSynchronize(tree->ctx->stream);
-    }
+    // every stream, as freeing the blocks would wait for: another may still read the tree
+    (void)hipSetDevice(tree->device);
+    (void)hipDeviceSynchronize();
     gz::tree_release(tree);
     delete tree;
     return GZ_OK;

@@ -741,36 +741,52 @@ __global__ __launch_bounds__(kThreads) void k_inner_moments(int lb, int count, M
 }
 
 // ---- host driver ---------------------------------------------------------------------------------
-static gz_status dalloc(void** p, size_t bytes) {
-    GZ_HIP(hipMalloc(p, std::max<size_t>(bytes, 64)));
+static gz_status tree_alloc(gz_tree* t, void** p, size_t bytes) {
+    *p = nullptr;
+    if (t->nblocks == gz_tree::kMaxBlocks)
+        return fail(GZ_ERR_INTERNAL, "gz_tree_build: more device blocks than a tree has");
+    gz_tree::Block b{};
+    GZ_TRY(t->blocks->get(bytes, &b.p, &b.bytes));
+    t->block[t->nblocks++] = b;
+    *p = b.p;
     return GZ_OK;
 }
 
+// Gives a block back while the tree is being built; nothing enqueued may use it any more.
+static void tree_drop(gz_tree* t, void* p) {
+    for (int i = 0; i < t->nblocks; ++i)
+        if (t->block[i].p == p) {
+            t->blocks->put(p, t->block[i].bytes);
+            t->block[i] = t->block[--t->nblocks];
+            return;
+        }
+}
+
 template <class T>
-static gz_status grow_array(T*& a, size_t used, size_t cap, hipStream_t st) {
-    T* b = nullptr;
-    GZ_TRY(dalloc(reinterpret_cast<void**>(&b), cap * sizeof(T)));
+static gz_status grow_array(gz_tree* t, T*& a, size_t used, size_t cap, hipStream_t st) {
+    void* b = nullptr;
+    GZ_TRY(tree_alloc(t, &b, cap * sizeof(T)));
     if (a && used) GZ_HIP(hipMemcpyAsync(b, a, used * sizeof(T), hipMemcpyDeviceToDevice, st));
     if (a) {
         GZ_HIP(hipStreamSynchronize(st));
-        GZ_HIP(hipFree(a));
+        tree_drop(t, a);
     }
-    a = b;
+    a = static_cast<T*>(b);
     return GZ_OK;
 }
 
 static gz_status grow_nodes(gz_tree* t, int used, int cap, hipStream_t st) {
-    GZ_TRY(grow_array(t->wn, used, cap, st));
-    GZ_TRY(grow_array(t->next, used, cap, st));
-    GZ_TRY(grow_array(t->parent, used, cap, st));
-    GZ_TRY(grow_array(t->nlo, used, cap, st));
-    GZ_TRY(grow_array(t->nhi, used, cap, st));
-    GZ_TRY(grow_array(t->gcx, used, cap, st));
-    GZ_TRY(grow_array(t->gcy, used, cap, st));
-    GZ_TRY(grow_array(t->gcz, used, cap, st));
-    GZ_TRY(grow_array(t->size, used, cap, st));
-    GZ_TRY(grow_array(t->delta, used, cap, st));
-    GZ_TRY(grow_array(t->soft, used, cap, st));
+    GZ_TRY(grow_array(t, t->wn, used, cap, st));
+    GZ_TRY(grow_array(t, t->next, used, cap, st));
+    GZ_TRY(grow_array(t, t->parent, used, cap, st));
+    GZ_TRY(grow_array(t, t->nlo, used, cap, st));
+    GZ_TRY(grow_array(t, t->nhi, used, cap, st));
+    GZ_TRY(grow_array(t, t->gcx, used, cap, st));
+    GZ_TRY(grow_array(t, t->gcy, used, cap, st));
+    GZ_TRY(grow_array(t, t->gcz, used, cap, st));
+    GZ_TRY(grow_array(t, t->size, used, cap, st));
+    GZ_TRY(grow_array(t, t->delta, used, cap, st));
+    GZ_TRY(grow_array(t, t->soft, used, cap, st));
     t->cap = cap;
     return GZ_OK;
 }
@@ -779,14 +795,10 @@ static gz_status grow_nodes(gz_tree* t, int used, int cap, hipStream_t st) {
 // velocities vcom (3 nn), the build moments (4 nn: mass, then COM), dp and dq (3 nn each) and
 // dmass (nn).
 static gz_status alloc_reuse(gz_tree* t, int nn, bool vel) {
-    if (t->reuse_mem) {
-        (void)hipFree(t->reuse_mem);
-        t->reuse_mem = nullptr;
-    }
     const size_t n = (size_t)std::max(nn, 1);
     const size_t fl = (2 * n * sizeof(float) + 255) & ~size_t(255);
     const size_t db = vel ? 14 * n * sizeof(double) : 0;
-    GZ_TRY(dalloc(&t->reuse_mem, fl + db));
+    GZ_TRY(tree_alloc(t, &t->reuse_mem, fl + db));
     uint8_t* b = static_cast<uint8_t*>(t->reuse_mem);
     t->vmax = reinterpret_cast<float*>(b);
     t->xpad = t->vmax + n;
@@ -803,13 +815,11 @@ static gz_status alloc_reuse(gz_tree* t, int nn, bool vel) {
     return GZ_OK;
 }
 
+// The caller has waited for the device: the blocks may be handed to the next build at once.
 void tree_release(gz_tree* t) {
-    void* ptrs[] = {t->skey, t->orderbuf, t->rank, t->leaf_of, t->slot_leaf, t->src, t->src_soft,
-                    t->wn, t->next, t->parent, t->nlo, t->nhi, t->gcx, t->gcy, t->gcz, t->size,
-                    t->delta, t->soft, t->level_begin_dev, t->cluster_start_dev, t->reuse_mem,
-                    t->hmax, t->svel, t->age};
-    for (void* p : ptrs)
-        if (p) (void)hipFree(p);
+    for (int i = 0; i < t->nblocks; ++i) t->blocks->put(t->block[i].p, t->block[i].bytes);
+    t->nblocks = 0;
+    if (t->hmax) (void)hipFree(t->hmax);
 }
 
 static float ev_ms(hipEvent_t a, hipEvent_t b) {
@@ -860,7 +870,8 @@ gz_status build_tree(gz_ctx* ctx, const gz_particles* p, const gz_build_opts* op
     uint32_t* live = reinterpret_cast<uint32_t*>(s0.as<uint8_t>() + s0_live);
     uint32_t* cstart_dev = nullptr;
     if (nc > 1) {
-        GZ_TRY(dalloc(reinterpret_cast<void**>(&t->cluster_start_dev), (nc + 1) * sizeof(uint32_t)));
+        GZ_TRY(tree_alloc(t, reinterpret_cast<void**>(&t->cluster_start_dev),
+                          (nc + 1) * sizeof(uint32_t)));
         std::vector<uint32_t> hc(nc + 1);
         for (int c = 0; c <= nc; ++c) hc[c] = (uint32_t)opts->cluster_start[c];
         GZ_HIP(hipMemcpy(t->cluster_start_dev, hc.data(), hc.size() * sizeof(uint32_t),
@@ -879,9 +890,9 @@ gz_status build_tree(gz_ctx* ctx, const gz_particles* p, const gz_build_opts* op
     GZ_HIP(hipEventRecord(ev[1], st));
 
     // --- live filter + keys
-    GZ_TRY(dalloc(reinterpret_cast<void**>(&t->rank), n * sizeof(uint32_t)));
-    GZ_TRY(dalloc(reinterpret_cast<void**>(&t->leaf_of), n * sizeof(int)));
-    GZ_TRY(dalloc(reinterpret_cast<void**>(&t->slot_leaf), n * sizeof(int)));
+    GZ_TRY(tree_alloc(t, reinterpret_cast<void**>(&t->rank), n * sizeof(uint32_t)));
+    GZ_TRY(tree_alloc(t, reinterpret_cast<void**>(&t->leaf_of), n * sizeof(int)));
+    GZ_TRY(tree_alloc(t, reinterpret_cast<void**>(&t->slot_leaf), n * sizeof(int)));
     const size_t nalloc = std::max<size_t>(n, 1);
     // order / keys ping-pong buffers
     DevMem& s2 = ctx->scratch[2];
@@ -923,8 +934,8 @@ gz_status build_tree(gz_ctx* ctx, const gz_particles* p, const gz_build_opts* op
 
     // --- sort (a forest: by key, then stably by cluster, so each cluster is one sorted block)
     GZ_TRY(radix_sort_pairs(k0, v0, k1, v1, nl, 3 * kMaxLevel, ctx->scratch[3], st));
-    GZ_TRY(dalloc(reinterpret_cast<void**>(&t->skey), nl * sizeof(uint64_t)));
-    GZ_TRY(dalloc(reinterpret_cast<void**>(&t->orderbuf), nl * sizeof(uint32_t)));
+    GZ_TRY(tree_alloc(t, reinterpret_cast<void**>(&t->skey), nl * sizeof(uint64_t)));
+    GZ_TRY(tree_alloc(t, reinterpret_cast<void**>(&t->orderbuf), nl * sizeof(uint32_t)));
     std::vector<int> rstart_h(nc + 1, 0);
     if (nc > 1 && nl > 0) {
         k_cluster_keys<<<grid_for(nl), kThreads, 0, st>>>(v0, nl, cstart_dev, nc, k1);
@@ -949,8 +960,8 @@ gz_status build_tree(gz_ctx* ctx, const gz_particles* p, const gz_build_opts* op
     GZ_HIP(hipEventRecord(ev[3], st));
 
     // --- sorted source copy
-    GZ_TRY(dalloc(reinterpret_cast<void**>(&t->src), nl * sizeof(double4)));
-    GZ_TRY(dalloc(reinterpret_cast<void**>(&t->src_soft), nl * sizeof(double)));
+    GZ_TRY(tree_alloc(t, reinterpret_cast<void**>(&t->src), nl * sizeof(double4)));
+    GZ_TRY(tree_alloc(t, reinterpret_cast<void**>(&t->src_soft), nl * sizeof(double)));
     if (n > nl) { // particles outside the tree (the others are written below)
         k_fill_u32<<<grid_for(n), kThreads, 0, st>>>(t->rank, n, 0xFFFFFFFFu);
         k_fill_u32<<<grid_for(n), kThreads, 0, st>>>(reinterpret_cast<uint32_t*>(t->leaf_of), n,
@@ -968,7 +979,7 @@ gz_status build_tree(gz_ctx* ctx, const gz_particles* p, const gz_build_opts* op
     t->level_begin.push_back(0);
     t->level_begin.push_back(nc);
     t->arena_grows = 0;
-    GZ_TRY(dalloc(reinterpret_cast<void**>(&t->level_begin_dev), kLevInts * sizeof(int)));
+    GZ_TRY(tree_alloc(t, reinterpret_cast<void**>(&t->level_begin_dev), kLevInts * sizeof(int)));
     int* lev = t->level_begin_dev;
     {
         // root: range [0, nl), the root cell, no parent, no successor. An empty particle set
@@ -1065,15 +1076,13 @@ gz_status build_tree(gz_ctx* ctx, const gz_particles* p, const gz_build_opts* op
     // --- reuse state (tree.h:250-317): vmax and xpad always, the velocity moments with velocities
     NodeVel nv{};
     GZ_TRY(alloc_reuse(t, nnodes, opts && opts->vx && opts->vy && opts->vz));
-    if (!t->age) GZ_TRY(dalloc(reinterpret_cast<void**>(&t->age), sizeof(double)));
+    GZ_TRY(tree_alloc(t, reinterpret_cast<void**>(&t->age), sizeof(double)));
     k_fill_u32<<<1, kThreads, 0, st>>>(reinterpret_cast<uint32_t*>(t->age), 2, 0u);
     nv.nn = nnodes;
     nv.vmax = t->vmax;
     nv.xpad = t->xpad;
     if (t->has_vel) {
-        if (t->svel) (void)hipFree(t->svel);
-        t->svel = nullptr;
-        GZ_TRY(dalloc(reinterpret_cast<void**>(&t->svel),
+        GZ_TRY(tree_alloc(t, reinterpret_cast<void**>(&t->svel),
                       std::max<size_t>(t->n_live, 1) * sizeof(double4)));
         if (t->n_live)
             k_gather_vel<<<grid_for(t->n_live), kThreads, 0, st>>>(t->orderbuf, t->n_live,

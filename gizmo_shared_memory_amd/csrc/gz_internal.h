@@ -5,6 +5,8 @@
 
 #include <cfloat>
 #include <cstdint>
+#include <memory>
+#include <mutex>
 #include <string>
 #include <utility>
 #include <vector>
@@ -160,6 +162,32 @@ struct DevMem {
     template <class T> T* as() const { return static_cast<T*>(p); }
 };
 
+// Device blocks that freed trees leave for the next build on their context: a tree is some 25
+// arrays, and at 4M particles freeing and allocating them took 4.6 of a rebuild's 5.3 ms. It
+// holds at most kBytes and kBlocks (beyond that blocks go back to the device), and gives
+// everything back when its context is destroyed or an allocation here finds no memory. Trees may
+// be freed by another thread than the one that builds (the list is locked), and after their
+// context (they share the cache's ownership; it then keeps nothing).
+class BlockCache {
+public:
+    static constexpr size_t kBytes = size_t(2) << 30;
+    static constexpr int kBlocks = 64;
+    // A block of at least `bytes` (*got of them): a kept one if it is not much larger.
+    gz_status get(size_t bytes, void** p, size_t* got);
+    // A block that nothing on the device uses any more.
+    void put(void* p, size_t bytes);
+    void drain();
+    void close(); // drain, and keep nothing from now on
+
+private:
+    std::mutex mu_;
+    void* ptr_[kBlocks];
+    size_t size_[kBlocks];
+    int n_ = 0;
+    size_t held_ = 0;
+    bool open_ = true;
+};
+
 // ---- device-wide primitives (gz_prims.hip) --------------------------------------------------
 // Exclusive scan of n uint32 values (in may equal out). total_dev, when non-null, receives the
 // sum (device). tmp must hold scan_tmp_bytes(n).
@@ -240,6 +268,7 @@ struct gz_ctx {
     hipStream_t stream = nullptr;
     bool own_stream = false;
     gz::DevMem scratch[16];
+    std::shared_ptr<gz::BlockCache> blocks;
     // the walk autotuner's choices, one per workload key (gz_walk_autotune)
     std::vector<std::pair<std::vector<long long>, gz_walk_opts>> tuned;
     hipEvent_t ev[16] = {};
@@ -319,6 +348,16 @@ struct gz_model {
 
 struct gz_tree {
     gz_ctx* ctx = nullptr;
+    int device = 0;
+    // every device block of the tree but hmax, and the context's cache they come from
+    std::shared_ptr<gz::BlockCache> blocks;
+    struct Block {
+        void* p;
+        size_t bytes;
+    };
+    static constexpr int kMaxBlocks = 32;
+    Block block[kMaxBlocks];
+    int nblocks = 0;
     size_t n = 0, n_live = 0;
     int nnodes = 0, nleaves = 0, depth = 0, arena_grows = 0, root = 0;
     int cap = 0;

@@ -62,6 +62,68 @@ void DevMem::release() {
     bytes = 0;
 }
 
+gz_status BlockCache::get(size_t bytes, void** p, size_t* got) {
+    const size_t want = (std::max<size_t>(bytes, 1) + 4095) & ~size_t(4095);
+    {
+        std::lock_guard<std::mutex> lock(mu_);
+        int best = -1;
+        for (int i = 0; i < n_; ++i)
+            if (size_[i] >= want && size_[i] - want <= want / 4 &&
+                (best < 0 || size_[i] < size_[best]))
+                best = i;
+        if (best >= 0) {
+            *p = ptr_[best];
+            *got = size_[best];
+            held_ -= size_[best];
+            --n_;
+            ptr_[best] = ptr_[n_];
+            size_[best] = size_[n_];
+            return GZ_OK;
+        }
+    }
+    hipError_t e = hipMalloc(p, want);
+    if (e == hipErrorOutOfMemory) {
+        (void)hipGetLastError();
+        drain();
+        e = hipMalloc(p, want);
+    }
+    if (e != hipSuccess) {
+        *p = nullptr;
+        return hip_fail(e, "hipMalloc", __FILE__, __LINE__);
+    }
+    *got = want;
+    return GZ_OK;
+}
+
+void BlockCache::put(void* p, size_t bytes) {
+    {
+        std::lock_guard<std::mutex> lock(mu_);
+        if (open_ && n_ < kBlocks && held_ + bytes <= kBytes) {
+            ptr_[n_] = p;
+            size_[n_] = bytes;
+            ++n_;
+            held_ += bytes;
+            return;
+        }
+    }
+    (void)hipFree(p);
+}
+
+void BlockCache::drain() {
+    std::lock_guard<std::mutex> lock(mu_);
+    for (int i = 0; i < n_; ++i) (void)hipFree(ptr_[i]);
+    n_ = 0;
+    held_ = 0;
+}
+
+void BlockCache::close() {
+    {
+        std::lock_guard<std::mutex> lock(mu_);
+        open_ = false;
+    }
+    drain();
+}
+
 // ---- wave / block scans ----------------------------------------------------------------------
 __device__ __forceinline__ uint32_t wave_inclusive_scan(uint32_t x) {
     return wave_incl_scan_dpp(x);

@@ -88,3 +88,23 @@ def test_arena_grows_between_levels(gz, oracle):
     assert T.info.arena_grows >= 1 and T.info.depth >= 18
     with pytest.raises(Exception, match="max_nodes"):
         gz.build(P, max_nodes=200)
+
+
+def test_freed_blocks_serve_other_trees(gz, oracle):
+    """Trees of different sizes built and freed in turn reuse each other's device blocks, with and
+    without velocities, and while another tree is alive."""
+    keep, kt, _ = _check(gz, oracle, _particles(30000, 0, 6))
+    want = gz.accel(kt, keep, np.arange(200), 0.7)
+    for n, dead in ((30001, 0), (29000, 5), (60000, 0), (30001, 2)):
+        case = _particles(n, dead, n)
+        _check(gz, oracle, case)
+        P = gz.Particles(*case)
+        T = gz.build(P, vel=case[:3])
+        T.refresh_walk_nodes(0.0)
+        got = T.download()
+        ref = gz.build(P).download()
+        for f in ("mass", "cx", "cy", "cz", "soft", "first", "plo", "leaf_of", "rank"):
+            assert np.array_equal(got[f], ref[f]), f
+        del T
+    for u, v in zip(want, gz.accel(kt, keep, np.arange(200), 0.7)):
+        assert bool((u == v).all())
