@@ -426,7 +426,7 @@ __global__ __launch_bounds__(kThreads) void k_split(int level, const int* __rest
     const int o = WIDE ? (lane >> 3) : (threadIdx.x & 7), probe = lane & 7;
     for (int c0 = blockIdx.x * kLevelChunk; c0 < count; c0 += gridDim.x * kLevelChunk) {
         uint32_t sum = 0; // children of this wave's nodes
-        for (int k = 0; k < kLevelChunk; k += kPer) {
+        for (int k = 0; k < kLevelChunk && c0 + k < count; k += kPer) {
             const int i = c0 + k + (int)threadIdx.x / kLanes;
             const bool live = i < count;
             int lo = 0, hi = 0;
@@ -482,15 +482,18 @@ __global__ __launch_bounds__(kThreads) void k_split(int level, const int* __rest
 // child. A workgroup adds up the chunk counts before its own. Eight lanes write one node's
 // children, so neighbouring lanes write neighbouring nodes. When the children would outgrow the
 // arena, nothing is emitted, the next level stays empty and lev[kLevNeed] tells the nodes needed.
-constexpr int kEmitChunks = 4; // chunks a workgroup emits at a time
+// A workgroup emits CHUNKS chunks at a time: four where a level may be large (each step adds up the
+// level's chunk counts), one in small trees, whose levels are a few steps long.
+constexpr int kEmitSmall = 1 << 18; // arenas up to this many nodes count as small
+template <int CHUNKS>
 __global__ __launch_bounds__(kThreads) void k_emit(
     int level, int cap, int* __restrict__ lev, const uint32_t* __restrict__ nkids,
     const uint32_t* __restrict__ chunk_sum, const int* __restrict__ oct_start,
     int* __restrict__ nlo, int* __restrict__ nhi, double* __restrict__ gcx,
     double* __restrict__ gcy, double* __restrict__ gcz, double* __restrict__ size,
     int* __restrict__ parent, int* __restrict__ next, WNode* __restrict__ wn) {
-    constexpr int kNodes = kEmitChunks * kLevelChunk; // one per thread
-    static_assert(kNodes == kThreads, "the prefix of a step is one value per thread");
+    constexpr int kNodes = CHUNKS * kLevelChunk;
+    static_assert(kNodes <= kThreads, "the prefix of a step is at most one value per thread");
     __shared__ uint32_t s_red[8];
     __shared__ int s_off[kNodes];
     const int lb = lev[level], le = lev[level + 1], count = le - lb;
@@ -524,20 +527,22 @@ __global__ __launch_bounds__(kThreads) void k_emit(
         if (!fits) return;
         // first child of each node of this step
         const int i = n0 + (int)threadIdx.x;
-        const uint32_t nk = (i < count) ? nkids[i] : 0u;
+        const bool mine = (int)threadIdx.x < kNodes && i < count;
+        const uint32_t nk = mine ? nkids[i] : 0u;
         uint32_t inc = wave_incl_scan_dpp(nk);
         __syncthreads();
         if (lane == 63) s_red[w] = inc;
         __syncthreads();
         for (int k = 0; k < w; ++k) inc += s_red[k];
-        s_off[threadIdx.x] = le + (int)(before + inc - nk);
-        if (i < count) {
-            wn[lb + i].first = nk ? s_off[threadIdx.x] : -1;
+        const int first = le + (int)(before + inc - nk);
+        if (mine) {
+            s_off[threadIdx.x] = first;
+            wn[lb + i].first = nk ? first : -1;
             wn[lb + i].nchild = (int)nk;
         }
         __syncthreads();
         const int o = threadIdx.x & 7;
-        for (int k = 0; k < kNodes; k += kThreads / 8) {
+        for (int k = 0; k < kNodes && n0 + k < count; k += kThreads / 8) {
             const int j = k + (int)threadIdx.x / 8, ij = n0 + j, node = lb + ij;
             const bool live = ij < count;
             const int kids = live ? (int)nkids[ij] : 0;
@@ -1010,8 +1015,8 @@ gz_status build_tree(gz_ctx* ctx, const gz_particles* p, const gz_build_opts* op
     for (size_t k = nl / (size_t)nc; k > 8; k >>= 3) ++batch;
     for (bool done = false; !done;) {
         // a level holds at most cap nodes
-        const size_t per = (size_t)cap, chunks = (per + kLevelChunk - 1) / kLevelChunk;
-        GZ_TRY(s4.reserve((per * 9 + chunks) * sizeof(int) + 768));
+        const size_t per = (size_t)cap, sums = (per + kLevelChunk - 1) / kLevelChunk;
+        GZ_TRY(s4.reserve((per * 9 + sums) * sizeof(int) + 768));
         int* oct = s4.as<int>();
         uint32_t* nk = reinterpret_cast<uint32_t*>(oct + 8 * per);
         uint32_t* csum = nk + per;
@@ -1030,10 +1035,12 @@ gz_status build_tree(gz_ctx* ctx, const gz_particles* p, const gz_build_opts* op
             else
                 k_split<false><<<gs, kThreads, 0, st>>>(L, lev, t->nlo, t->nhi, t->skey, oct, nk,
                                                         csum);
-            const unsigned ge = (unsigned)std::min<long long>((most + kThreads - 1) / kThreads,
-                                                              1024);
-            k_emit<<<ge, kThreads, 0, st>>>(L, cap, lev, nk, csum, oct, t->nlo, t->nhi, t->gcx,
-                                            t->gcy, t->gcz, t->size, t->parent, t->next, t->wn);
+            const int chunks = (cap <= kEmitSmall) ? 1 : 4;
+            const long long nodes = (long long)chunks * kLevelChunk;
+            const unsigned ge = (unsigned)std::min<long long>((most + nodes - 1) / nodes, 1024);
+            const auto emit = (chunks == 1) ? k_emit<1> : k_emit<4>;
+            emit<<<ge, kThreads, 0, st>>>(L, cap, lev, nk, csum, oct, t->nlo, t->nhi, t->gcx,
+                                          t->gcy, t->gcz, t->size, t->parent, t->next, t->wn);
             GZ_HIP(hipGetLastError());
         }
         int h[kLevInts];

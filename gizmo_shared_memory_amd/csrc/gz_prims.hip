@@ -391,6 +391,7 @@ __global__ __launch_bounds__(kRsThreads) void k_rs_scatter(
     uint32_t gplace, total;
     if (direct) {
         uint32_t before = 0, all = 0;
+#pragma unroll 8
         for (uint32_t b = 0; b < nb; ++b) {
             const uint32_t c = offs[(size_t)b * kRsRadix + tid];
             before += (b < blockIdx.x) ? c : 0u;
