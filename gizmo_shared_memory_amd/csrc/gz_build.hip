@@ -314,10 +314,8 @@ __global__ __launch_bounds__(kThreads) void k_gather_rec(const uint32_t* __restr
     const size_t r = (size_t)blockIdx.x * kThreads + threadIdx.x;
     if (r >= nl) return;
     const double4* p = reinterpret_cast<const double4*>(rec + orderbuf[r]);
-    const double4 q = p[0];
-    const double s = p[1].x;
-    src[r] = q;
-    src_soft[r] = s;
+    src[r] = p[0];
+    if (src_soft) src_soft[r] = p[1].x;
 }
 
 __global__ __launch_bounds__(kThreads) void k_gather_sorted(
@@ -328,7 +326,7 @@ __global__ __launch_bounds__(kThreads) void k_gather_sorted(
     if (r >= nl) return;
     const uint32_t p = orderbuf[r];
     src[r] = make_double4(x[p], y[p], z[p], m[p]);
-    src_soft[r] = soft ? soft[p] : 0.0;
+    if (src_soft) src_soft[r] = soft ? soft[p] : 0.0;
 }
 
 // grow: the records' memory may be allocated (else they are used only if there is room already).
@@ -350,6 +348,11 @@ static gz_status gather_sources(const gz_particles* p, const uint32_t* orderbuf,
     }
     GZ_HIP(hipGetLastError());
     return GZ_OK;
+}
+
+gz_status gather_live(gz_ctx* ctx, const gz_particles* p, const gz_tree* t, double4* out) {
+    return gather_sources(p, t->orderbuf, t->n_live, out, nullptr, ctx->scratch[2], true,
+                          ctx->stream);
 }
 
 // The inverse permutation and each particle's leaf, from the sorted side.

@@ -3,26 +3,31 @@
 //
 // The reference iterates each target privately: search the tree within h, sum the kernel over the
 // gas neighbours, and take a bracket-guarded Newton step on N_eff(h) = ball_vol(h) sum_j W until
-// N_eff is within the (widening) tolerance of the neighbour target. Here every still-unconverged
-// target advances one step per round, and a round is one kernel (k_density_round): each target
-// has a lane, a wavefront holds up to 64 targets that are neighbours in Morton order, and the wave
-// walks the union of their own searches depth first, one node at a time (the nodes' search boxes
-// packed into 32-byte records per call). A lane waits on a node only while the reference's node
-// test (hydro.cc:55-72, on the float search nodes) has admitted its sphere at every ancestor; at
-// a reached leaf, each waiting lane tests every particle against its sphere (hydro.cc:80-87) and
-// notes a neighbour in its column of an LDS buffer; a lane adds its noted neighbours' kernel
-// terms whenever some column fills, and at the end. Depth first with children in octant order is
-// the tree's slot order, which is the order of the reference's neighbour list, so each lane adds
-// the reference's terms in the reference's order without a stored list. The lane then applies
-// the reference's update, and the targets that are done leave the active list (a stable
-// compaction, so the waves keep their Morton locality).
+// N_eff is within the (widening) tolerance of the neighbour target. Here it is three kernels, each
+// adding the reference's terms in the reference's order (its list is in the tree's slot order, which
+// is depth first with children in octant order):
 //
-// Two cases leave this path for k_density_far, where a wavefront takes a single target, tests a
-// node's children together and a leaf's particles together, and adds the terms in the same order.
-// A target whose radius exceeds kFarLeaf times its leaf's side would make its wave of 64 walk a
-// large part of the tree one node and one particle at a time: it takes a wave of its own after the
-// round. And once kLoopTargets or fewer targets remain, one launch gives each a wave that iterates
-// it to the end, instead of a round (and a host round trip) per step.
+//   * k_density_round, while many targets are unconverged: every target one step per round, a lane
+//     per target and 64 Morton-neighbouring targets per wave. The wave walks the tree once for all
+//     of them, up to 64 nodes at a time (their search boxes packed into 32-byte records per call)
+//     on a stack kept in depth-first order, stages the particles of the leaves it meets in LDS,
+//     and every lane tests each against its own sphere and notes the neighbours' slots in its
+//     column of an LDS buffer; whenever some column is nearly full, and at the end, the lanes add
+//     their neighbours' terms. The targets that are done leave the active list (a stable
+//     compaction, so the waves keep their Morton locality).
+//   * k_density_near, for the last kLoopTargets: a wave per target, iterated to the end on
+//     candidates collected once.
+//   * k_density_far, a wave per target on the tree, for spheres that hold many particles: in a
+//     round, targets whose radius exceeds kFarLeaf times their leaf's side (one of them would make
+//     its wave of 64 walk a large part of the tree), and among the last, those with more than
+//     kNearMax candidates.
+//
+// What bounds a round: at 4.2M targets (Hernquist, 3% from converged) 38,500 VALU instructions a
+// wave, busy 4.4 of 7.0 ms, the rest latency at 2.5 waves per SIMD (LDS): about 14 instructions for
+// each of some 1,000 staged particles, and 81 steps of about 110 for the terms (33 neighbours a
+// lane; a buffer fills with the lanes unevenly advanced). Walking one node at a time with the
+// general square root and division it took 8.9 ms. The neighbours' live values are put in slot
+// order once per call, where a wave's lanes find them in the same lines.
 //
 // The one difference from the reference's arithmetic is pow(dx, 2) in the 3D face-closure test,
 // taken here as dx * dx (correctly rounded; glibc's pow is within half an ulp of it, not always
@@ -31,7 +36,9 @@
 #include <cmath>
 #include <cstring>
 
+#include "gz_features.h"
 #include "gz_internal.h"
+#include "gz_wave.h"
 
 namespace gz {
 namespace {
@@ -40,8 +47,15 @@ constexpr double kPi = 3.14159265358979323846;
 constexpr int kMaxIter = 100; // hydro.cc:201
 constexpr int kWavesWanted = 2048; // a round's targets are spread thinner below this many waves
 constexpr int kNbBuf = 32;          // neighbours each lane holds before their terms are added
+constexpr int kDensStack = 640;     // entries of a round wave's stack ...
+constexpr int kDensSpare = 160;     // ... of which a window of one node may need 7 a level
+constexpr int kDensRun = 16;        // leaves taken together, when as many are next in order
 constexpr double kFarLeaf = 4.0;    // radius over leaf side beyond which a target takes the lists
-constexpr uint32_t kLoopTargets = 131072; // active targets few enough to iterate in one launch
+// Active targets few enough to iterate in one launch. Rounds are cheaper per target while a wave's
+// targets are neighbours; the fewer are left, the further apart they lie and the more launches and
+// read-backs they cost: on 4.2M targets the solve took 22.8 ms with 131,072, 22.3 with 524,288 and
+// 23.9 with 1,048,576; on 300k 4.7, 3.55 and 3.54, on 1M 8.4, 8.8 and 13.7.
+constexpr uint32_t kLoopTargets = 393216;
 
 // kernel_norm, ball_vol, kernel_w, kernel_dwdh (hydro.h:29-65): cubic spline of support h in dim
 // dimensions, operand for operand.
@@ -55,29 +69,56 @@ __device__ __forceinline__ double ball_vol(double h, int dim) {
     if (dim == 2) return kPi * h * h;
     return 4.0 * kPi / 3.0 * h * h * h;
 }
-__device__ __forceinline__ double kernel_w(double r, double h, int dim) {
-    const double q = r / h;
-    if (q >= 1.0) return 0.0;
-    const double norm = knorm(h, dim);
-    if (q < 0.5) return norm * (1.0 - 6.0 * q * q + 6.0 * q * q * q);
-    const double u = 1.0 - q;
-    return norm * 2.0 * u * u * u;
+// The correctly rounded square root and quotient, as the IEEE operations give them, in fewer
+// instructions than the compiler's general expansions (which scale for the whole exponent range):
+// the hardware's estimate or a rounded reciprocal, refined with fused multiply-adds until the last
+// correction is a rounding of the exact remainder (P. Markstein, IBM J. Res. Dev. 34 (1990) 111).
+// Outside the ranges where every intermediate is exact the general operation is used.
+__device__ __forceinline__ double sqrt_rn(double x) {
+    if ((x > 0.0 && x < 1e-250) || !(x <= 1e250)) return sqrt(x);
+    const double y = __builtin_amdgcn_rsq(x);
+    double g = x * y, h = 0.5 * y;
+    const double e = __builtin_fma(-h, g, 0.5);
+    g = __builtin_fma(g, e, g);
+    h = __builtin_fma(h, e, h);
+    g = __builtin_fma(__builtin_fma(-g, g, x), h, g);
+    g = __builtin_fma(__builtin_fma(-g, g, x), h, g);
+    return (x > 0.0) ? g : x; // (0 stays 0)
 }
-__device__ __forceinline__ double kernel_dwdh(double r, double h, int dim) {
-    const double q = r / h;
-    if (q >= 1.0) return 0.0;
-    const double norm = knorm(h, dim);
-    double f, fp;
-    if (q < 0.5) {
-        f = 1.0 - 6.0 * q * q + 6.0 * q * q * q;
-        fp = -12.0 * q + 18.0 * q * q;
-    } else {
-        const double u = 1.0 - q;
-        f = 2.0 * u * u * u;
-        fp = -6.0 * u * u;
+
+// W(r) and dW/dh(r) (hydro.h:36-65) for one support h: operand for operand, with what depends on
+// h alone computed once.
+struct Kernel {
+    double h, rh, norm, norm2, c1; // rh = 1/h; norm2 = norm * 2; c1 = -(dim / h) * norm
+    bool general;                  // h outside the range of the short quotient
+    __device__ __forceinline__ void set(double h_, int dim) {
+        h = h_;
+        rh = 1.0 / h;
+        norm = knorm(h, dim);
+        norm2 = norm * 2.0;
+        c1 = -((double)dim / h) * norm;
+        general = !(h > 1e-120 && h < 1e120);
     }
-    return -((double)dim / h) * norm * f - (q / h) * norm * fp;
-}
+    // a / h (a of a size where a quotient that underflows changes no sum it enters)
+    __device__ __forceinline__ double over_h(double a) const {
+        if (general) return a / h;
+        double q = a * rh;
+        q = __builtin_fma(__builtin_fma(-q, h, a), rh, q);
+        return __builtin_fma(__builtin_fma(-q, h, a), rh, q);
+    }
+    __device__ __forceinline__ void at(double r, double* w, double* dwdh) const {
+        const double q = over_h(r);
+        const double t = 6.0 * q * q, u = 1.0 - q;
+        const double f_in = 1.0 - t + t * q, f_out = 2.0 * u * u * u;
+        const double fp_in = -12.0 * q + 18.0 * q * q, fp_out = -6.0 * u * u;
+        const bool in = q < 0.5;
+        const double f = in ? f_in : f_out, fp = in ? fp_in : fp_out;
+        const double ww = in ? norm * f_in : norm2 * u * u * u;
+        const double d = c1 * f - over_h(q) * norm * fp;
+        *w = (q >= 1.0) ? 0.0 : ww;
+        *dwdh = (q >= 1.0) ? 0.0 : d;
+    }
+};
 
 // invert_moments (shmem/vec.h:43-63) of the symmetric moments e (xx yy zz xy yz xz) into b
 // (row-major 3x3, zero outside the live block); false when degenerate. 3D is Mat3::invert
@@ -148,6 +189,10 @@ struct DensArgs {
     const uint32_t* targets;
     const double *x, *y, *z, *m;
     const uint8_t* type; // null: all gas
+    // the particles' live values by slot (x, y, z, m, and whether gas), or null: read through
+    // orderbuf from the arrays above
+    const double4* live;
+    const uint8_t* live_gas;
     double des_ngb, ngb_tol;
     int n_dims;
     const double* cond_prev; // by particle, or null
@@ -170,22 +215,52 @@ struct DensArgs {
     const uint32_t* orderbuf;
     int root, nclusters;
     double tau;
+    const int* moved; // nonzero: some particle lies outside its build-time cell
 };
 
 // The terms one gas neighbour j adds to a target at (p0, p1, p2) with support h (hydro.cc:206-217):
 // v = {W, dW/dh, m W, dx dx W, dy dy W, dz dz W, dx dy W, dy dz W, dx dz W, dx W, dy W, dz W}, and
 // whether r < h. Non-gas neighbours add nothing (returns false).
 constexpr int kTerms = 12;
-__device__ __forceinline__ bool density_terms(const DensArgs& a, uint32_t j, double p0, double p1,
-                                              double p2, double h, int dim, double* v,
-                                              bool* inside) {
-    if (a.type && a.type[j] != 0) return false; // gas neighbours only
-    const double d0 = a.x[j] - p0, d1 = a.y[j] - p1, d2 = a.z[j] - p2;
-    const double r = sqrt(d0 * d0 + d1 * d1 + d2 * d2);
-    const double w = kernel_w(r, h, dim);
+// Lane l's value, as a scalar; the wave's largest value.
+__device__ __forceinline__ float lane_f(float v, int l) {
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
+}
+__device__ __forceinline__ int wave_max_i(int v) {
+    for (int d = 32; d >= 1; d >>= 1) v = max(v, __shfl_xor(v, d));
+    return v;
+}
+// Set bits of m below this lane.
+__device__ __forceinline__ int lanes_under(uint64_t m) {
+    return (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32),
+                                          __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+}
+struct Neighbour {
+    double x, y, z, m;
+    bool gas;
+};
+__device__ __forceinline__ Neighbour neighbour_at(const DensArgs& a, uint32_t slot) {
+    Neighbour n;
+    if (a.live) {
+        const double4 q = a.live[slot];
+        n.x = q.x; n.y = q.y; n.z = q.z; n.m = q.w;
+        n.gas = !a.live_gas || a.live_gas[slot] != 0;
+    } else {
+        const uint32_t j = a.orderbuf[slot];
+        n.x = a.x[j]; n.y = a.y[j]; n.z = a.z[j]; n.m = a.m[j];
+        n.gas = !a.type || a.type[j] == 0;
+    }
+    return n;
+}
+__device__ __forceinline__ bool density_terms(const Neighbour& nb, double p0, double p1, double p2,
+                                              const Kernel& kern, double* v, bool* inside) {
+    if (!nb.gas) return false; // gas neighbours only
+    const double d0 = nb.x - p0, d1 = nb.y - p1, d2 = nb.z - p2;
+    const double r = sqrt_rn(d0 * d0 + d1 * d1 + d2 * d2);
+    double w;
+    kern.at(r, &w, &v[1]);
     v[0] = w;
-    v[1] = kernel_dwdh(r, h, dim);
-    v[2] = a.m[j] * w;
+    v[2] = nb.m * w;
     v[3] = d0 * d0 * w;
     v[4] = d1 * d1 * w;
     v[5] = d2 * d2 * w;
@@ -195,7 +270,7 @@ __device__ __forceinline__ bool density_terms(const DensArgs& a, uint32_t j, dou
     v[9] = d0 * w;
     v[10] = d1 * w;
     v[11] = d2 * w;
-    *inside = r < h;
+    *inside = r < kern.h;
     return true;
 }
 
@@ -205,18 +280,28 @@ struct DensSums {
     int n_inside;
 };
 
+// A target's solve between steps: its radius, the bracket, the iteration.
+struct DensState {
+    double h, lo, hi;
+    int it;
+};
+
 // The rest of one step (hydro.cc:218-296) from the target's sums: the final pass's outputs when
 // out of iterations, else the corrections, the convergence test and the Newton / bisection step.
-__device__ void density_update(const DensArgs& a, int k, uint32_t t, uint32_t p, double h, int it,
-                               const DensSums& S) {
+// True: the target is done (its outputs written by a lane with `write`, its radius is st.h).
+__device__ bool density_step(const DensArgs& a, uint32_t t, uint32_t p, DensState& st,
+                             const DensSums& S, bool write) {
     const int dim = a.n_dims;
+    const double h = st.h;
+    const int it = st.it;
     if (it >= kMaxIter) {
         // out of iterations: rho and the count at the last h (hydro.cc:285-295)
-        a.rho[t] = S.s[2];
-        a.nngb[t] = S.n_inside;
-        a.iters[t] = kMaxIter;
-        a.keep[k] = 0;
-        return;
+        if (write) {
+            a.rho[t] = S.s[2];
+            a.nngb[t] = S.n_inside;
+            a.iters[t] = kMaxIter;
+        }
+        return true;
     }
     const double weight_sum = S.s[0], dweight_dh = S.s[1];
     const double* mom = S.s + 3;
@@ -258,13 +343,14 @@ __device__ void density_update(const DensArgs& a, int k, uint32_t t, uint32_t p,
         tol_eff = fmin(0.25 * des_eff, tol_eff * exp(0.1 * log(des_eff / (16.0 * tol_eff)) * it));
     const double residual = n_eff - des_eff;
     if (fabs(residual) < tol_eff) {
-        a.rho[t] = S.s[2];
-        a.nngb[t] = S.n_inside;
-        a.iters[t] = it;
-        a.keep[k] = 0;
-        return;
+        if (write) {
+            a.rho[t] = S.s[2];
+            a.nngb[t] = S.n_inside;
+            a.iters[t] = it;
+        }
+        return true;
     }
-    double h_lo = a.h_lo[t], h_hi = a.h_hi[t];
+    double h_lo = st.lo, h_hi = st.hi;
     if (residual > 0) h_hi = h;
     else h_lo = h;
     // Newton on N_eff(h), guarded by the bracket (hydro.cc:271-281)
@@ -274,11 +360,42 @@ __device__ void density_update(const DensArgs& a, int k, uint32_t t, uint32_t p,
         if (h_hi > 0) h_next = (h_lo > 0) ? sqrt(h_lo * h_hi) : 0.5 * h_hi;
         else h_next = h * ((residual > 0) ? 0.7 : 1.6);
     }
-    a.h[t] = h_next;
-    a.h_lo[t] = h_lo;
-    a.h_hi[t] = h_hi;
-    a.iter[t] = it + 1;
+    st = {h_next, h_lo, h_hi, it + 1};
+    return false;
+}
+
+// A step whose state lives in memory; keep: the target (entry k of the active list) goes on.
+__device__ void density_update(const DensArgs& a, int k, uint32_t t, uint32_t p, double h, int it,
+                               const DensSums& S) {
+    DensState st{h, a.h_lo[t], a.h_hi[t], it};
+    if (density_step(a, t, p, st, S, true)) {
+        a.keep[k] = 0;
+        return;
+    }
+    a.h[t] = st.h;
+    a.h_lo[t] = st.lo;
+    a.h_hi[t] = st.hi;
+    a.iter[t] = st.it;
     a.keep[k] = 1;
+}
+
+// Packed sums: the neighbours' terms lie in s_v in traversal order, and lane c < 12 adds term c of
+// each to acc. Eight are read together: the additions stay in order, their reads do not wait for
+// each other.
+__device__ __forceinline__ double add_terms(const double (*s_v)[65], int lane, int n, double acc) {
+    if (lane < kTerms) {
+        const double* v = s_v[lane];
+        int i = 0;
+        for (; i + 8 <= n; i += 8) {
+            double u[8];
+#pragma unroll
+            for (int j = 0; j < 8; ++j) u[j] = v[i + j];
+#pragma unroll
+            for (int j = 0; j < 8; ++j) acc += u[j];
+        }
+        for (; i < n; ++i) acc += v[i];
+    }
+    return acc;
 }
 
 // One step for each of its targets (a.act[e] for block e), one wavefront per target walking that
@@ -287,13 +404,12 @@ __device__ void density_update(const DensArgs& a, int k, uint32_t t, uint32_t p,
 // among a node's children up to its next admitted interior child are taken together, their
 // particles (contiguous slot ranges) spread over the lanes in slot order, tested against the
 // sphere, and the neighbours' terms computed into LDS in that order. Lane c (c < 12) then adds
-// term c of each, in order, and lane 12 counts those inside h, so every sum is the round's, term
-// by term. For the targets whose spheres reach far beyond their leaf, and for the last few
-// targets: with LOOP, the wave repeats its target's steps until the target is done.
+// term c of each, in order, so every sum is the round's, term by term. For the targets whose
+// spheres reach far beyond their leaf; with LOOP, the wave repeats its target's steps until the
+// target is done.
 template <bool LOOP>
 __global__ __launch_bounds__(64) void k_density_far(DensArgs a) {
     __shared__ double s_v[kTerms][65]; // rows padded so the 12 adding lanes hit distinct banks
-    __shared__ int s_in[64];
     const int lane = threadIdx.x;
     const int e = blockIdx.x;
     const int dim = a.n_dims;
@@ -306,6 +422,8 @@ __global__ __launch_bounds__(64) void k_density_far(DensArgs a) {
         const double h = a.h[t];
         const int it = a.iter[t];
         const double r2 = h * h; // the search's radius_sq (hydro.cc:50)
+        Kernel kern;
+        kern.set(h, dim);
         // the node test of the forward search (hydro.cc:55-72), as the rounds evaluate it
         auto admits = [&](const SRec& nr) -> bool {
             double dist = h + (double)nr.half + (double)nr.xpad;
@@ -319,15 +437,11 @@ __global__ __launch_bounds__(64) void k_density_far(DensArgs a) {
             return !(dx * dx + dy * dy + dz * dz > ds * ds);
         };
         double acc = 0.0; // lane c < 12: term c's sum
-        int n_in = 0;     // lane 12: the count inside h
+        int n_in = 0;     // the count inside h (the same in every lane)
         int nbuf = 0;     // neighbours waiting in s_v (the same in every lane)
         auto flush = [&]() {
             __syncthreads();
-            if (lane < kTerms) {
-                for (int i = 0; i < nbuf; ++i) acc += s_v[lane][i];
-            } else if (lane == kTerms) {
-                for (int i = 0; i < nbuf; ++i) n_in += s_in[i];
-            }
+            acc = add_terms(s_v, lane, nbuf, acc);
             __syncthreads();
             nbuf = 0;
         };
@@ -341,18 +455,18 @@ __global__ __launch_bounds__(64) void k_density_far(DensArgs a) {
                 const double4 q = a.src[s];
                 const double ex = q.x - qx, ey = q.y - qy, ez = q.z - qz;
                 if (ex * ex + ey * ey + ez * ez < r2)
-                    ok = density_terms(a, a.orderbuf[s], qx, qy, qz, h, dim, v, &inside);
+                    ok = density_terms(neighbour_at(a, s), qx, qy, qz, kern, v, &inside);
             }
             const uint64_t om = __ballot(ok);
             if (om == 0) return;
             const int n_ok = __builtin_popcountll(om);
             if (nbuf + n_ok > 64) flush();
             if (ok) {
-                const int pos = nbuf + __builtin_popcountll(om & ((1ull << lane) - 1));
+                const int pos = nbuf + lanes_under(om);
 #pragma unroll
                 for (int c = 0; c < kTerms; ++c) s_v[c][pos] = v[c];
-                s_in[pos] = inside ? 1 : 0;
             }
+            n_in += __builtin_popcountll(__ballot(ok && inside));
             nbuf += n_ok;
         };
         // the admitted leaves run (bit j: child cf + j), their particles in slot order
@@ -467,7 +581,7 @@ __global__ __launch_bounds__(64) void k_density_far(DensArgs a) {
         DensSums S;
 #pragma unroll
         for (int c = 0; c < kTerms; ++c) S.s[c] = __shfl(acc, c);
-        S.n_inside = __shfl(n_in, kTerms);
+        S.n_inside = n_in;
         if (lane == 0) density_update(a, e, t, p, h, it, S);
         if (!LOOP) break;
         __syncthreads(); // the update's state, written by lane 0, for every lane
@@ -475,11 +589,207 @@ __global__ __launch_bounds__(64) void k_density_far(DensArgs a) {
     }
 }
 
+// The last kLoopTargets targets, a wavefront each (target a.act[e] for block e), iterated to the
+// end. The wave collects its target's candidates once, out to kNearMargin times the radius, up to
+// 64 nodes in depth-first order at a time, and keeps them in registers (candidate 64 k + lane), in
+// slot order: a step is then a distance test and the terms of those inside, without the tree, until
+// the radius outgrows the collection. (Targets that run to the 100-iteration cap, whose walks one
+// node at a time set the launch's time, took 39 us a step before, and 2-3 us now.) When some
+// particle has left its cell the candidates are collected for each step at its own radius, under
+// the reference's node tests. A sphere of more than kNearMax candidates is left to k_density_far
+// (appended to far_list, its state in memory).
+constexpr int kNearSlots = 4; // candidates a lane holds
+constexpr int kNearMax = 64 * kNearSlots;
+constexpr double kNearMargin = 1.15;
+__global__ __launch_bounds__(64, 3) void k_density_near(DensArgs a) {
+    // the collection's stack and leaf runs, then a step's packed terms
+    __shared__ union {
+        double v[kTerms][65];
+        struct {
+            int stk[kDensStack], lpre[64], lplo[64];
+        } w;
+    } s;
+    __shared__ uint32_t s_cand[kNearMax];
+    const int lane = threadIdx.x;
+    const int e = blockIdx.x;
+    const uint32_t t = a.act[e];
+    const uint32_t p = a.targets[t];
+    const double qx = a.x[p], qy = a.y[p], qz = a.z[p];
+    const bool fresh = *a.moved == 0;
+    DensState st{a.h[t], a.h_lo[t], a.h_hi[t], a.iter[t]};
+    double cx[kNearSlots], cy[kNearSlots], cz[kNearSlots]; // the tree's copy of the positions
+    Neighbour nb[kNearSlots];
+    int nc = 0;
+    double hc = 0.0;   // the radius the candidates reach
+    bool have = false; // they can serve another step
+
+    for (;;) {
+        if (!have || !(st.h <= hc)) {
+            // collect: the search at radius hc, its particles tested against the sphere
+            hc = (fresh && st.h > 0) ? st.h * kNearMargin : st.h;
+            const double c2 = hc * hc;
+            nc = 0;
+            int r_next = (a.nclusters > 1) ? 0 : a.root;
+            const int r_end = (a.nclusters > 1) ? a.nclusters : a.root + 1;
+            int sp = 0;
+            while (nc <= kNearMax) {
+                __syncthreads();
+                if (sp == 0) {
+                    if (r_next == r_end) break;
+                    sp = min(64, r_end - r_next);
+                    if (lane < sp) s.w.stk[sp - 1 - lane] = r_next + lane;
+                    r_next += sp;
+                    __syncthreads();
+                }
+                // (the stack, its window and its bound are k_density_round's)
+                const int w = min(sp, max(1, min(64, (kDensStack - kDensSpare - sp) / 7)));
+                int ent = 0;
+                if (lane < w) ent = s.w.stk[sp - 1 - lane];
+                const uint64_t leaf_m = __ballot(lane < w && ent < 0);
+                const int run = (~leaf_m == 0) ? 64 : (int)__builtin_ctzll(~leaf_m);
+                if (run < kDensRun && run < w) {
+                    int n = 0, link = 0;
+                    if (lane < w && ent < 0) {
+                        n = 1;
+                    } else if (lane < w) {
+                        const SRec r = a.srec[ent];
+                        double dist = hc + (double)r.half + (double)r.xpad;
+                        if (a.tau > 0) dist += (double)r.vmax * a.tau;
+                        const double dx = (double)r.cx - qx, dy = (double)r.cy - qy,
+                                     dz = (double)r.cz - qz;
+                        const double ds = dist + 0.7320508075688772 * (double)r.half;
+                        if (!(dx > dist || -dx > dist) && !(dy > dist || -dy > dist) &&
+                            !(dz > dist || -dz > dist) &&
+                            !(dx * dx + dy * dy + dz * dz > ds * ds)) {
+                            link = r.link;
+                            n = (link < 0) ? 1 : r.span;
+                            if (link < 0) ent = ~ent;
+                        }
+                    }
+                    int total;
+                    const int off = wave_excl_scan(n, total);
+                    const int top = sp - w + total - 1;
+                    __syncthreads();
+                    if (n > 0 && ent < 0) {
+                        s.w.stk[top - off] = ent;
+                    } else {
+                        for (int j = 0; j < n; ++j) s.w.stk[top - off - j] = link + j;
+                    }
+                    sp = top + 1;
+                    continue;
+                }
+                sp -= run;
+                int plo = 0, cnt = 0;
+                if (lane < run) {
+                    const SRec r = a.srec[~ent];
+                    plo = ~r.link;
+                    cnt = r.span - plo;
+                }
+                const uint64_t some = __ballot(cnt > 0);
+                int total;
+                const int off = wave_excl_scan(cnt, total);
+                if (cnt > 0) {
+                    const int li = lanes_under(some);
+                    s.w.lpre[li] = off;
+                    s.w.lplo[li] = plo;
+                }
+                __syncthreads();
+                const int nleaf = __builtin_popcountll(some);
+                for (int g0 = 0; g0 < total; g0 += 64) {
+                    const int g = g0 + lane;
+                    bool in = false;
+                    int slot = 0;
+                    if (g < total) {
+                        int lo_ = 0, hi_ = nleaf; // the last leaf li with lpre[li] <= g
+                        while (hi_ - lo_ > 1) {
+                            const int mid = (lo_ + hi_) >> 1;
+                            if (s.w.lpre[mid] <= g) lo_ = mid;
+                            else hi_ = mid;
+                        }
+                        slot = s.w.lplo[lo_] + (g - s.w.lpre[lo_]);
+                        const double4 q = a.src[slot];
+                        const double ex = q.x - qx, ey = q.y - qy, ez = q.z - qz;
+                        in = ex * ex + ey * ey + ez * ez < c2;
+                    }
+                    const uint64_t im = __ballot(in);
+                    const int pos = nc + lanes_under(im);
+                    if (in && pos < kNearMax) s_cand[pos] = (uint32_t)slot;
+                    nc += __builtin_popcountll(im);
+                }
+            }
+            if (nc > kNearMax) {
+                if (lane == 0) {
+                    a.h[t] = st.h;
+                    a.h_lo[t] = st.lo;
+                    a.h_hi[t] = st.hi;
+                    a.iter[t] = st.it;
+                    a.keep[e] = 0; // k_density_far takes it to the end
+                    a.far_list[atomicAdd(a.n_far, 1u)] = (uint32_t)e;
+                }
+                return;
+            }
+#pragma unroll
+            for (int k = 0; k < kNearSlots; ++k) {
+                if (64 * k + lane < nc) {
+                    const uint32_t slot = s_cand[64 * k + lane];
+                    const double4 q = a.src[slot];
+                    cx[k] = q.x; cy[k] = q.y; cz[k] = q.z;
+                    nb[k] = neighbour_at(a, slot);
+                }
+            }
+            have = fresh;
+        }
+        const double r2 = st.h * st.h;
+        Kernel kern;
+        kern.set(st.h, a.n_dims);
+        double acc = 0.0;
+        int n_in = 0, nbuf = 0;
+#pragma unroll
+        for (int k = 0; k < kNearSlots; ++k) {
+            if (64 * k >= nc) break;
+            double v[kTerms];
+            bool inside = false, ok = false;
+            if (64 * k + lane < nc) {
+                const double ex = cx[k] - qx, ey = cy[k] - qy, ez = cz[k] - qz;
+                if (ex * ex + ey * ey + ez * ez < r2)
+                    ok = density_terms(nb[k], qx, qy, qz, kern, v, &inside);
+            }
+            const uint64_t om = __ballot(ok);
+            const int n_ok = __builtin_popcountll(om);
+            if (nbuf + n_ok > 64) {
+                __syncthreads();
+                acc = add_terms(s.v, lane, nbuf, acc);
+                nbuf = 0;
+            }
+            __syncthreads();
+            if (ok) {
+                const int pos = nbuf + lanes_under(om);
+#pragma unroll
+                for (int c = 0; c < kTerms; ++c) s.v[c][pos] = v[c];
+            }
+            n_in += __builtin_popcountll(__ballot(ok && inside));
+            nbuf += n_ok;
+        }
+        __syncthreads();
+        acc = add_terms(s.v, lane, nbuf, acc);
+        __syncthreads();
+        DensSums S;
+#pragma unroll
+        for (int c = 0; c < kTerms; ++c) S.s[c] = __shfl(acc, c);
+        S.n_inside = n_in;
+        if (density_step(a, t, p, st, S, lane == 0)) break;
+    }
+    if (lane == 0) {
+        a.h[t] = st.h;
+        a.keep[e] = 0;
+    }
+}
+
 // One step for every active target (see the top of the file): tpw targets per wavefront, lane l
 // holding active entry wave * tpw + l. A target whose radius reaches far beyond its own leaf would
 // make its wave walk a large part of the tree one node at a time; it is queued for a wave of its
 // own (k_density_far) and takes no part here.
-__global__ __launch_bounds__(64) void k_density_round(DensArgs a) {
+__global__ __launch_bounds__(64, 3) void k_density_round(DensArgs a) {
     const int lane = threadIdx.x;
     // Block b runs on XCD b % 8: each XCD gets one contiguous share of the Morton-ordered waves.
     const int b = blockIdx.x, nb = gridDim.x;
@@ -508,18 +818,25 @@ __global__ __launch_bounds__(64) void k_density_round(DensArgs a) {
             mine = false;
         }
     }
-    // Each lane's neighbours (particle indices, in traversal order) wait in its column of s_nb
-    // until some column is full or the walk ends; then every lane adds its waiting neighbours'
-    // terms, in order. A lane reads back only what it wrote itself, so no barrier is needed.
+    // Each lane's neighbours (slots, in traversal order) wait in its column of s_nb until some
+    // column is full or the walk ends; then every lane adds its waiting neighbours' terms, in
+    // order. A lane reads back only what it wrote itself, so no barrier is needed.
     __shared__ uint32_t s_nb[kNbBuf][64];
+    Kernel kern;
+    kern.set(h, dim);
     DensSums S;
     int nb_n = 0;
     auto flush = [&]() {
-        for (int e = 0; __ballot(e < nb_n) != 0; ++e) {
+        const int most = __builtin_amdgcn_readfirstlane((int)wave_max_i(nb_n));
+        Neighbour next{};
+        if (nb_n > 0) next = neighbour_at(a, s_nb[0][lane]);
+        for (int e = 0; e < most; ++e) {
+            const Neighbour nb = next;
+            if (e + 1 < nb_n) next = neighbour_at(a, s_nb[e + 1][lane]);
             if (e < nb_n) {
                 double v[kTerms];
                 bool inside = false;
-                if (density_terms(a, s_nb[e][lane], qx, qy, qz, h, dim, v, &inside)) {
+                if (density_terms(nb, qx, qy, qz, kern, v, &inside)) {
 #pragma unroll
                     for (int c = 0; c < kTerms; ++c) S.s[c] += v[c];
                     if (inside) ++S.n_inside;
@@ -539,73 +856,167 @@ __global__ __launch_bounds__(64) void k_density_round(DensArgs a) {
 #pragma unroll
     for (int c = 0; c < kTerms; ++c) S.s[c] = 0.0;
     S.n_inside = 0;
-    // The current sibling range (next node, nodes left, lanes waiting on it) and the
-    // ranges above it, entry e in lane e of stf/stc/stl/sth: one per tree level, below the
-    // roots' range (a forest's roots are nodes 0..nc-1, searched in that order).
-    int cf = (a.nclusters > 1) ? 0 : a.root;
-    int cc = (a.nclusters > 1) ? a.nclusters : 1;
-    uint64_t cm = lanes;
+    // the node test of the forward search for this lane's target (hydro.cc:55-72)
+    auto admits = [&](float cx, float cy, float cz, float half, float xpad, float vmax) -> bool {
+        double dist = h + (double)half + (double)xpad;
+        if (a.tau > 0) dist += (double)vmax * a.tau;
+        const double dx = (double)cx - qx, dy = (double)cy - qy, dz = (double)cz - qz;
+        if (!mine || dx > dist || -dx > dist || dy > dist || -dy > dist || dz > dist || -dz > dist)
+            return false;
+        const double ds = dist + 0.7320508075688772 * (double)half;
+        return !(dx * dx + dy * dy + dz * dz > ds * ds);
+    };
+    // the same for all targets at once: their box, their largest radius (a node that any target
+    // admits passes: each step is monotone in the bounds)
+    // (a target with a NaN finds nothing, and stays out of them)
+    const bool sound = mine && qx == qx && qy == qy && qz == qz && h == h;
+    const double lo0 = wave_min_d(sound ? qx : 1e300), hi0 = wave_max_d(sound ? qx : -1e300);
+    const double lo1 = wave_min_d(sound ? qy : 1e300), hi1 = wave_max_d(sound ? qy : -1e300);
+    const double lo2 = wave_min_d(sound ? qz : 1e300), hi2 = wave_max_d(sound ? qz : -1e300);
+    const double hmax = wave_max_d(sound ? h : 0.0);
+
+    // Every particle lies in its build-time cell (or within half the margin that the search nodes
+    // have beyond it): then a particle within the radius is in leaves that the node test admits,
+    // and the test on distance alone picks the reference's neighbours. Otherwise each leaf's node
+    // test is kept per target.
+    const bool fresh = *a.moved == 0;
+
+    // The walk's stack, in depth-first order from its top: nodes still to be tested, and (as ~node)
+    // leaves that the targets' box admits, waiting for the nodes before them.
+    __shared__ int s_stk[kDensStack];
+    __shared__ double4 s_p[64];
+    __shared__ uint32_t s_slot[64];
+    __shared__ uint64_t s_pm[64], s_lm[64]; // the lanes that test a particle / a leaf's particles
+    __shared__ int s_lpre[64], s_lplo[64];
+    const uint32_t bit = 1u << (lane & 31);
+    const uint32_t* pm = reinterpret_cast<const uint32_t*>(s_pm) + (lane >> 5);
+    // the staged particles against every target: a neighbour's slot is written behind the ones a
+    // lane holds, and stays there if it counts (four at a time between checks for room)
+    const double r2t = mine ? r2 : -1.0;
+    auto test4 = [&](int e0, int np, auto allowed) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int e = e0 + j; // (up to 63: entries past np are not counted)
+            const double4 q = s_p[e];
+            const double ex = q.x - qx, ey = q.y - qy, ez = q.z - qz;
+            const bool in = ex * ex + ey * ey + ez * ez < r2t && e < np && allowed(e);
+            s_nb[nb_n][lane] = s_slot[e];
+            nb_n += in ? 1 : 0;
+        }
+    };
+    int r_next = (a.nclusters > 1) ? 0 : a.root; // a forest's roots in order, up to 64 at a time
+    const int r_end = (a.nclusters > 1) ? a.nclusters : a.root + 1;
     int sp = 0;
-    int stf = 0, stc = 0, stl = 0, sth = 0;
     for (;;) {
-        if (cc == 0) {
-            if (sp == 0) break;
-            --sp;
-            cf = __builtin_amdgcn_readlane(stf, sp);
-            cc = __builtin_amdgcn_readlane(stc, sp);
-            cm = ((uint64_t)(uint32_t)__builtin_amdgcn_readlane(sth, sp) << 32) |
-                 (uint64_t)(uint32_t)__builtin_amdgcn_readlane(stl, sp);
+        if (sp == 0) {
+            if (r_next == r_end) break;
+            sp = min(64, r_end - r_next);
+            if (lane < sp) s_stk[sp - 1 - lane] = r_next + lane;
+            r_next += sp;
+            __syncthreads();
         }
-        const int node = cf;
-        ++cf;
-        --cc;
-        const bool wait = (cm >> lane) & 1ull;
-        // the node test of the forward search, per lane (hydro.cc:55-72), exactly as the
-        // device search evaluates it
-        const SRec nr = ld_const(a.srec + node);
-        double dist = h + (double)nr.half + (double)nr.xpad;
-        if (a.tau > 0) dist += (double)nr.vmax * a.tau;
-        const double dx = (double)nr.cx - qx, dy = (double)nr.cy - qy, dz = (double)nr.cz - qz;
-        bool hit = false;
-        if (wait && !(dx > dist || -dx > dist) && !(dy > dist || -dy > dist) &&
-            !(dz > dist || -dz > dist)) {
-            const double ds = dist + 0.7320508075688772 * (double)nr.half;
-            hit = !(dx * dx + dy * dy + dz * dz > ds * ds);
-        }
-        const uint64_t om = __ballot(hit);
-        if (om == 0) continue;
-        if (nr.link < 0) {
-            // the leaf's particles in slot order: a neighbour when within the radius (the
-            // tree's copy of the position, as the search tests it)
-            // (four records loaded together, then noted one by one in slot order)
-            for (int s0 = ~nr.link; s0 < nr.span; s0 += 4) {
-                double4 q[4];
-#pragma unroll
-                for (int j = 0; j < 4; ++j)
-                    if (s0 + j < nr.span) q[j] = ld_const(a.src + s0 + j);
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    if (s0 + j >= nr.span) break;
-                    const double ex = q[j].x - qx, ey = q[j].y - qy, ez = q[j].z - qz;
-                    const bool in = hit && ex * ex + ey * ey + ez * ez < r2;
-                    if (__ballot(in) == 0) continue;
-                    if (__ballot(nb_n == kNbBuf) != 0) flush();
-                    if (in) s_nb[nb_n++][lane] = ld_const(a.orderbuf + s0 + j);
+        // the window: the first w nodes in depth-first order, one per lane. Replacing one by its
+        // children adds at most 7, so a nearly full stack gets a smaller window; at a window of
+        // one it grows by 7 a level at most, which kDensSpare covers.
+        const int w = min(sp, max(1, min(64, (kDensStack - kDensSpare - sp) / 7)));
+        int ent = 0;
+        if (lane < w) ent = s_stk[sp - 1 - lane];
+        const uint64_t leaf_m = __ballot(lane < w && ent < 0);
+        const int run = (~leaf_m == 0) ? 64 : (int)__builtin_ctzll(~leaf_m);
+        if (run < kDensRun && run < w) {
+            // test the window's nodes against the targets' box, the interior ones then for each
+            // target (a box that straddles a jump of the Morton order admits more than any target)
+            SRec r{};
+            int n = 0; // entries that replace this one
+            bool inner = false;
+            if (lane < w) {
+                if (ent < 0) {
+                    n = 1;
+                } else {
+                    r = a.srec[ent];
+                    double dist = hmax + (double)r.half + (double)r.xpad;
+                    if (a.tau > 0) dist += (double)r.vmax * a.tau;
+                    const double c0 = r.cx, c1 = r.cy, c2 = r.cz;
+                    const double d0 = fmax(0.0, fmax(lo0 - c0, c0 - hi0));
+                    const double d1 = fmax(0.0, fmax(lo1 - c1, c1 - hi1));
+                    const double d2 = fmax(0.0, fmax(lo2 - c2, c2 - hi2));
+                    const double ds = dist + 0.7320508075688772 * (double)r.half;
+                    if (d0 <= dist && d1 <= dist && d2 <= dist &&
+                        d0 * d0 + d1 * d1 + d2 * d2 <= ds * ds) {
+                        inner = r.link >= 0;
+                        if (!inner) {
+                            n = 1;
+                            ent = ~ent;
+                        }
+                    }
                 }
             }
+            for (uint64_t rem = __ballot(inner); rem != 0; rem &= rem - 1) {
+                const int l = (int)__builtin_ctzll(rem);
+                const bool hit = admits(lane_f(r.cx, l), lane_f(r.cy, l), lane_f(r.cz, l),
+                                        lane_f(r.half, l), lane_f(r.xpad, l), lane_f(r.vmax, l));
+                if (__ballot(hit) != 0 && lane == l) n = r.span;
+            }
+            int total;
+            const int off = wave_excl_scan(n, total);
+            const int top = sp - w + total - 1;
+            __syncthreads();
+            if (n > 0 && ent < 0) {
+                s_stk[top - off] = ent;
+            } else {
+                for (int j = 0; j < n; ++j) s_stk[top - off - j] = r.link + j;
+            }
+            sp = top + 1;
+            __syncthreads();
             continue;
         }
-        // descend: the node's remaining siblings (if any) wait on the stack below its
-        // children
-        const bool top = lane == sp;
-        stf = top ? cf : stf;
-        stc = top ? cc : stc;
-        stl = top ? (int)(uint32_t)cm : stl;
-        sth = top ? (int)(uint32_t)(cm >> 32) : sth;
-        sp += (cc > 0) ? 1 : 0;
-        cf = nr.link;
-        cc = nr.span;
-        cm = om;
+        // the run of leaves at the top: which targets admit each, and their particles in slot order
+        sp -= run;
+        SRec r{};
+        if (lane < run) r = a.srec[~ent];
+        uint64_t mym = fresh ? ~0ull : 0ull;
+        for (int l = 0; l < run && !fresh; ++l) {
+            const uint64_t m = __ballot(admits(lane_f(r.cx, l), lane_f(r.cy, l), lane_f(r.cz, l),
+                                               lane_f(r.half, l), lane_f(r.xpad, l),
+                                               lane_f(r.vmax, l)));
+            if (lane == l) mym = m;
+        }
+        const int plo = ~r.link, cnt = (lane < run && mym != 0) ? r.span - plo : 0;
+        const uint64_t some = __ballot(cnt > 0);
+        if (some == 0) continue;
+        int total;
+        const int off = wave_excl_scan(cnt, total);
+        if (cnt > 0) {
+            const int li = lanes_under(some);
+            s_lpre[li] = off;
+            s_lplo[li] = plo;
+            s_lm[li] = mym;
+        }
+        __syncthreads();
+        const int nleaf = __builtin_popcountll(some);
+        for (int g0 = 0; g0 < total; g0 += 64) {
+            const int g = g0 + lane;
+            if (g < total) {
+                int lo_ = 0, hi_ = nleaf; // the last leaf li with s_lpre[li] <= g
+                while (hi_ - lo_ > 1) {
+                    const int mid = (lo_ + hi_) >> 1;
+                    if (s_lpre[mid] <= g) lo_ = mid;
+                    else hi_ = mid;
+                }
+                const int slot = s_lplo[lo_] + (g - s_lpre[lo_]);
+                s_p[lane] = a.src[slot];
+                s_slot[lane] = (uint32_t)slot;
+                s_pm[lane] = s_lm[lo_];
+            }
+            __syncthreads();
+            const int np = min(64, total - g0);
+            for (int e0 = 0; e0 < np; e0 += 4) {
+                if (__ballot(nb_n > kNbBuf - 4) != 0) flush();
+                if (fresh) test4(e0, np, [](int) { return true; });
+                else test4(e0, np, [&](int e) { return (pm[2 * e] & bit) != 0; });
+            }
+            __syncthreads();
+        }
     }
     flush();
     if (mine) density_update(a, k, t, p, h, it, S);
@@ -634,6 +1045,33 @@ __global__ __launch_bounds__(256) void k_density_srec(int nn, const WNode* __res
     r.link = (w.first >= 0) ? w.first : ~w.plo;
     r.span = (w.first >= 0) ? w.nchild : w.phi;
     out[i] = r;
+}
+
+// Whether each slot's particle is gas.
+__global__ __launch_bounds__(256) void k_density_gas(size_t nl, const uint32_t* __restrict__ order,
+                                                     const uint8_t* __restrict__ type,
+                                                     uint8_t* __restrict__ gas) {
+    const size_t r = (size_t)blockIdx.x * 256 + threadIdx.x;
+    if (r < nl) gas[r] = type[order[r]] == 0 ? 1 : 0;
+}
+
+// Sets *moved when a slot's position (the tree's copy) lies outside its leaf's cell by more than
+// tol on some axis.
+__global__ __launch_bounds__(256) void k_density_moved(size_t nl, const double4* __restrict__ src,
+                                                       const int* __restrict__ slot_leaf,
+                                                       const double* __restrict__ gcx,
+                                                       const double* __restrict__ gcy,
+                                                       const double* __restrict__ gcz,
+                                                       const double* __restrict__ size, double tol,
+                                                       int* __restrict__ moved) {
+    const size_t r = (size_t)blockIdx.x * 256 + threadIdx.x;
+    if (r >= nl) return;
+    const double4 q = src[r];
+    const int leaf = slot_leaf[r];
+    const double lim = 0.5 * size[leaf] + tol;
+    const bool in = fabs(q.x - gcx[leaf]) <= lim && fabs(q.y - gcy[leaf]) <= lim &&
+                    fabs(q.z - gcz[leaf]) <= lim; // (false for a NaN)
+    if (!in) *moved = 1;
 }
 
 // Start state: every target active at its first guess; a target outside the particle set flags
@@ -761,6 +1199,10 @@ extern "C" gz_status gz_tree_density(gz_ctx* ctx, const gz_tree* tree, const gz_
         off += (bytes + 255) & ~size_t(255);
         return o;
     };
+    // Many targets: the particles' live values are put in slot order first, where the targets of a
+    // wave find their neighbours together (a neighbour's four values cost four scattered reads
+    // otherwise, several times a call)
+    const bool by_slot = n_t >= tree->n_live / 8;
     const size_t o_lo = take(n_t * 8), o_hi = take(n_t * 8), o_iter = take(n_t * 4),
                  o_act = take(n_t * 4), o_nxt = take(n_t * 4), o_keep = take((n_t + 1) * 4),
                  o_scan = take((n_t + 1) * 4), o_kept = take((n_t + 1) * 4),
@@ -768,6 +1210,8 @@ extern "C" gz_status gz_tree_density(gz_ctx* ctx, const gz_tree* tree, const gz_
                  o_v0 = take(n_t * 4), o_v1 = take(n_t * 4), o_far = take(n_t * 4),
                  o_fact = take(n_t * 4), o_fkeep = take(n_t * 4),
                  o_srec = take((size_t)std::max(tree->nnodes, 1) * sizeof(SRec)),
+                 o_live = take(by_slot ? tree->n_live * sizeof(double4) : 0),
+                 o_gas = take(by_slot && p->type ? tree->n_live : 0),
                  o_misc = take(256), o_tmp = take(scan_tmp_bytes(n_t + 1));
     DevMem& mem = ctx->scratch[13];
     GZ_TRY(mem.reserve(off));
@@ -785,6 +1229,7 @@ extern "C" gz_status gz_tree_density(gz_ctx* ctx, const gz_tree* tree, const gz_
     int* d_status = reinterpret_cast<int*>(base + o_misc + 128);
     int* d_sort = reinterpret_cast<int*>(base + o_misc + 192); // bit 1: bad index; [1]: unsorted
     uint32_t* d_nfar = reinterpret_cast<uint32_t*>(base + o_misc + 224);
+    int* d_moved = reinterpret_cast<int*>(base + o_misc + 240);
     uint32_t* d_far = reinterpret_cast<uint32_t*>(base + o_far);
     uint32_t* d_fact = reinterpret_cast<uint32_t*>(base + o_fact);
     uint32_t* d_fkeep = reinterpret_cast<uint32_t*>(base + o_fkeep);
@@ -866,11 +1311,29 @@ extern "C" gz_status gz_tree_density(gz_ctx* ctx, const gz_tree* tree, const gz_
     a.far_list = d_far;
     a.n_far = d_nfar;
     a.srec = reinterpret_cast<const SRec*>(base + o_srec);
+    const double snode_eps = 1e-6 * tree->root_box[3];
     if (tree->nnodes > 0) {
         k_density_srec<<<(unsigned)((tree->nnodes + 255) / 256), 256, 0, st>>>(
             tree->nnodes, tree->wn, tree->gcx, tree->gcy, tree->gcz, tree->size, tree->xpad,
-            tree->vmax, 1e-6 * tree->root_box[3], reinterpret_cast<SRec*>(base + o_srec));
+            tree->vmax, snode_eps, reinterpret_cast<SRec*>(base + o_srec));
         GZ_HIP(hipGetLastError());
+    }
+    if (tree->n_live > 0) {
+        k_density_moved<<<(unsigned)((tree->n_live + 255) / 256), 256, 0, st>>>(
+            tree->n_live, tree->src, tree->slot_leaf, tree->gcx, tree->gcy, tree->gcz, tree->size,
+            0.5 * snode_eps, d_moved);
+        GZ_HIP(hipGetLastError());
+    }
+    a.moved = d_moved;
+    if (by_slot && tree->n_live > 0) {
+        GZ_TRY(gather_live(ctx, p, tree, reinterpret_cast<double4*>(base + o_live)));
+        a.live = reinterpret_cast<const double4*>(base + o_live);
+        if (p->type) {
+            k_density_gas<<<(unsigned)((tree->n_live + 255) / 256), 256, 0, st>>>(
+                tree->n_live, tree->orderbuf, p->type, base + o_gas);
+            GZ_HIP(hipGetLastError());
+            a.live_gas = base + o_gas;
+        }
     }
     a.wn = tree->wn;
     a.size = tree->size;
@@ -895,14 +1358,12 @@ extern "C" gz_status gz_tree_density(gz_ctx* ctx, const gz_tree* tree, const gz_
         a.tpw = tpw;
         const bool loop = n_act <= kLoopTargets;
         GZ_TRY(fill_zero_u32(d_nfar, 1, st));
-        if (loop) k_density_far<true><<<n_act, 64, 0, st>>>(a);
+        if (loop) k_density_near<<<n_act, 64, 0, st>>>(a);
         else k_density_round<<<(n_act + tpw - 1) / tpw, 64, 0, st>>>(a);
         GZ_HIP(hipGetLastError());
         uint32_t n_far = 0;
-        if (!loop) {
-            GZ_HIP(hipMemcpyAsync(&n_far, d_nfar, sizeof n_far, hipMemcpyDeviceToHost, st));
-            GZ_HIP(hipStreamSynchronize(st));
-        }
+        GZ_HIP(hipMemcpyAsync(&n_far, d_nfar, sizeof n_far, hipMemcpyDeviceToHost, st));
+        GZ_HIP(hipStreamSynchronize(st));
         if (n_far > 0) {
             // the far targets: a wave each, in the round's order (their keep flags are then
             // moved to the round's positions)
@@ -913,11 +1374,13 @@ extern "C" gz_status gz_tree_density(gz_ctx* ctx, const gz_tree* tree, const gz_
             f.act = d_fact;
             f.n_act = (int)n_far;
             f.keep = d_fkeep;
-            k_density_far<false><<<n_far, 64, 0, st>>>(f);
+            if (loop) k_density_far<true><<<n_far, 64, 0, st>>>(f);
+            else k_density_far<false><<<n_far, 64, 0, st>>>(f);
             GZ_HIP(hipGetLastError());
             k_density_far_keep<<<gf, 256, 0, st>>>((int)n_far, d_far, d_fkeep, d_keep);
             GZ_HIP(hipGetLastError());
         }
+        if (loop) break; // every target is done
         // the targets still active, in their order: kept positions, then their target indices
         GZ_TRY(exclusive_scan_u32(d_keep, d_scan, n_act, d_total, base + o_tmp, st, d_kept));
         uint32_t n_next = 0;

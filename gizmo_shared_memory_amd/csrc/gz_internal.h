@@ -412,5 +412,7 @@ struct gz_tree {
 namespace gz {
 gz_status build_tree(gz_ctx* ctx, const gz_particles* p, const gz_build_opts* opts, gz_tree* t);
 gz_status regather_sources(gz_ctx* ctx, const gz_particles* p, gz_tree* t);
+// (x, y, z, m) of p in t's slot order.
+gz_status gather_live(gz_ctx* ctx, const gz_particles* p, const gz_tree* t, double4* out);
 void tree_release(gz_tree* t);
 } // namespace gz
