@@ -38,6 +38,7 @@
 
 #include "gz_features.h"
 #include "gz_internal.h"
+#include "gz_spheres.h"
 #include "gz_wave.h"
 
 namespace gz {
@@ -47,9 +48,6 @@ constexpr double kPi = 3.14159265358979323846;
 constexpr int kMaxIter = 100; // hydro.cc:201
 constexpr int kWavesWanted = 2048; // a round's targets are spread thinner below this many waves
 constexpr int kNbBuf = 32;          // neighbours each lane holds before their terms are added
-constexpr int kDensStack = 640;     // entries of a round wave's stack ...
-constexpr int kDensSpare = 160;     // ... of which a window of one node may need 7 a level
-constexpr int kDensRun = 16;        // leaves taken together, when as many are next in order
 constexpr double kFarLeaf = 4.0;    // radius over leaf side beyond which a target takes the lists
 // Active targets few enough to iterate in one launch. Rounds are cheaper per target while a wave's
 // targets are neighbours; the fewer are left, the further apart they lie and the more launches and
@@ -158,15 +156,6 @@ __device__ __forceinline__ bool invert_moments(const double* e, double* b, int d
     return true;
 }
 
-// One search node as the fused rounds read it: one 32-byte scalar load per visit. The centre and
-// half side are the float search node's (tree.cc:496-506); xpad and vmax as the tree holds them;
-// link is the first child, or ~plo for a leaf, and span the child count, or phi for a leaf.
-struct alignas(32) SRec {
-    float cx, cy, cz, half;
-    float xpad, vmax;
-    int link, span;
-};
-
 // A read of memory no kernel of the solve writes (the tree's records), through the constant
 // address space: at a wave-uniform address it is a scalar load, served by the scalar cache.
 template <class T>
@@ -208,32 +197,20 @@ struct DensArgs {
     // the tree: its search nodes (built per call), the side of each node (the far test), the
     // sorted copy of the particles and their indices, the roots, and the time since the build
     // (the vmax pad)
-    const SRec* srec;
+    SphereNodes nodes;
     const WNode* wn;
     const double* size;
     const double4* src;
     const uint32_t* orderbuf;
-    int root, nclusters;
-    double tau;
-    const int* moved; // nonzero: some particle lies outside its build-time cell
 };
 
 // The terms one gas neighbour j adds to a target at (p0, p1, p2) with support h (hydro.cc:206-217):
 // v = {W, dW/dh, m W, dx dx W, dy dy W, dz dz W, dx dy W, dy dz W, dx dz W, dx W, dy W, dz W}, and
 // whether r < h. Non-gas neighbours add nothing (returns false).
 constexpr int kTerms = 12;
-// Lane l's value, as a scalar; the wave's largest value.
-__device__ __forceinline__ float lane_f(float v, int l) {
-    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
-}
 __device__ __forceinline__ int wave_max_i(int v) {
     for (int d = 32; d >= 1; d >>= 1) v = max(v, __shfl_xor(v, d));
     return v;
-}
-// Set bits of m below this lane.
-__device__ __forceinline__ int lanes_under(uint64_t m) {
-    return (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32),
-                                          __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
 }
 struct Neighbour {
     double x, y, z, m;
@@ -416,8 +393,8 @@ __global__ __launch_bounds__(64) void k_density_far(DensArgs a) {
     const uint32_t t = a.act[e];
     const uint32_t p = a.targets[t];
     const double qx = a.x[p], qy = a.y[p], qz = a.z[p];
-    const int r_first = (a.nclusters > 1) ? 0 : a.root;
-    const int r_count = (a.nclusters > 1) ? a.nclusters : 1;
+    const int r_first = (a.nodes.nclusters > 1) ? 0 : a.nodes.root;
+    const int r_count = (a.nodes.nclusters > 1) ? a.nodes.nclusters : 1;
     for (;;) {
         const double h = a.h[t];
         const int it = a.iter[t];
@@ -427,7 +404,7 @@ __global__ __launch_bounds__(64) void k_density_far(DensArgs a) {
         // the node test of the forward search (hydro.cc:55-72), as the rounds evaluate it
         auto admits = [&](const SRec& nr) -> bool {
             double dist = h + (double)nr.half + (double)nr.xpad;
-            if (a.tau > 0) dist += (double)nr.vmax * a.tau;
+            if (a.nodes.tau > 0) dist += (double)nr.vmax * a.nodes.tau;
             const double dx = (double)nr.cx - qx, dy = (double)nr.cy - qy,
                          dz = (double)nr.cz - qz;
             if ((dx > dist || -dx > dist) || (dy > dist || -dy > dist) ||
@@ -473,7 +450,7 @@ __global__ __launch_bounds__(64) void k_density_far(DensArgs a) {
         auto leaves = [&](int cf, uint64_t run) {
             int plo = 0, cnt = 0, off = 0, total = 0;
             if ((run >> lane) & 1ull) {
-                const SRec c = a.srec[cf + lane];
+                const SRec c = a.nodes.srec[cf + lane];
                 plo = ~c.link;
                 cnt = c.span - plo;
             }
@@ -516,7 +493,7 @@ __global__ __launch_bounds__(64) void k_density_far(DensArgs a) {
             {
                 bool hit = false, leaf = false;
                 if (lane < min(64, r_count - r0)) {
-                    const SRec c = a.srec[cf + lane];
+                    const SRec c = a.nodes.srec[cf + lane];
                     hit = admits(c);
                     leaf = c.link < 0;
                 }
@@ -548,7 +525,7 @@ __global__ __launch_bounds__(64) void k_density_far(DensArgs a) {
                 // siblings, which wait on the stack
                 const int node = cf + (int)__builtin_ctzll(cm);
                 cm &= cm - 1;
-                const SRec nr = ld_const(a.srec + node);
+                const SRec nr = ld_const(a.nodes.srec + node);
                 if (inside_sphere(nr)) {
                     const WNode w = ld_const(a.wn + node);
                     for (int s0 = w.plo; s0 < w.phi; s0 += 64)
@@ -557,7 +534,7 @@ __global__ __launch_bounds__(64) void k_density_far(DensArgs a) {
                 }
                 bool hit = false, leaf = false;
                 if (lane < nr.span) {
-                    const SRec c = a.srec[nr.link + lane];
+                    const SRec c = a.nodes.srec[nr.link + lane];
                     hit = admits(c);
                     leaf = c.link < 0;
                 }
@@ -606,7 +583,7 @@ __global__ __launch_bounds__(64, 3) void k_density_near(DensArgs a) {
     __shared__ union {
         double v[kTerms][65];
         struct {
-            int stk[kDensStack], lpre[64], lplo[64];
+            int stk[kSphStack], lpre[64], lplo[64];
         } w;
     } s;
     __shared__ uint32_t s_cand[kNearMax];
@@ -615,7 +592,7 @@ __global__ __launch_bounds__(64, 3) void k_density_near(DensArgs a) {
     const uint32_t t = a.act[e];
     const uint32_t p = a.targets[t];
     const double qx = a.x[p], qy = a.y[p], qz = a.z[p];
-    const bool fresh = *a.moved == 0;
+    const bool fresh = *a.nodes.moved == 0;
     DensState st{a.h[t], a.h_lo[t], a.h_hi[t], a.iter[t]};
     double cx[kNearSlots], cy[kNearSlots], cz[kNearSlots]; // the tree's copy of the positions
     Neighbour nb[kNearSlots];
@@ -629,8 +606,8 @@ __global__ __launch_bounds__(64, 3) void k_density_near(DensArgs a) {
             hc = (fresh && st.h > 0) ? st.h * kNearMargin : st.h;
             const double c2 = hc * hc;
             nc = 0;
-            int r_next = (a.nclusters > 1) ? 0 : a.root;
-            const int r_end = (a.nclusters > 1) ? a.nclusters : a.root + 1;
+            int r_next = (a.nodes.nclusters > 1) ? 0 : a.nodes.root;
+            const int r_end = (a.nodes.nclusters > 1) ? a.nodes.nclusters : a.nodes.root + 1;
             int sp = 0;
             while (nc <= kNearMax) {
                 __syncthreads();
@@ -642,19 +619,19 @@ __global__ __launch_bounds__(64, 3) void k_density_near(DensArgs a) {
                     __syncthreads();
                 }
                 // (the stack, its window and its bound are k_density_round's)
-                const int w = min(sp, max(1, min(64, (kDensStack - kDensSpare - sp) / 7)));
+                const int w = min(sp, max(1, min(64, (kSphStack - kSphSpare - sp) / 7)));
                 int ent = 0;
                 if (lane < w) ent = s.w.stk[sp - 1 - lane];
                 const uint64_t leaf_m = __ballot(lane < w && ent < 0);
                 const int run = (~leaf_m == 0) ? 64 : (int)__builtin_ctzll(~leaf_m);
-                if (run < kDensRun && run < w) {
+                if (run < kSphRun && run < w) {
                     int n = 0, link = 0;
                     if (lane < w && ent < 0) {
                         n = 1;
                     } else if (lane < w) {
-                        const SRec r = a.srec[ent];
+                        const SRec r = a.nodes.srec[ent];
                         double dist = hc + (double)r.half + (double)r.xpad;
-                        if (a.tau > 0) dist += (double)r.vmax * a.tau;
+                        if (a.nodes.tau > 0) dist += (double)r.vmax * a.nodes.tau;
                         const double dx = (double)r.cx - qx, dy = (double)r.cy - qy,
                                      dz = (double)r.cz - qz;
                         const double ds = dist + 0.7320508075688772 * (double)r.half;
@@ -681,7 +658,7 @@ __global__ __launch_bounds__(64, 3) void k_density_near(DensArgs a) {
                 sp -= run;
                 int plo = 0, cnt = 0;
                 if (lane < run) {
-                    const SRec r = a.srec[~ent];
+                    const SRec r = a.nodes.srec[~ent];
                     plo = ~r.link;
                     cnt = r.span - plo;
                 }
@@ -856,195 +833,31 @@ __global__ __launch_bounds__(64, 3) void k_density_round(DensArgs a) {
 #pragma unroll
     for (int c = 0; c < kTerms; ++c) S.s[c] = 0.0;
     S.n_inside = 0;
-    // the node test of the forward search for this lane's target (hydro.cc:55-72)
-    auto admits = [&](float cx, float cy, float cz, float half, float xpad, float vmax) -> bool {
-        double dist = h + (double)half + (double)xpad;
-        if (a.tau > 0) dist += (double)vmax * a.tau;
-        const double dx = (double)cx - qx, dy = (double)cy - qy, dz = (double)cz - qz;
-        if (!mine || dx > dist || -dx > dist || dy > dist || -dy > dist || dz > dist || -dz > dist)
-            return false;
-        const double ds = dist + 0.7320508075688772 * (double)half;
-        return !(dx * dx + dy * dy + dz * dz > ds * ds);
-    };
-    // the same for all targets at once: their box, their largest radius (a node that any target
-    // admits passes: each step is monotone in the bounds)
-    // (a target with a NaN finds nothing, and stays out of them)
-    const bool sound = mine && qx == qx && qy == qy && qz == qz && h == h;
-    const double lo0 = wave_min_d(sound ? qx : 1e300), hi0 = wave_max_d(sound ? qx : -1e300);
-    const double lo1 = wave_min_d(sound ? qy : 1e300), hi1 = wave_max_d(sound ? qy : -1e300);
-    const double lo2 = wave_min_d(sound ? qz : 1e300), hi2 = wave_max_d(sound ? qz : -1e300);
-    const double hmax = wave_max_d(sound ? h : 0.0);
-
-    // Every particle lies in its build-time cell (or within half the margin that the search nodes
-    // have beyond it): then a particle within the radius is in leaves that the node test admits,
-    // and the test on distance alone picks the reference's neighbours. Otherwise each leaf's node
-    // test is kept per target.
-    const bool fresh = *a.moved == 0;
-
-    // The walk's stack, in depth-first order from its top: nodes still to be tested, and (as ~node)
-    // leaves that the targets' box admits, waiting for the nodes before them.
-    __shared__ int s_stk[kDensStack];
-    __shared__ double4 s_p[64];
-    __shared__ uint32_t s_slot[64];
-    __shared__ uint64_t s_pm[64], s_lm[64]; // the lanes that test a particle / a leaf's particles
-    __shared__ int s_lpre[64], s_lplo[64];
-    const uint32_t bit = 1u << (lane & 31);
-    const uint32_t* pm = reinterpret_cast<const uint32_t*>(s_pm) + (lane >> 5);
     // the staged particles against every target: a neighbour's slot is written behind the ones a
     // lane holds, and stays there if it counts (four at a time between checks for room)
+    __shared__ SphereLds lds;
     const double r2t = mine ? r2 : -1.0;
-    auto test4 = [&](int e0, int np, auto allowed) {
+    walk_spheres(a.nodes, mine, qx, qy, qz, h, lds, nullptr, [&](int np, auto allowed) {
+        for (int e0 = 0; e0 < np; e0 += 4) {
+            if (__ballot(nb_n > kNbBuf - 4) != 0) flush();
+            auto test4 = [&](auto ok) {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int e = e0 + j; // (up to 63: entries past np are not counted)
-            const double4 q = s_p[e];
-            const double ex = q.x - qx, ey = q.y - qy, ez = q.z - qz;
-            const bool in = ex * ex + ey * ey + ez * ez < r2t && e < np && allowed(e);
-            s_nb[nb_n][lane] = s_slot[e];
-            nb_n += in ? 1 : 0;
-        }
-    };
-    int r_next = (a.nclusters > 1) ? 0 : a.root; // a forest's roots in order, up to 64 at a time
-    const int r_end = (a.nclusters > 1) ? a.nclusters : a.root + 1;
-    int sp = 0;
-    for (;;) {
-        if (sp == 0) {
-            if (r_next == r_end) break;
-            sp = min(64, r_end - r_next);
-            if (lane < sp) s_stk[sp - 1 - lane] = r_next + lane;
-            r_next += sp;
-            __syncthreads();
-        }
-        // the window: the first w nodes in depth-first order, one per lane. Replacing one by its
-        // children adds at most 7, so a nearly full stack gets a smaller window; at a window of
-        // one it grows by 7 a level at most, which kDensSpare covers.
-        const int w = min(sp, max(1, min(64, (kDensStack - kDensSpare - sp) / 7)));
-        int ent = 0;
-        if (lane < w) ent = s_stk[sp - 1 - lane];
-        const uint64_t leaf_m = __ballot(lane < w && ent < 0);
-        const int run = (~leaf_m == 0) ? 64 : (int)__builtin_ctzll(~leaf_m);
-        if (run < kDensRun && run < w) {
-            // test the window's nodes against the targets' box, the interior ones then for each
-            // target (a box that straddles a jump of the Morton order admits more than any target)
-            SRec r{};
-            int n = 0; // entries that replace this one
-            bool inner = false;
-            if (lane < w) {
-                if (ent < 0) {
-                    n = 1;
-                } else {
-                    r = a.srec[ent];
-                    double dist = hmax + (double)r.half + (double)r.xpad;
-                    if (a.tau > 0) dist += (double)r.vmax * a.tau;
-                    const double c0 = r.cx, c1 = r.cy, c2 = r.cz;
-                    const double d0 = fmax(0.0, fmax(lo0 - c0, c0 - hi0));
-                    const double d1 = fmax(0.0, fmax(lo1 - c1, c1 - hi1));
-                    const double d2 = fmax(0.0, fmax(lo2 - c2, c2 - hi2));
-                    const double ds = dist + 0.7320508075688772 * (double)r.half;
-                    if (d0 <= dist && d1 <= dist && d2 <= dist &&
-                        d0 * d0 + d1 * d1 + d2 * d2 <= ds * ds) {
-                        inner = r.link >= 0;
-                        if (!inner) {
-                            n = 1;
-                            ent = ~ent;
-                        }
-                    }
+                for (int j = 0; j < 4; ++j) {
+                    const int e = e0 + j; // (up to 63: entries past np are not counted)
+                    const double4 q = lds.p[e];
+                    const double ex = q.x - qx, ey = q.y - qy, ez = q.z - qz;
+                    const bool in = ex * ex + ey * ey + ez * ez < r2t && e < np && ok(e);
+                    s_nb[nb_n][lane] = lds.id[e];
+                    nb_n += in ? 1 : 0;
                 }
-            }
-            for (uint64_t rem = __ballot(inner); rem != 0; rem &= rem - 1) {
-                const int l = (int)__builtin_ctzll(rem);
-                const bool hit = admits(lane_f(r.cx, l), lane_f(r.cy, l), lane_f(r.cz, l),
-                                        lane_f(r.half, l), lane_f(r.xpad, l), lane_f(r.vmax, l));
-                if (__ballot(hit) != 0 && lane == l) n = r.span;
-            }
-            int total;
-            const int off = wave_excl_scan(n, total);
-            const int top = sp - w + total - 1;
-            __syncthreads();
-            if (n > 0 && ent < 0) {
-                s_stk[top - off] = ent;
-            } else {
-                for (int j = 0; j < n; ++j) s_stk[top - off - j] = r.link + j;
-            }
-            sp = top + 1;
-            __syncthreads();
-            continue;
+            };
+            if (allowed.all) test4([](int) { return true; });
+            else test4(allowed);
         }
-        // the run of leaves at the top: which targets admit each, and their particles in slot order
-        sp -= run;
-        SRec r{};
-        if (lane < run) r = a.srec[~ent];
-        uint64_t mym = fresh ? ~0ull : 0ull;
-        for (int l = 0; l < run && !fresh; ++l) {
-            const uint64_t m = __ballot(admits(lane_f(r.cx, l), lane_f(r.cy, l), lane_f(r.cz, l),
-                                               lane_f(r.half, l), lane_f(r.xpad, l),
-                                               lane_f(r.vmax, l)));
-            if (lane == l) mym = m;
-        }
-        const int plo = ~r.link, cnt = (lane < run && mym != 0) ? r.span - plo : 0;
-        const uint64_t some = __ballot(cnt > 0);
-        if (some == 0) continue;
-        int total;
-        const int off = wave_excl_scan(cnt, total);
-        if (cnt > 0) {
-            const int li = lanes_under(some);
-            s_lpre[li] = off;
-            s_lplo[li] = plo;
-            s_lm[li] = mym;
-        }
-        __syncthreads();
-        const int nleaf = __builtin_popcountll(some);
-        for (int g0 = 0; g0 < total; g0 += 64) {
-            const int g = g0 + lane;
-            if (g < total) {
-                int lo_ = 0, hi_ = nleaf; // the last leaf li with s_lpre[li] <= g
-                while (hi_ - lo_ > 1) {
-                    const int mid = (lo_ + hi_) >> 1;
-                    if (s_lpre[mid] <= g) lo_ = mid;
-                    else hi_ = mid;
-                }
-                const int slot = s_lplo[lo_] + (g - s_lpre[lo_]);
-                s_p[lane] = a.src[slot];
-                s_slot[lane] = (uint32_t)slot;
-                s_pm[lane] = s_lm[lo_];
-            }
-            __syncthreads();
-            const int np = min(64, total - g0);
-            for (int e0 = 0; e0 < np; e0 += 4) {
-                if (__ballot(nb_n > kNbBuf - 4) != 0) flush();
-                if (fresh) test4(e0, np, [](int) { return true; });
-                else test4(e0, np, [&](int e) { return (pm[2 * e] & bit) != 0; });
-            }
-            __syncthreads();
-        }
-    }
+    });
     flush();
     if (mine) density_update(a, k, t, p, h, it, S);
     if (far) a.far_list[atomicAdd(a.n_far, 1u)] = (uint32_t)k;
-}
-
-// The search nodes of the fused rounds, one per tree node.
-__global__ __launch_bounds__(256) void k_density_srec(int nn, const WNode* __restrict__ wn,
-                                                      const double* __restrict__ gcx,
-                                                      const double* __restrict__ gcy,
-                                                      const double* __restrict__ gcz,
-                                                      const double* __restrict__ size,
-                                                      const float* __restrict__ xpad,
-                                                      const float* __restrict__ vmax,
-                                                      double snode_eps, SRec* __restrict__ out) {
-    const int i = blockIdx.x * 256 + threadIdx.x;
-    if (i >= nn) return;
-    const WNode w = wn[i];
-    SRec r;
-    r.cx = (float)gcx[i];
-    r.cy = (float)gcy[i];
-    r.cz = (float)gcz[i];
-    r.half = snode_half_of(gcx[i], gcy[i], gcz[i], size[i], snode_eps);
-    r.xpad = xpad[i];
-    r.vmax = vmax[i];
-    r.link = (w.first >= 0) ? w.first : ~w.plo;
-    r.span = (w.first >= 0) ? w.nchild : w.phi;
-    out[i] = r;
 }
 
 // Whether each slot's particle is gas.
@@ -1053,25 +866,6 @@ __global__ __launch_bounds__(256) void k_density_gas(size_t nl, const uint32_t* 
                                                      uint8_t* __restrict__ gas) {
     const size_t r = (size_t)blockIdx.x * 256 + threadIdx.x;
     if (r < nl) gas[r] = type[order[r]] == 0 ? 1 : 0;
-}
-
-// Sets *moved when a slot's position (the tree's copy) lies outside its leaf's cell by more than
-// tol on some axis.
-__global__ __launch_bounds__(256) void k_density_moved(size_t nl, const double4* __restrict__ src,
-                                                       const int* __restrict__ slot_leaf,
-                                                       const double* __restrict__ gcx,
-                                                       const double* __restrict__ gcy,
-                                                       const double* __restrict__ gcz,
-                                                       const double* __restrict__ size, double tol,
-                                                       int* __restrict__ moved) {
-    const size_t r = (size_t)blockIdx.x * 256 + threadIdx.x;
-    if (r >= nl) return;
-    const double4 q = src[r];
-    const int leaf = slot_leaf[r];
-    const double lim = 0.5 * size[leaf] + tol;
-    const bool in = fabs(q.x - gcx[leaf]) <= lim && fabs(q.y - gcy[leaf]) <= lim &&
-                    fabs(q.z - gcz[leaf]) <= lim; // (false for a NaN)
-    if (!in) *moved = 1;
 }
 
 // Start state: every target active at its first guess; a target outside the particle set flags
@@ -1310,21 +1104,8 @@ extern "C" gz_status gz_tree_density(gz_ctx* ctx, const gz_tree* tree, const gz_
     a.slot_leaf = tree->slot_leaf;
     a.far_list = d_far;
     a.n_far = d_nfar;
-    a.srec = reinterpret_cast<const SRec*>(base + o_srec);
-    const double snode_eps = 1e-6 * tree->root_box[3];
-    if (tree->nnodes > 0) {
-        k_density_srec<<<(unsigned)((tree->nnodes + 255) / 256), 256, 0, st>>>(
-            tree->nnodes, tree->wn, tree->gcx, tree->gcy, tree->gcz, tree->size, tree->xpad,
-            tree->vmax, snode_eps, reinterpret_cast<SRec*>(base + o_srec));
-        GZ_HIP(hipGetLastError());
-    }
-    if (tree->n_live > 0) {
-        k_density_moved<<<(unsigned)((tree->n_live + 255) / 256), 256, 0, st>>>(
-            tree->n_live, tree->src, tree->slot_leaf, tree->gcx, tree->gcy, tree->gcz, tree->size,
-            0.5 * snode_eps, d_moved);
-        GZ_HIP(hipGetLastError());
-    }
-    a.moved = d_moved;
+    GZ_TRY(launch_sphere_nodes(tree, tau, reinterpret_cast<SRec*>(base + o_srec), d_moved,
+                               &a.nodes, st));
     if (by_slot && tree->n_live > 0) {
         GZ_TRY(gather_live(ctx, p, tree, reinterpret_cast<double4*>(base + o_live)));
         a.live = reinterpret_cast<const double4*>(base + o_live);
@@ -1339,9 +1120,6 @@ extern "C" gz_status gz_tree_density(gz_ctx* ctx, const gz_tree* tree, const gz_
     a.size = tree->size;
     a.src = tree->src;
     a.orderbuf = tree->orderbuf;
-    a.root = tree->root;
-    a.nclusters = tree->n_clusters;
-    a.tau = tau;
 
     // rounds: a target takes at most 100 steps and one last search
     uint32_t n_act = (uint32_t)n_t;

@@ -3,21 +3,22 @@
 // whose own kernel reaches centre q although q's does not (ngb_search_reverse, with the node
 // hmax of Tree::init_hmax / raise_hmax, tree.cc:286-338).
 //
-// One wavefront per group of 64 consecutive queries. Up to 64 stacked nodes are tested at once,
-// one per lane: first against the group's bounding box with the group's largest radius (for the
-// reverse search: the node's hmax, and only if it exceeds the group's smallest kernel radius),
-// then with the reference's own node test for each query of the group in turn, a node staying
-// only if some query admits it — so the wave walks the union of its queries' traversals even when
-// the group straddles a jump of the Morton order. Node boxes are the reference's SNode boxes
-// (half side widened for float centres) grown by vmax * tau + xpad. The particles of kept leaves
-// are staged through LDS 64 at a time and each lane tests its own query against every staged
-// particle with the reference's FP64 expression, so the sets are exact. Two passes: counts, then
-// (with the offsets) the sorted slots of each query's neighbours, which map to particle indices
-// in Morton order, the reference's traversal order.
+// The forward search is walk_spheres (gz_spheres.h) with a lane per query (below). The reverse
+// search takes one wavefront per group of 64 consecutive queries: up to 64 stacked nodes are tested
+// at once, one per lane, first against the group's bounding box with the node's hmax (and only if
+// it exceeds the group's smallest kernel radius), then with the reference's own node test for
+// each query of the group in turn, a node staying only if some query admits it — so the wave walks
+// the union of its queries' traversals even when the group straddles a jump of the Morton order.
+// Node boxes are the reference's SNode boxes (half side widened for float centres) grown by
+// vmax * tau + xpad. The particles of kept leaves are staged through LDS 64 at a time and each lane
+// tests its own query against every staged particle with the reference's FP64 expression, so the
+// sets are exact. Two passes: counts, then (with the offsets) the sorted slots of each query's
+// neighbours, which map to particle indices in Morton order, the reference's traversal order.
 #include <cfloat>
 
 #include "gz_features.h"
 #include "gz_internal.h"
+#include "gz_spheres.h"
 #include "gz_wave.h"
 
 namespace gz {
@@ -43,7 +44,7 @@ struct NgbArgs {
     uint32_t* count;     // pass 1: neighbours per query
     const size_t* start; // pass 2: CSR offsets
     uint32_t* slots;     // pass 2: the neighbours' sorted slots
-    // reverse search: node hmax, the gas kernel radii by particle, the gas count
+    // node hmax, the gas kernel radii by particle, the gas count
     const float* hmax;
     const double* h;
     size_t n_gas;
@@ -54,12 +55,11 @@ __device__ __forceinline__ float snode_half(const NgbArgs& a, int i) {
     return snode_half_of(a.gcx[i], a.gcy[i], a.gcz[i], a.size[i], a.snode_eps);
 }
 
-// REV: the reverse search (hydro.cc:110-148). radius[q] is then the query's own kernel radius h_q,
-// a node is a candidate only when its hmax exceeds the smallest h_q of the group, its reach is
-// hmax instead of the query radius, and a leaf particle j counts when it is gas and
-// h_q <= r < h[j].
-template <bool FILL, bool REV>
-__global__ __launch_bounds__(64) void k_ngb(NgbArgs a) {
+// The reverse search (hydro.cc:110-148): radius[q] is the query's own kernel radius h_q, a node is a
+// candidate only when its hmax exceeds the smallest h_q of the group, its reach is hmax, and a
+// leaf particle j counts when it is gas and h_q <= r < h[j].
+template <bool FILL>
+__global__ __launch_bounds__(64) void k_ngb_rev(NgbArgs a) {
     __shared__ int s_lpre[64], s_lplo[64]; // kept leaves: first staged index, first slot
     __shared__ double s_px[64], s_py[64], s_pz[64], s_h2[64];
     __shared__ int s_slot[64];
@@ -80,8 +80,7 @@ __global__ __launch_bounds__(64) void k_ngb(NgbArgs a) {
         const double lo0 = wave_min_d(live ? qx : 1e300), hi0 = wave_max_d(live ? qx : -1e300);
         const double lo1 = wave_min_d(live ? qy : 1e300), hi1 = wave_max_d(live ? qy : -1e300);
         const double lo2 = wave_min_d(live ? qz : 1e300), hi2 = wave_max_d(live ? qz : -1e300);
-        const double rmax = wave_max_d(live ? r : 0.0);
-        const double rmin = REV ? wave_min_d(live ? r : 1e300) : 0.0;
+        const double rmin = wave_min_d(live ? r : 1e300);
         const double r2 = r * r;
         uint32_t found = 0;
         size_t out = live && FILL ? a.start[q] : 0;
@@ -114,15 +113,15 @@ __global__ __launch_bounds__(64) void k_ngb(NgbArgs a) {
             if (node >= 0) {
                 const WNode w = a.wn[node];
                 const float half = snode_half(a, node);
-                const double hm = REV ? (double)a.hmax[node] : 0.0;
-                double dist = (REV ? hm : rmax) + (double)half + (double)a.xpad[node];
+                const double hm = (double)a.hmax[node];
+                double dist = hm + (double)half + (double)a.xpad[node];
                 if (a.tau > 0) dist += (double)a.vmax[node] * a.tau;
                 const double c0 = (double)(float)a.gcx[node], c1 = (double)(float)a.gcy[node],
                              c2 = (double)(float)a.gcz[node];
                 const double d0 = fmax(0.0, fmax(lo0 - c0, c0 - hi0));
                 const double d1 = fmax(0.0, fmax(lo1 - c1, c1 - hi1));
                 const double d2 = fmax(0.0, fmax(lo2 - c2, c2 - hi2));
-                if ((!REV || hm > rmin) && d0 <= dist && d1 <= dist && d2 <= dist) {
+                if (hm > rmin && d0 <= dist && d1 <= dist && d2 <= dist) {
                     const double ds = dist + 0.7320508075688772 * (double)half;
                     keep = d0 * d0 + d1 * d1 + d2 * d2 <= ds * ds;
                 }
@@ -154,10 +153,10 @@ __global__ __launch_bounds__(64) void k_ngb(NgbArgs a) {
                     rem &= rem - 1;
                     const double b0 = __shfl(nc0, sl), b1 = __shfl(nc1, sl), b2 = __shfl(nc2, sl);
                     const double bh = __shfl(nhalf, sl), bx = __shfl(nxpad, sl);
-                    const double bv = __shfl(nvmax, sl), bm = REV ? __shfl(nhm, sl) : 0.0;
+                    const double bv = __shfl(nvmax, sl), bm = __shfl(nhm, sl);
                     bool hit = false;
-                    if (live && (!REV || bm > r)) {
-                        double dist = (REV ? bm : r) + bh + bx;
+                    if (live && bm > r) {
+                        double dist = bm + bh + bx;
                         if (a.tau > 0) dist += bv * a.tau;
                         const double dx = b0 - qx, dy = b1 - qy, dz = b2 - qz;
                         if (!(dx > dist || -dx > dist) && !(dy > dist || -dy > dist) &&
@@ -212,18 +211,16 @@ __global__ __launch_bounds__(64) void k_ngb(NgbArgs a) {
                         s_py[lane] = p.y;
                         s_pz[lane] = p.z;
                         s_slot[lane] = s;
-                        if (REV) {
-                            const uint32_t j = a.orderbuf[s];
-                            const double hj = (j < a.n_gas) ? a.h[j] : 0.0;
-                            s_h2[lane] = (j < a.n_gas) ? hj * hj : -1.0; // -1: not gas
-                        }
+                        const uint32_t j = a.orderbuf[s];
+                        const double hj = (j < a.n_gas) ? a.h[j] : 0.0;
+                        s_h2[lane] = (j < a.n_gas) ? hj * hj : -1.0; // -1: not gas
                     }
                     __syncthreads();
                     const int cnt = min(64, ptot - base);
                     for (int e = 0; e < cnt; ++e) {
                         const double ex = s_px[e] - qx, ey = s_py[e] - qy, ez = s_pz[e] - qz;
                         const double d2 = ex * ex + ey * ey + ez * ez;
-                        const bool in = REV ? (d2 >= r2 && d2 < s_h2[e]) : (d2 < r2);
+                        const bool in = d2 >= r2 && d2 < s_h2[e];
                         if (live && in) {
                             if (FILL) a.slots[out++] = (uint32_t)s_slot[e];
                             ++found;
@@ -357,25 +354,35 @@ __global__ void k_u32_to_size(int n, const uint32_t* __restrict__ in, size_t* __
 }
 
 // The sum of the per-query counts in 64 bits (the 32-bit scan that makes the offsets would wrap
-// past 2^32 - 1 pairs): a grid-stride sum per thread, a wave sum, one atomic per wave.
+// past 2^32 - 1 pairs): a grid-stride sum per thread, one atomic per workgroup.
 // The largest count too, which picks how the lists are sorted.
 __global__ __launch_bounds__(256) void k_sum_counts(int n, const uint32_t* __restrict__ in,
                                                     unsigned long long* __restrict__ out,
                                                     uint32_t* __restrict__ max_out) {
-    long long s = 0;
+    __shared__ unsigned long long ss[4];
+    __shared__ uint32_t sm[4];
+    unsigned long long s = 0;
     uint32_t mx = 0;
     for (int i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256) {
         s += in[i];
         mx = max(mx, in[i]);
     }
     for (int d = 32; d >= 1; d >>= 1) {
-        s += __shfl_xor(s, d);
+        s += (unsigned long long)__shfl_xor((long long)s, d);
         mx = max(mx, (uint32_t)__shfl_xor((int)mx, d));
     }
     if ((threadIdx.x & 63) == 0) {
-        if (s) atomicAdd(out, (unsigned long long)s);
-        if (mx) atomicMax(max_out, mx);
+        ss[threadIdx.x >> 6] = s;
+        sm[threadIdx.x >> 6] = mx;
     }
+    __syncthreads();
+    if (threadIdx.x != 0) return;
+    for (int k = 1; k < 4; ++k) {
+        s += ss[k];
+        mx = max(mx, sm[k]);
+    }
+    if (s) atomicAdd(out, s);
+    if (mx) atomicMax(max_out, mx);
 }
 
 // h rounded up to float, so that the float bound stays one-sided (tree.cc:286-290).
@@ -384,6 +391,138 @@ __device__ __forceinline__ float h_as_bound(double h) {
     return ((double)f < h) ? nextafterf(f, 1e30f) : f;
 }
 
+// ---- the forward search ----------------------------------------------------------------------------
+// A lane per query, 64 consecutive queries per wave, on walk_spheres: a query meets its neighbours
+// in slot order, which is its list's order. The first launch counts them and keeps the first
+// kNgbRow in a row per query, so that a list is found, counted and ordered in one walk; only
+// queries with longer lists are walked again (FILL), straight into their place in the CSR.
+constexpr int kNgbRow = 64;
+constexpr size_t kNgbRowsMax = size_t(1) << 30; // bytes of rows beyond which every list is walked twice
+
+struct NgbFwd {
+    SphereNodes nodes;
+    const double *cx, *cy, *cz, *radius;
+    const uint32_t* orderbuf;
+    int nq, qpw;
+    uint32_t* count;
+    uint32_t* rows; // kNgbRow per query, or NULL
+    const size_t* start;
+    uint32_t* found;
+};
+
+template <bool FILL>
+__global__ __launch_bounds__(64) void k_ngb_fwd(NgbFwd a) {
+    __shared__ SphereLds lds;
+    const int lane = threadIdx.x;
+    // Block b runs on XCD b % 8: each XCD gets one contiguous share of the queries.
+    const int b = blockIdx.x, nb = gridDim.x;
+    const int xcd = b & 7, per = nb >> 3, rem = nb & 7;
+    const int q = (xcd * per + min(xcd, rem) + (b >> 3)) * a.qpw + lane;
+    bool mine = lane < a.qpw && q < a.nq;
+    uint32_t* out = nullptr;
+    if (FILL) {
+        if (mine) {
+            const size_t s = a.start[q];
+            out = a.found + s;
+            mine = a.start[q + 1] - s > (size_t)(a.rows ? kNgbRow : 0);
+        }
+        if (__ballot(mine) == 0) return;
+    } else if (a.rows && mine) {
+        out = a.rows + (size_t)q * kNgbRow;
+    }
+    double qx = 0, qy = 0, qz = 0, r = 0;
+    if (mine) {
+        qx = a.cx[q]; qy = a.cy[q]; qz = a.cz[q];
+        r = a.radius[q];
+    }
+    const double r2 = mine ? r * r : -1.0;
+    const uint32_t room = FILL ? 0xFFFFFFFFu : (a.rows ? (uint32_t)kNgbRow : 0u);
+    uint32_t n = 0;
+    walk_spheres(a.nodes, mine, qx, qy, qz, r, lds, a.orderbuf, [&](int np, auto allowed) {
+        auto test = [&](auto ok) {
+#pragma unroll 4
+            for (int e = 0; e < np; ++e) {
+                const double4 p = lds.p[e];
+                const double ex = p.x - qx, ey = p.y - qy, ez = p.z - qz;
+                if (ex * ex + ey * ey + ez * ez < r2 && ok(e)) {
+                    if (n < room) out[n] = lds.id[e];
+                    ++n;
+                }
+            }
+        };
+        if (allowed.all) test([](int) { return true; });
+        else test(allowed);
+    });
+    if (!FILL && mine) a.count[q] = n;
+}
+
+// The rows into their places: half a wave per query, those with longer lists left to the FILL
+// launch.
+__global__ __launch_bounds__(256) void k_ngb_rows(int nq, const size_t* __restrict__ start,
+                                                  const uint32_t* __restrict__ rows,
+                                                  uint32_t* __restrict__ found) {
+    const int lane = threadIdx.x & 31;
+    for (int q = blockIdx.x * 8 + (threadIdx.x >> 5); q < nq; q += gridDim.x * 8) {
+        const size_t s = start[q];
+        const int n = (int)min((size_t)(kNgbRow + 1), start[q + 1] - s);
+        if (n > kNgbRow) continue;
+        const uint32_t* row = rows + (size_t)q * kNgbRow;
+        if (lane < n) found[s + lane] = row[lane];
+        if (lane + 32 < n) found[s + lane + 32] = row[lane + 32];
+    }
+}
+
+// The search nodes, one per tree node.
+__global__ __launch_bounds__(256) void k_sphere_nodes(int nn, const WNode* __restrict__ wn,
+                                                      const double* __restrict__ gcx,
+                                                      const double* __restrict__ gcy,
+                                                      const double* __restrict__ gcz,
+                                                      const double* __restrict__ size,
+                                                      const float* __restrict__ xpad,
+                                                      const float* __restrict__ vmax,
+                                                      double snode_eps, SRec* __restrict__ out) {
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i >= nn) return;
+    out[i] = search_node(wn, gcx, gcy, gcz, size, xpad, vmax, snode_eps, i);
+}
+
+// Sets *moved when a slot's position (the tree's copy) lies outside its leaf's cell by more than
+// tol on some axis.
+__global__ __launch_bounds__(256) void k_sphere_moved(size_t nl, const double4* __restrict__ src,
+                                                       const int* __restrict__ slot_leaf,
+                                                       const double* __restrict__ gcx,
+                                                       const double* __restrict__ gcy,
+                                                       const double* __restrict__ gcz,
+                                                       const double* __restrict__ size, double tol,
+                                                       int* __restrict__ moved) {
+    const size_t r = (size_t)blockIdx.x * 256 + threadIdx.x;
+    if (r >= nl) return;
+    const double4 q = src[r];
+    const int leaf = slot_leaf[r];
+    const double lim = 0.5 * size[leaf] + tol;
+    const bool in = fabs(q.x - gcx[leaf]) <= lim && fabs(q.y - gcy[leaf]) <= lim &&
+                    fabs(q.z - gcz[leaf]) <= lim; // (false for a NaN)
+    if (!in) *moved = 1;
+}
+
+gz_status launch_sphere_nodes(const gz_tree* t, double tau, SRec* srec, int* moved,
+                              SphereNodes* out, hipStream_t st) {
+    const double snode_eps = 1e-6 * t->root_box[3];
+    *out = {srec, moved, t->wn, t->gcx, t->gcy, t->gcz, t->size, t->xpad, t->vmax,
+            snode_eps, t->src, t->root, t->n_clusters, tau};
+    if (!srec) return GZ_OK;
+    if (t->nnodes > 0)
+        k_sphere_nodes<<<(unsigned)((t->nnodes + 255) / 256), 256, 0, st>>>(
+            t->nnodes, t->wn, t->gcx, t->gcy, t->gcz, t->size, t->xpad, t->vmax, snode_eps, srec);
+    if (t->n_live > 0)
+        k_sphere_moved<<<(unsigned)((t->n_live + 255) / 256), 256, 0, st>>>(
+            t->n_live, t->src, t->slot_leaf, t->gcx, t->gcy, t->gcz, t->size, 0.5 * snode_eps,
+            moved);
+    GZ_HIP(hipGetLastError());
+    return GZ_OK;
+}
+
+// ---- the reverse search's node hmax ---------------------------------------------------------------
 // init_hmax (tree.cc:332-338): each leaf takes the largest rounded-up h of its gas particles (an
 // atomic max on the float's bits, which order like the values for h >= 0), then each level from
 // the bottom takes the largest of its children's. The reference's per-particle climb with an
@@ -442,16 +581,11 @@ using namespace gz;
 
 namespace {
 
-gz_status ngb_pass(NgbArgs& a, bool fill, bool rev, int waves, hipStream_t st) {
+gz_status ngb_rev_pass(NgbArgs& a, bool fill, int waves, hipStream_t st) {
     GZ_TRY(fill_zero_u32(reinterpret_cast<uint32_t*>(a.queue), 2, st));
     const int grid = std::max(1, std::min(waves, a.ngroups));
-    if (rev) {
-        if (fill) k_ngb<true, true><<<grid, 64, 0, st>>>(a);
-        else k_ngb<false, true><<<grid, 64, 0, st>>>(a);
-    } else {
-        if (fill) k_ngb<true, false><<<grid, 64, 0, st>>>(a);
-        else k_ngb<false, false><<<grid, 64, 0, st>>>(a);
-    }
+    if (fill) k_ngb_rev<true><<<grid, 64, 0, st>>>(a);
+    else k_ngb_rev<false><<<grid, 64, 0, st>>>(a);
     GZ_HIP(hipGetLastError());
     return GZ_OK;
 }
@@ -495,7 +629,15 @@ static gz_status ngb_run(gz_ctx* ctx, const gz_tree* tree, const double* cx, con
     }
     DevMem& s = ctx->scratch[10];
     const size_t cnt_bytes = ((n_q + 1) * sizeof(uint32_t) + 255) & ~size_t(255);
-    GZ_TRY(s.reserve(cnt_bytes + 256 + scan_tmp_bytes(n_q + 1)));
+    const size_t tmp_bytes = (256 + scan_tmp_bytes(n_q + 1) + 255) & ~size_t(255);
+    // forward: the search nodes, and a row per query unless the caller has room for longer lists
+    // (packing reads the whole tree, 75 us at 4M particles: for a few queries it would be most of
+    // the search)
+    const bool packed = !rev && n_q >= tree->n_live / 16;
+    const size_t srec_bytes = packed ? (size_t)tree->nnodes * sizeof(SRec) : 0;
+    const size_t row_bytes = n_q * kNgbRow * sizeof(uint32_t);
+    const bool rows = !rev && found && cap / kNgbRow <= n_q && row_bytes <= kNgbRowsMax;
+    GZ_TRY(s.reserve(cnt_bytes + tmp_bytes + srec_bytes + (rows ? row_bytes : 0)));
     uint8_t* b = s.as<uint8_t>();
     uint32_t* count = reinterpret_cast<uint32_t*>(b);
     int* misc = reinterpret_cast<int*>(b + cnt_bytes);
@@ -531,8 +673,28 @@ static gz_status ngb_run(gz_ctx* ctx, const gz_tree* tree, const double* cx, con
     unsigned long long* total64 = reinterpret_cast<unsigned long long*>(misc + 4);
     uint32_t* max_count = reinterpret_cast<uint32_t*>(misc + 6);
     GZ_TRY(fill_zero_u32(reinterpret_cast<uint32_t*>(total64), 3, st));
-    GZ_TRY(ngb_pass(a, false, rev, waves, st));
-    k_sum_counts<<<(unsigned)std::min<size_t>(1024, (n_q + 255) / 256), 256, 0, st>>>(
+    NgbFwd f{};
+    const unsigned fgrid = (unsigned)a.ngroups;
+    if (rev) {
+        GZ_TRY(ngb_rev_pass(a, false, waves, st));
+    } else {
+        GZ_TRY(fill_zero_u32(reinterpret_cast<uint32_t*>(misc), 9, st));
+        GZ_TRY(launch_sphere_nodes(
+            tree, tau, packed ? reinterpret_cast<SRec*>(b + cnt_bytes + tmp_bytes) : nullptr,
+            packed ? misc + 8 : nullptr, &f.nodes, st));
+        f.cx = cx; f.cy = cy; f.cz = cz; f.radius = radius;
+        f.orderbuf = tree->orderbuf;
+        f.nq = a.nq;
+        f.qpw = a.qpw;
+        f.count = count;
+        f.rows = rows ? reinterpret_cast<uint32_t*>(b + cnt_bytes + tmp_bytes + srec_bytes)
+                      : nullptr;
+        f.start = start;
+        f.found = found;
+        k_ngb_fwd<false><<<fgrid, 64, 0, st>>>(f);
+        GZ_HIP(hipGetLastError());
+    }
+    k_sum_counts<<<(unsigned)std::min<size_t>(256, (n_q + 255) / 256), 256, 0, st>>>(
         (int)n_q, count, total64, max_count);
     GZ_HIP(hipGetLastError());
     // offsets: exclusive scan of the counts (count[n_q] = 0 gives the total at start[n_q])
@@ -564,12 +726,25 @@ static gz_status ngb_run(gz_ctx* ctx, const gz_tree* tree, const double* cx, con
                     "queries", who, h_total);
     *total = tot32;
     if (!found || cap < (size_t)tot32 || tot32 == 0) return GZ_OK;
+    if (!rev) {
+        if (rows) {
+            k_ngb_rows<<<(unsigned)std::min<size_t>((n_q + 7) / 8, 16384), 256, 0, st>>>(
+                (int)n_q, start, f.rows, found);
+            GZ_HIP(hipGetLastError());
+        }
+        if (!rows || h_max > (uint32_t)kNgbRow) {
+            k_ngb_fwd<true><<<fgrid, 64, 0, st>>>(f);
+            GZ_HIP(hipGetLastError());
+        }
+        GZ_HIP(hipStreamSynchronize(st));
+        return GZ_OK;
+    }
     // pass 2: the neighbours' slots, then sorted and mapped to particle indices
     DevMem& sl = ctx->scratch[11];
     GZ_TRY(sl.reserve((size_t)tot32 * sizeof(uint32_t)));
     a.start = start;
     a.slots = sl.as<uint32_t>();
-    GZ_TRY(ngb_pass(a, true, rev, waves, st));
+    GZ_TRY(ngb_rev_pass(a, true, waves, st));
     if (h_max > (uint32_t)kFinishLds && (size_t)tot32 <= kRadixFinishMax) {
         DevMem& kb = ctx->scratch[15];
         const size_t nk = tot32;

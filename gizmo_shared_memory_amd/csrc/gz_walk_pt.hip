@@ -58,12 +58,6 @@ __global__ __launch_bounds__(256) void k_pt_keys(const uint32_t* __restrict__ ta
     if (i > 0 && slot_of(i - 1) > key) atomicOr(misc + 1, 1);
 }
 
-// Set bits of m below this lane.
-__device__ __forceinline__ int lanes_under(uint64_t m) {
-    return (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32),
-                                          __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
-}
-
 // A pair's term as the factors that a fused multiply-add sums: t0 f, t1 f, t2 f (POT: t0 f). When
 // `use` is false (the target itself) or the two coincide, f is 0 with finite offsets, so every
 // lane runs the same instructions; only pairs inside the kernel branch off.

@@ -33,4 +33,10 @@ __device__ __forceinline__ int wave_excl_scan(int v, int& total) {
     return x - v;
 }
 
+// Set bits of m below this lane.
+__device__ __forceinline__ int lanes_under(uint64_t m) {
+    return (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32),
+                                          __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+}
+
 } // namespace gz
