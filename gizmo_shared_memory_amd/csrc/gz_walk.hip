@@ -201,9 +201,28 @@ __device__ __forceinline__ double uniform_d(double v) {
     return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
 }
 
+// The walk kernel's arguments (they are its only parameter) as its once-a-group code reads them. The
+// compiler loads a by-value argument at the kernel's entry and keeps it in scalar registers
+// throughout; the FP64 walks had some 100 to 150 scalar values too many for that and read them back
+// from vector lanes, 30 to 50 v_readlane per batch of nodes. They read the arguments again from
+// the argument segment instead: 7.89 -> 7.68 ms for 4M Hernquist, the tidal walk of 1M 4.38 ->
+// 4.31. The FP32 walk has fewer, gained nothing (8M learned 5.90 both ways), and keeps them.
+using ArgMem = const __attribute__((address_space(4))) WalkArgs;
+template <bool AGAIN>
+__device__ __forceinline__ auto& group_args(const WalkArgs& a) {
+    if constexpr (AGAIN) {
+        ArgMem* p = (ArgMem*)__builtin_amdgcn_kernarg_segment_ptr();
+        asm volatile("" : "+s"(p)); // not the pointer it was: loads through it are not merged
+        return *p;
+    } else {
+        return a;
+    }
+}
+
 // Position and softening of target slot i: from the tree's sorted copy when the target is in the
 // tree, else from the particle arrays.
-__device__ __forceinline__ void target_data(const WalkArgs& a, int i, double& px, double& py,
+template <class Args>
+__device__ __forceinline__ void target_data(Args& a, int i, double& px, double& py,
                                             double& pz, double& pe) {
     const int s = a.tslot[i];
     if (s >= 0) {
@@ -220,8 +239,8 @@ __device__ __forceinline__ void target_data(const WalkArgs& a, int i, double& px
 // The opening bounds of group g (tree.cc:683-702: bounding box, largest softening, smallest aold),
 // computed by the group's own wavefront. Min and max are exact, so every lane ends with the same
 // values whatever the reduction order. A learned tolerance enters as a factor on aold_min.
-__device__ __forceinline__ GroupInfo group_bounds(const WalkArgs& a, int g, int ngroups,
-                                                  int lane) {
+template <class Args>
+__device__ __forceinline__ GroupInfo group_bounds(Args& a, int g, int ngroups, int lane) {
     const int lo = a.gstart[g];
     const int hi = (g + 1 < ngroups) ? a.gstart[g + 1] : a.nt;
     double bx0 = 1e300, by0 = 1e300, bz0 = 1e300, bx1 = -1e300, by1 = -1e300, bz1 = -1e300;
@@ -356,6 +375,7 @@ __global__ __launch_bounds__(64, TJ ? 3 : ((FP64 && COUNT) ? 4 : 5)) void k_walk
             // groups at a time was slower than single ones: the waves end less evenly.)
             int v = -1;
             if (lane == 0) {
+                int* const queue = group_args<FP64>(a).queue;
                 const int x0 = blockIdx.x & 7;
                 constexpr int C = kXcdChunk;
                 const int nch = (ngroups + C - 1) / C; // chunks; chunk k belongs to XCD k % 8
@@ -363,7 +383,7 @@ __global__ __launch_bounds__(64, TJ ? 3 : ((FP64 && COUNT) ? 4 : 5)) void k_walk
                     const int x = (x0 + k) & 7;
                     const int myc = (nch > x) ? (nch - x + 7) / 8 : 0; // chunks of XCD x
                     const int n = myc * C;
-                    const int c = atomicAdd(&a.queue[x * kQueueStride], 1);
+                    const int c = atomicAdd(&queue[x * kQueueStride], 1);
                     if (c < n) {
                         const int gg = ((c / C) * 8 + x) * C + (c % C);
                         if (gg < ngroups) v = gg;
@@ -385,7 +405,11 @@ __global__ __launch_bounds__(64, TJ ? 3 : ((FP64 && COUNT) ? 4 : 5)) void k_walk
             if (g >= ngroups) break;
         }
 
-        GroupInfo gi = a.groups ? a.groups[g] : group_bounds(a, g, ngroups, lane);
+        GroupInfo gi;
+        {
+            auto& c = group_args<FP64>(a);
+            gi = c.groups ? c.groups[g] : group_bounds(c, g, ngroups, lane);
+        }
         // every field is the same in all lanes: keep them in scalar registers
         for (int k = 0; k < 3; ++k) {
             gi.lo[k] = uniform_d(gi.lo[k]);
@@ -426,7 +450,7 @@ __global__ __launch_bounds__(64, TJ ? 3 : ((FP64 && COUNT) ? 4 : 5)) void k_walk
             double pe_t = 1e300; // the target's softening (FP64), for the uniform-kernel test
             if (tvalid) {
                 double px, py, pz, pe;
-                target_data(a, tlo + t, px, py, pz, pe);
+                target_data(group_args<FP64>(a), tlo + t, px, py, pz, pe);
                 pe_t = pe;
                 if (FP64) {
                     tx = (real)px; ty = (real)py; tz = (real)pz;
@@ -439,16 +463,22 @@ __global__ __launch_bounds__(64, TJ ? 3 : ((FP64 && COUNT) ? 4 : 5)) void k_walk
             double tt[6] = {0}, jj[3] = {0}; // tidal (xx yy zz xy yz xz), jerk (TJ only)
             double tvx = 0, tvy = 0, tvz = 0;
             if (TJ && tvalid && a.jerk) {
-                const uint32_t p = a.targets[tlo + t];
-                tvx = a.pvx[p]; tvy = a.pvy[p]; tvz = a.pvz[p];
+                auto& c = group_args<FP64>(a);
+                const uint32_t p = c.targets[tlo + t];
+                tvx = c.pvx[p]; tvy = c.pvy[p]; tvz = c.pvz[p];
             }
             int mcount = 0, pcount = 0;
             bool overflow = false;
             // FP32: when no particle below the group's root is softer than the chunk's least
             // softened target, every pair's kernel extent max(h_t, h_s) is the target's own, so
             // the particle loop takes h = h_t and its reciprocal powers once per lane
-            const int groot = root_of(a.targets[gi.tlo], a.cluster_start, a.nclusters, a.root);
-            const bool uni = !FP64 && a.node_soft[groot] <= wave_min_d(pe_t);
+            int groot;
+            bool uni = false;
+            {
+                auto& c = group_args<FP64>(a);
+                groot = root_of(c.targets[gi.tlo], c.cluster_start, c.nclusters, c.root);
+                if (!FP64) uni = c.node_soft[groot] <= wave_min_d(pe_t);
+            }
 
             // Evaluate both lists against every target of the chunk.
             auto flush = [&]() {
@@ -765,10 +795,11 @@ __global__ __launch_bounds__(64, TJ ? 3 : ((FP64 && COUNT) ? 4 : 5)) void k_walk
                         if (TJ) {
                             double4 ext = make_double4(0.0, 0.0, 0.0, (double)w.soft);
                             if (a.jerk) {
-                                const size_t nn = (size_t)a.nnodes;
-                                ext.x = a.nvel[node];
-                                ext.y = a.nvel[nn + node];
-                                ext.z = a.nvel[2 * nn + node];
+                                auto& c = group_args<FP64>(a);
+                                const size_t nn = (size_t)c.nnodes;
+                                ext.x = c.nvel[node];
+                                ext.y = c.nvel[nn + node];
+                                ext.z = c.nvel[2 * nn + node];
                             }
                             s_mext[slot_m] = ext;
                         }
@@ -878,11 +909,12 @@ __global__ __launch_bounds__(64, TJ ? 3 : ((FP64 && COUNT) ? 4 : 5)) void k_walk
                 if (node >= 0) w = a.wn[node];
             }
             if (overflow) {
+                auto& c = group_args<FP64>(a);
                 if (!GSTACK && lane == 0) {
-                    const int slot = atomicAdd(a.n_retry, 1);
-                    a.retry_list[slot] = g;
+                    const int slot = atomicAdd(c.n_retry, 1);
+                    c.retry_list[slot] = g;
                 }
-                if (GSTACK && lane == 0) atomicOr(a.status, 1);
+                if (GSTACK && lane == 0) atomicOr(c.status, 1);
                 g_visit = g_multi = g_pair = 0; // the retry counts this group
                 __syncthreads();
                 break; // the whole group is redone by the global-stack launch
@@ -913,19 +945,20 @@ __global__ __launch_bounds__(64, TJ ? 3 : ((FP64 && COUNT) ? 4 : 5)) void k_walk
                     }
                 }
             }
+            auto& o = group_args<FP64>(a);
             if (TJ && tvalid && sub == 0) {
-                const size_t ntt = (size_t)a.nt, slot = (size_t)(tlo + t);
+                const size_t ntt = (size_t)o.nt, slot = (size_t)(tlo + t);
 #pragma unroll
-                for (int c = 0; c < 6; ++c) a.tidal[c * ntt + slot] = tt[c];
-                if (a.jerk) {
+                for (int c = 0; c < 6; ++c) o.tidal[c * ntt + slot] = tt[c];
+                if (o.jerk) {
 #pragma unroll
-                    for (int c = 0; c < 3; ++c) a.jerk[c * ntt + slot] = a.G * jj[c];
+                    for (int c = 0; c < 3; ++c) o.jerk[c * ntt + slot] = o.G * jj[c];
                 }
             }
             if (tvalid && sub == 0) {
-                a.ax[tlo + t] = a.G * accx;
-                a.ay[tlo + t] = a.G * accy;
-                a.az[tlo + t] = a.G * accz;
+                o.ax[tlo + t] = o.G * accx;
+                o.ay[tlo + t] = o.G * accy;
+                o.az[tlo + t] = o.G * accz;
             }
         }
         if (COUNT) {
