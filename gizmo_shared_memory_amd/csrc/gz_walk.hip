@@ -460,7 +460,8 @@ __global__ __launch_bounds__(64, TJ ? 3 : ((FP64 && COUNT) ? 4 : 5)) void k_walk
                 te = (real)pe;
             }
             double accx = 0, accy = 0, accz = 0;
-            double tt[6] = {0}, jj[3] = {0}; // tidal (xx yy zz xy yz xz), jerk (TJ only)
+            // TJ: the tidal tensor's d d part (xx yy zz xy yz xz) and delta part, the jerk
+            double tt[6] = {0}, trace = 0, jj[3] = {0};
             double tvx = 0, tvy = 0, tvz = 0;
             if (TJ && tvalid && a.jerk) {
                 auto& c = group_args<FP64>(a);
@@ -493,23 +494,30 @@ __global__ __launch_bounds__(64, TJ ? 3 : ((FP64 && COUNT) ? 4 : 5)) void k_walk
                     // tree.cc:811-871: g1 and g2 are the first and second kernel-derivative
                     // factors; the tidal tensor is -g1 delta + g2 d d (no G), the jerk
                     // g1 dv - (dv . d) g2 d
+                    // (multiply-adds are fused, as the sums of the FP64 walk below are, and the
+                    // delta term is summed once and taken off the diagonal at the end: 26
+                    // operations for the sums of a pair instead of 50)
                     auto tj = [&](double dx, double dy, double dz, double g1, double g2,
                                   const double4& v) {
-                        accx += dx * g1;
-                        accy += dy * g1;
-                        accz += dz * g1;
-                        tt[0] += -g1 + dx * dx * g2;
-                        tt[1] += -g1 + dy * dy * g2;
-                        tt[2] += -g1 + dz * dz * g2;
-                        tt[3] += dx * dy * g2;
-                        tt[4] += dy * dz * g2;
-                        tt[5] += dx * dz * g2;
+                        accx = __builtin_fma(dx, g1, accx);
+                        accy = __builtin_fma(dy, g1, accy);
+                        accz = __builtin_fma(dz, g1, accz);
+                        trace += g1;
+                        const double gx = dx * g2, gy = dy * g2, gz = dz * g2;
+                        tt[0] = __builtin_fma(dx, gx, tt[0]);
+                        tt[1] = __builtin_fma(dy, gy, tt[1]);
+                        tt[2] = __builtin_fma(dz, gz, tt[2]);
+                        tt[3] = __builtin_fma(dx, gy, tt[3]);
+                        tt[4] = __builtin_fma(dy, gz, tt[4]);
+                        tt[5] = __builtin_fma(dx, gz, tt[5]);
                         if (a.jerk) {
                             const double dvx = v.x - tvx, dvy = v.y - tvy, dvz = v.z - tvz;
-                            const double vdotr = dvx * dx + dvy * dy + dvz * dz;
-                            jj[0] += g1 * dvx - vdotr * g2 * dx;
-                            jj[1] += g1 * dvy - vdotr * g2 * dy;
-                            jj[2] += g1 * dvz - vdotr * g2 * dz;
+                            // -(dv . d) g2
+                            const double w = -__builtin_fma(
+                                dvx, gx, __builtin_fma(dvy, gy, dvz * gz));
+                            jj[0] = __builtin_fma(w, dx, __builtin_fma(g1, dvx, jj[0]));
+                            jj[1] = __builtin_fma(w, dy, __builtin_fma(g1, dvy, jj[1]));
+                            jj[2] = __builtin_fma(w, dz, __builtin_fma(g1, dvz, jj[2]));
                         }
                     };
                     // an accepted node lies outside both softenings (u >= 1), where the two
@@ -933,6 +941,8 @@ __global__ __launch_bounds__(64, TJ ? 3 : ((FP64 && COUNT) ? 4 : 5)) void k_walk
                     accz += uz;
                 }
                 if (TJ) {
+                    const double u0 = __shfl(trace, src);
+                    if (take) trace += u0;
 #pragma unroll
                     for (int c = 0; c < 6; ++c) {
                         const double u = __shfl(tt[c], src);
@@ -949,7 +959,8 @@ __global__ __launch_bounds__(64, TJ ? 3 : ((FP64 && COUNT) ? 4 : 5)) void k_walk
             if (TJ && tvalid && sub == 0) {
                 const size_t ntt = (size_t)o.nt, slot = (size_t)(tlo + t);
 #pragma unroll
-                for (int c = 0; c < 6; ++c) o.tidal[c * ntt + slot] = tt[c];
+                for (int c = 0; c < 6; ++c)
+                    o.tidal[c * ntt + slot] = (c < 3) ? tt[c] - trace : tt[c];
                 if (o.jerk) {
 #pragma unroll
                     for (int c = 0; c < 3; ++c) o.jerk[c * ntt + slot] = o.G * jj[c];
