@@ -58,29 +58,26 @@ __global__ __launch_bounds__(256) void k_pt_keys(const uint32_t* __restrict__ ta
     if (i > 0 && slot_of(i - 1) > key) atomicOr(misc + 1, 1);
 }
 
-// A pair's term as the factors that a fused multiply-add sums: t0 f, t1 f, t2 f (POT: t0 f). When
-// `use` is false (the target itself) or the two coincide, f is 0 with finite offsets, so every
-// lane runs the same instructions; only pairs inside the kernel branch off.
+// A pair's term as the factors that a fused multiply-add sums: t0 f, t1 f, t2 f (POT: t0 f). f is 0
+// when the two coincide, as a target in the tree and its own particle do exactly (both are read
+// from the sorted copy): the reference skips those. Only pairs inside the kernel branch off.
 template <bool POT>
-__device__ __forceinline__ void pt_pair(const double4 q, double es, bool use, double px, double py,
+__device__ __forceinline__ void pt_pair(const double4 q, double es, double px, double py,
                                         double pz, double pe1, double& t0, double& t1, double& t2,
                                         double& f) {
     const double ex = q.x - px, ey = q.y - py, ez = q.z - pz;
     const double r2 = __builtin_fma(ex, ex, __builtin_fma(ey, ey, ez * ez));
-    const bool ok = use & (r2 > 0);
-    const double r2s = ok ? r2 : 1.0;
     const double h = dmax_w(pe1, es);
-    const double inv = rsqrt_d(r2s);
-    const double m = ok ? q.w : 0.0;
+    const double inv = rsqrt_d(r2); // (NaN at 0, where f is not used)
     if (POT) {
         double v = -inv;
-        if (ok & (r2s < h * h)) v = pair_potential_inside(r2s, inv, h);
-        t0 = m;
-        f = v;
+        if (r2 < h * h) v = pair_potential_inside(r2, inv, h);
+        t0 = q.w;
+        f = (r2 > 0) ? v : 0.0;
     } else {
-        f = inv * inv * inv;
-        if (ok & (r2s < h * h)) f = pair_force_over_r_inside(r2s, inv, h);
-        f *= m;
+        double v = inv * inv * inv;
+        if (r2 < h * h) v = pair_force_over_r_inside(r2, inv, h);
+        f = (r2 > 0) ? v * q.w : 0.0;
         t0 = ex;
         t1 = ey;
         t2 = ez;
@@ -140,9 +137,9 @@ __global__ __launch_bounds__(64) void k_walk_pt(PtArgs a) {
     double sx = 0, sy = 0, sz = 0;
 
     // one pair term for this lane's target
-    auto pair = [&](const double4 q, double es, bool use) {
+    auto pair = [&](const double4 q, double es) {
         double t0, t1 = 0, t2 = 0, f;
-        pt_pair<POT>(q, es, use, px, py, pz, pe1, t0, t1, t2, f);
+        pt_pair<POT>(q, es, px, py, pz, pe1, t0, t1, t2, f);
         sx = __builtin_fma(t0, f, sx);
         if (!POT) {
             sy = __builtin_fma(t1, f, sy);
@@ -185,13 +182,15 @@ __global__ __launch_bounds__(64) void k_walk_pt(PtArgs a) {
                 const double4* qp = a.src + w.plo;
                 const double* ep = a.src_soft + w.plo;
                 int s = w.plo;
-                for (; s + 1 < phi; s += 2, qp += 2, ep += 2) {
-                    const double4 q0 = qp[0], q1 = qp[1];
-                    const double e0 = ep[0], e1 = ep[1];
-                    pair(q0, e0, act & (s != my));
-                    pair(q1, e1, act & (s + 1 != my));
+                if (act) { // (the lanes that wait on the leaf, once for all its particles)
+                    for (; s + 1 < phi; s += 2, qp += 2, ep += 2) {
+                        const double4 q0 = qp[0], q1 = qp[1];
+                        const double e0 = ep[0], e1 = ep[1];
+                        pair(q0, e0);
+                        pair(q1, e1);
+                    }
+                    if (s < phi) pair(qp[0], ep[0]);
                 }
-                if (s < phi) pair(qp[0], ep[0], act & (s != my));
             } else {
                 // tree.cc:552-557 (accel) and :915-920 (potential): the offset to the node's
                 // centre of mass, its squared norm, and open_node with the target's own bounds
@@ -355,7 +354,7 @@ __global__ __launch_bounds__(64) void k_walk_pt1(PtArgs a) {
                     const int s = nd->plo + (g - s_pre[lo]);
                     const double4 q = a.src[s];
                     const double es = a.src_soft[s];
-                    pt_pair<POT>(q, es, s != my, px, py, pz, pe1, t0, t1, t2, f);
+                    pt_pair<POT>(q, es, px, py, pz, pe1, t0, t1, t2, f);
                 } else {
                     pt_node<POT>(nd->cx - px, nd->cy - py, nd->cz - pz, nd->mass, true, t0, t1,
                                  t2, f);
