@@ -226,6 +226,10 @@ gz_status walk(gz_ctx* ctx, const gz_tree* tree, const gz_particles* p, const ui
     a.theta_sq = theta * theta;
     a.ngroups = (int)ngroups;
     a.ngroups_dev = packed_dev;
+    // groups packed to group_size targets hold three quarters of that on average
+    a.groups_expected =
+        packed_dev ? (int)std::min<size_t>(ngroups, n_t * 4 / (3 * (size_t)group_size) + 1)
+                   : (int)ngroups;
     a.root = tree->root;
     a.cluster_start = tree->cluster_start_dev;
     a.nclusters = tree->n_clusters;
@@ -1121,6 +1125,7 @@ gz_status gz_walk_plan_launch(gz_ctx* ctx, gz_walk_plan* P, double theta, double
     a.group_scale = nullptr;
     a.theta_sq = theta * theta;
     a.ngroups = P->ngroups;
+    a.groups_expected = P->ngroups;
     a.root = tree->root;
     a.cluster_start = tree->cluster_start_dev;
     a.nclusters = tree->n_clusters;

@@ -77,6 +77,7 @@ struct WalkArgs {
     // the group count on the device, set when the host has only an upper bound (ngroups) for it:
     // the walk then reads the count itself instead of waiting for it to be read back
     const uint32_t* ngroups_dev;
+    int groups_expected;    // their likely count, by which the launch is shaped
     int root;
     const uint32_t* cluster_start; // forest: particle offsets of the clusters; NULL: one tree
     int nclusters;

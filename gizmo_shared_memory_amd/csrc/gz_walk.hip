@@ -314,16 +314,24 @@ __device__ __forceinline__ float spline_inside_f(float r2, float inv, float g3, 
 // leave room for three.
 // TJ (FP64 only): the tidal tensor and, when velocities are given, the jerk, accumulated in the
 // same walk (tree.cc:811-871).
-template <bool FP64, bool COUNT, bool GSTACK, bool TJ = false>
-__global__ __launch_bounds__(64, TJ ? 3 : ((FP64 && COUNT) ? 4 : 5)) void k_walk(WalkArgs a) {
+// W (FP32 only): wavefronts per group, for launches of too few groups to fill the GPU, whose time is
+// that of the slowest group (30,000 particles: one outer group of 64 targets meets every particle
+// of the tree). Each of the W waves walks the whole group, with lists of its own, but evaluates
+// only every W-th list, the others meanwhile walking on; the lists' sums meet in LDS and the first
+// wave adds them in list order, so a target's result is the bits of a single wave's. A barrier of
+// the workgroup every W lists is all the waves wait for.
+template <bool FP64, bool COUNT, bool GSTACK, bool TJ = false, int W = 1>
+__global__ __launch_bounds__(64 * W, TJ ? 3 : ((FP64 && COUNT) ? 4 : 5))
+void k_walk(WalkArgs a) {
     static_assert(!TJ || FP64, "the tidal tensor and jerk are FP64 walks");
+    static_assert(W == 1 || (!FP64 && !COUNT && !GSTACK), "several waves: the plain FP32 walk");
     using real = typename WalkTypes<FP64>::real;
     using real4 = typename WalkTypes<FP64>::real4;
     constexpr int kMono = FP64 ? kMonoD : kMonoF;
     constexpr int kPair = FP64 ? kPairD : kPairF;
     // The node stack lives in LDS; a group whose stack would outgrow it is handed to a second
     // launch of this kernel (GSTACK) that keeps the stack in a per-wave slice of global memory.
-    __shared__ int s_stack[GSTACK ? 1 : kWalkStack];
+    __shared__ int s_stack_w[W][GSTACK ? 1 : kWalkStack];
     // Interaction lists. An accepted node always lies outside every target's softening (the
     // first arm of open_node), so monopoles are Newtonian and need no softening (the FP32 walk
     // also lists there the particles of opened leaves that lie outside every target's kernel);
@@ -331,14 +339,35 @@ __global__ __launch_bounds__(64, TJ ? 3 : ((FP64 && COUNT) ? 4 : 5)) void k_walk
     // The FP32 lists end in up to kPadF zero-mass entries far away, so that every lane steps
     // through whole slice steps with no per-lane bounds test (the loop stays wave-uniform).
     constexpr int kPad = FP64 ? 0 : kPadF;
-    __shared__ real4 s_mono[kMono + kPad];
-    __shared__ real4 s_pair[kPair + kPad];
-    __shared__ real s_psoft[kPair + kPad];
+    __shared__ real4 s_mono_w[W][kMono + kPad];
+    __shared__ real4 s_pair_w[W][kPair + kPad];
+    __shared__ real s_psoft_w[W][kPair + kPad];
     // TJ: node velocity and softening per monopole, source velocity per particle entry
     __shared__ double4 s_mext[TJ ? kMono : 1];
     __shared__ double4 s_pext[TJ ? kPair : 1];
-    __shared__ int s_lpre[65];
-    __shared__ int s_lplo[64];
+    __shared__ int s_lpre_w[W][65];
+    __shared__ int s_lplo_w[W][64];
+    // W > 1: the sums of the last W lists, twice over (one set is added while the next is written),
+    // and the group that the workgroup holds
+    __shared__ float s_part[2][W > 1 ? W : 1][3][W > 1 ? 64 : 1];
+    __shared__ int s_group;
+    const int wave = (W > 1) ? __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6) : 0;
+    int* const s_stack = s_stack_w[wave];
+    real4* const s_mono = s_mono_w[wave];
+    real4* const s_pair = s_pair_w[wave];
+    real* const s_psoft = s_psoft_w[wave];
+    int* const s_lpre = s_lpre_w[wave];
+    int* const s_lplo = s_lplo_w[wave];
+    // Between a wave's own writes and reads of its LDS (a workgroup of one wave: the barrier is
+    // only that).
+    auto wave_sync = [&]() {
+        if (W == 1) {
+            __syncthreads();
+        } else {
+            __threadfence_block();
+            __builtin_amdgcn_wave_barrier();
+        }
+    };
     int* const stk = GSTACK ? a.gstack + (size_t)blockIdx.x * (size_t)a.gstack_cap : s_stack;
     const int scap = GSTACK ? a.gstack_cap
                             : (a.stack_limit > 0 ? min(a.stack_limit, kWalkStack) : kWalkStack);
@@ -346,12 +375,12 @@ __global__ __launch_bounds__(64, TJ ? 3 : ((FP64 && COUNT) ? 4 : 5)) void k_walk
     // would overflow LDS, the bottom of the LDS stack moves to the slice, and it comes back when
     // LDS runs empty. The logical stack, and so the traversal order, is that of an unbounded stack.
     int* const spill = (!GSTACK && a.persistent && a.spill)
-                           ? a.spill + (size_t)blockIdx.x * (size_t)a.spill_cap
+                           ? a.spill + ((size_t)blockIdx.x * W + wave) * (size_t)a.spill_cap
                            : nullptr;
 
     // the group count: read from the device when the host holds only an upper bound
     const int ngroups = a.ngroups_dev ? (int)*a.ngroups_dev : a.ngroups;
-    const int lane = threadIdx.x;
+    const int lane = (W > 1) ? (int)threadIdx.x & 63 : (int)threadIdx.x;
     long long n_visit = 0, n_multi = 0, n_pair = 0;
     int max_sp = 0;
 
@@ -374,7 +403,7 @@ __global__ __launch_bounds__(64, TJ ? 3 : ((FP64 && COUNT) ? 4 : 5)) void k_walk
             // cost the learned FP32 walk of 8M 0.5 of its 6.5 ms. Claiming runs of 2 to 16
             // groups at a time was slower than single ones: the waves end less evenly.)
             int v = -1;
-            if (lane == 0) {
+            if (lane == 0 && wave == 0) {
                 int* const queue = group_args<FP64>(a).queue;
                 const int x0 = blockIdx.x & 7;
                 constexpr int C = kXcdChunk;
@@ -391,7 +420,14 @@ __global__ __launch_bounds__(64, TJ ? 3 : ((FP64 && COUNT) ? 4 : 5)) void k_walk
                     }
                 }
             }
-            g = __shfl(v, 0);
+            if (W > 1) {
+                __syncthreads(); // the group before is done with s_group and s_part
+                if (threadIdx.x == 0) s_group = v;
+                __syncthreads();
+                g = __builtin_amdgcn_readfirstlane(s_group);
+            } else {
+                g = __shfl(v, 0);
+            }
             if (g < 0) break;
         } else {
             // Block b runs on XCD b % 8; give each XCD one contiguous share of the Morton-ordered
@@ -469,6 +505,15 @@ __global__ __launch_bounds__(64, TJ ? 3 : ((FP64 && COUNT) ? 4 : 5)) void k_walk
                 tvx = c.pvx[p]; tvy = c.pvy[p]; tvz = c.pvz[p];
             }
             int mcount = 0, pcount = 0;
+            int lists = 0; // W > 1: lists evaluated by all waves so far
+            // W > 1: the sums of lists [from, to), in order (the first wave's accumulators)
+            auto add_lists = [&](int from, int to) {
+                for (int n = from; n < to && wave == 0; ++n) {
+                    accx += (double)s_part[(n / W) & 1][n % W][0][lane];
+                    accy += (double)s_part[(n / W) & 1][n % W][1][lane];
+                    accz += (double)s_part[(n / W) & 1][n % W][2][lane];
+                }
+            };
             bool overflow = false;
             // FP32: when no particle below the group's root is softer than the chunk's least
             // softened target, every pair's kernel extent max(h_t, h_s) is the target's own, so
@@ -483,13 +528,22 @@ __global__ __launch_bounds__(64, TJ ? 3 : ((FP64 && COUNT) ? 4 : 5)) void k_walk
 
             // Evaluate both lists against every target of the chunk.
             auto flush = [&]() {
+                if (W > 1 && lists % W != wave) { // another wave's list
+                    mcount = 0;
+                    pcount = 0;
+                    if (++lists % W == 0) {
+                        __syncthreads();
+                        add_lists(lists - W, lists);
+                    }
+                    return;
+                }
                 if (!FP64 && lane < 2 * L) {
                     const real4 far = {(real)1e18, (real)1e18, (real)1e18, (real)0};
                     s_mono[mcount + lane] = far;
                     s_pair[pcount + lane] = far;
                     s_psoft[pcount + lane] = (real)0;
                 }
-                __syncthreads();
+                wave_sync();
                 if (TJ) {
                     // tree.cc:811-871: g1 and g2 are the first and second kernel-derivative
                     // factors; the tidal tensor is -g1 delta + g2 d d (no G), the jerk
@@ -689,13 +743,24 @@ __global__ __launch_bounds__(64, TJ ? 3 : ((FP64 && COUNT) ? 4 : 5)) void k_walk
                             pair(s_pair[j1 + js], s_psoft[j1 + js], j1 + js);
                         }
                     }
-                    accx += (double)fx;
-                    accy += (double)fy;
-                    accz += (double)fz;
+                    if (W > 1) {
+                        float* const part = s_part[(lists / W) & 1][wave][0];
+                        part[lane] = fx;
+                        part[64 + lane] = fy;
+                        part[128 + lane] = fz;
+                    } else {
+                        accx += (double)fx;
+                        accy += (double)fy;
+                        accz += (double)fz;
+                    }
                 }
-                __syncthreads();
+                wave_sync();
                 mcount = 0;
                 pcount = 0;
+                if (W > 1 && ++lists % W == 0) {
+                    __syncthreads();
+                    add_lists(lists - W, lists);
+                }
             };
 
             // Node batches: the next batch is popped from the stack while this batch's lists
@@ -760,7 +825,7 @@ __global__ __launch_bounds__(64, TJ ? 3 : ((FP64 && COUNT) ? 4 : 5)) void k_walk
                         const int i = lane + 64 * r;
                         hold[r] = (i < keep) ? stk[ms + i] : 0;
                     }
-                    __syncthreads();
+                    wave_sync();
 #pragma unroll
                     for (int r = 0; r < kSpillKeep / 64; ++r) {
                         const int i = lane + 64 * r;
@@ -773,7 +838,7 @@ __global__ __launch_bounds__(64, TJ ? 3 : ((FP64 && COUNT) ? 4 : 5)) void k_walk
                 sp += ctot;
                 if (COUNT) max_sp = max(max_sp, gsp + sp);
                 if (GSTACK) __threadfence_block();
-                __syncthreads();
+                wave_sync();
                 if (sp < 64 && gsp > 0) {
                     // fewer than a batch left in LDS: slide them up and bring back the top of
                     // the spilled part beneath them, so the batch popped next is the same top
@@ -781,12 +846,12 @@ __global__ __launch_bounds__(64, TJ ? 3 : ((FP64 && COUNT) ? 4 : 5)) void k_walk
                     const int r = min(gsp, min(scap / 2, scap - sp));
                     const int held = (lane < sp) ? stk[lane] : 0;
                     __threadfence_block();
-                    __syncthreads();
+                    wave_sync();
                     if (lane < sp) stk[r + lane] = held;
                     for (int i = lane; i < r; i += 64) stk[i] = spill[gsp - r + i];
                     gsp -= r;
                     sp += r;
-                    __syncthreads();
+                    wave_sync();
                 }
                 k = min(sp, 64);
                 const int base = sp - k;
@@ -829,7 +894,7 @@ __global__ __launch_bounds__(64, TJ ? 3 : ((FP64 && COUNT) ? 4 : 5)) void k_walk
                         s_lplo[li] = plo;
                     }
                     if (lane == 0) s_lpre[nleaf] = ptot;
-                    __syncthreads();
+                    wave_sync();
                     if (!FP64) {
                         // one entry per lane: near particles to the particle list, far ones to
                         // the monopole list (both counted as pair interactions)
@@ -909,7 +974,7 @@ __global__ __launch_bounds__(64, TJ ? 3 : ((FP64 && COUNT) ? 4 : 5)) void k_walk
                         }
                     }
                 }
-                __syncthreads();
+                wave_sync();
                 // the next batch's nodes are loaded here, after this batch's lists are built:
                 // loading them earlier keeps 16 more registers live through the list building
                 // and the flushes (measured 2% slower), and other waves hide the latency
@@ -918,7 +983,7 @@ __global__ __launch_bounds__(64, TJ ? 3 : ((FP64 && COUNT) ? 4 : 5)) void k_walk
             }
             if (overflow) {
                 auto& c = group_args<FP64>(a);
-                if (!GSTACK && lane == 0) {
+                if (!GSTACK && lane == 0 && wave == 0) {
                     const int slot = atomicAdd(c.n_retry, 1);
                     c.retry_list[slot] = g;
                 }
@@ -928,6 +993,12 @@ __global__ __launch_bounds__(64, TJ ? 3 : ((FP64 && COUNT) ? 4 : 5)) void k_walk
                 break; // the whole group is redone by the global-stack launch
             }
             if (mcount > 0 || pcount > 0) flush();
+            if (W > 1) {
+                __syncthreads();
+                add_lists(lists / W * W, lists);
+                __syncthreads(); // the next chunk's lists come after these sums are read
+                if (wave != 0) continue;
+            }
 
             // combine the slices of each target pairwise (log2 L steps), then write (tree.cc:880)
             for (int step = 1; step < L; step <<= 1) {
@@ -1196,9 +1267,27 @@ gz_status launch_walk(const WalkArgs& a, bool fp64, bool count, hipStream_t st) 
     } else if (fp64) {
         if (count) k_walk<true, true, false><<<grid, 64, 0, st>>>(a);
         else k_walk<true, false, false><<<grid, 64, 0, st>>>(a);
-    } else {
-        if (count) k_walk<false, true, false><<<grid, 64, 0, st>>>(a);
+    } else if (count) {
+        k_walk<false, true, false><<<grid, 64, 0, st>>>(a);
+    } else if (a.persistent && a.waves_per_cu == 0) {
+        // Waves per group: the fewer groups there are for the GPU's 5,120 waves, the more. All
+        // targets of n particles, ms a force call (tree build included) with 1 | 2 | 4 | 8 waves:
+        // 4,000 .86 | .77 | .72 | .69; 30,000 2.42 | 1.94 | 1.60 | 1.42 (650 groups); 65,536 2.98 |
+        // 2.37 | 1.98 | 1.83; 131,072 1.06 | .98 | 1.00 | 1.13; 262,147 1.20 | 1.20 | 1.29 | 1.54;
+        // 1M (walk only) .84 | .99 | 1.40 | 2.26. Of 1M particles 64 targets .50 | .45 | .41 |
+        // .40; 4,099 .65 | .54 | .47 | .46; 30,000 .70 | .59 | .59 | .70; 200,000 .83 | .84 | .99 |
+        // 1.35. Eight up to a tenth of the waves, four up to 0.4, two up to their number.
+        int waves = 0;
+        GZ_TRY(persistent_waves(&waves));
+        const long long n = a.groups_expected;
+        const int w = (10 * n <= waves) ? 8 : (5 * n <= 2 * waves) ? 4 : (n <= waves) ? 2 : 1;
+        grid = (unsigned)std::min<long long>(std::max(waves / w, 1), a.ngroups);
+        if (w == 8) k_walk<false, false, false, false, 8><<<grid, 512, 0, st>>>(a);
+        else if (w == 4) k_walk<false, false, false, false, 4><<<grid, 256, 0, st>>>(a);
+        else if (w == 2) k_walk<false, false, false, false, 2><<<grid, 128, 0, st>>>(a);
         else k_walk<false, false, false><<<grid, 64, 0, st>>>(a);
+    } else {
+        k_walk<false, false, false><<<grid, 64, 0, st>>>(a);
     }
     GZ_HIP(hipGetLastError());
     return GZ_OK;
