@@ -606,94 +606,16 @@ __global__ __launch_bounds__(64, 3) void k_density_near(DensArgs a) {
             hc = (fresh && st.h > 0) ? st.h * kNearMargin : st.h;
             const double c2 = hc * hc;
             nc = 0;
-            int r_next = (a.nodes.nclusters > 1) ? 0 : a.nodes.root;
-            const int r_end = (a.nodes.nclusters > 1) ? a.nodes.nclusters : a.nodes.root + 1;
-            int sp = 0;
-            while (nc <= kNearMax) {
-                __syncthreads();
-                if (sp == 0) {
-                    if (r_next == r_end) break;
-                    sp = min(64, r_end - r_next);
-                    if (lane < sp) s.w.stk[sp - 1 - lane] = r_next + lane;
-                    r_next += sp;
-                    __syncthreads();
-                }
-                // (the stack, its window and its bound are k_density_round's)
-                const int w = min(sp, max(1, min(64, (kSphStack - kSphSpare - sp) / 7)));
-                int ent = 0;
-                if (lane < w) ent = s.w.stk[sp - 1 - lane];
-                const uint64_t leaf_m = __ballot(lane < w && ent < 0);
-                const int run = (~leaf_m == 0) ? 64 : (int)__builtin_ctzll(~leaf_m);
-                if (run < kSphRun && run < w) {
-                    int n = 0, link = 0;
-                    if (lane < w && ent < 0) {
-                        n = 1;
-                    } else if (lane < w) {
-                        const SRec r = a.nodes.srec[ent];
-                        double dist = hc + (double)r.half + (double)r.xpad;
-                        if (a.nodes.tau > 0) dist += (double)r.vmax * a.nodes.tau;
-                        const double dx = (double)r.cx - qx, dy = (double)r.cy - qy,
-                                     dz = (double)r.cz - qz;
-                        const double ds = dist + 0.7320508075688772 * (double)r.half;
-                        if (!(dx > dist || -dx > dist) && !(dy > dist || -dy > dist) &&
-                            !(dz > dist || -dz > dist) &&
-                            !(dx * dx + dy * dy + dz * dz > ds * ds)) {
-                            link = r.link;
-                            n = (link < 0) ? 1 : r.span;
-                            if (link < 0) ent = ~ent;
-                        }
-                    }
-                    int total;
-                    const int off = wave_excl_scan(n, total);
-                    const int top = sp - w + total - 1;
-                    __syncthreads();
-                    if (n > 0 && ent < 0) {
-                        s.w.stk[top - off] = ent;
-                    } else {
-                        for (int j = 0; j < n; ++j) s.w.stk[top - off - j] = link + j;
-                    }
-                    sp = top + 1;
-                    continue;
-                }
-                sp -= run;
-                int plo = 0, cnt = 0;
-                if (lane < run) {
-                    const SRec r = a.nodes.srec[~ent];
-                    plo = ~r.link;
-                    cnt = r.span - plo;
-                }
-                const uint64_t some = __ballot(cnt > 0);
-                int total;
-                const int off = wave_excl_scan(cnt, total);
-                if (cnt > 0) {
-                    const int li = lanes_under(some);
-                    s.w.lpre[li] = off;
-                    s.w.lplo[li] = plo;
-                }
-                __syncthreads();
-                const int nleaf = __builtin_popcountll(some);
-                for (int g0 = 0; g0 < total; g0 += 64) {
-                    const int g = g0 + lane;
-                    bool in = false;
-                    int slot = 0;
-                    if (g < total) {
-                        int lo_ = 0, hi_ = nleaf; // the last leaf li with lpre[li] <= g
-                        while (hi_ - lo_ > 1) {
-                            const int mid = (lo_ + hi_) >> 1;
-                            if (s.w.lpre[mid] <= g) lo_ = mid;
-                            else hi_ = mid;
-                        }
-                        slot = s.w.lplo[lo_] + (g - s.w.lpre[lo_]);
-                        const double4 q = a.src[slot];
-                        const double ex = q.x - qx, ey = q.y - qy, ez = q.z - qz;
-                        in = ex * ex + ey * ey + ez * ez < c2;
-                    }
-                    const uint64_t im = __ballot(in);
-                    const int pos = nc + lanes_under(im);
-                    if (in && pos < kNearMax) s_cand[pos] = (uint32_t)slot;
-                    nc += __builtin_popcountll(im);
-                }
-            }
+            walk_sphere<true>(a.nodes, qx, qy, qz, hc, s.w.stk, s.w.lpre, s.w.lplo,
+                              [&](bool some, int slot, const double4& q) {
+                const double ex = q.x - qx, ey = q.y - qy, ez = q.z - qz;
+                const bool in = some && ex * ex + ey * ey + ez * ez < c2;
+                const uint64_t im = __ballot(in);
+                const int pos = nc + lanes_under(im);
+                if (in && pos < kNearMax) s_cand[pos] = (uint32_t)slot;
+                nc += __builtin_popcountll(im);
+                return nc <= kNearMax;
+            });
             if (nc > kNearMax) {
                 if (lane == 0) {
                     a.h[t] = st.h;

@@ -355,24 +355,29 @@ __global__ void k_u32_to_size(int n, const uint32_t* __restrict__ in, size_t* __
 
 // The sum of the per-query counts in 64 bits (the 32-bit scan that makes the offsets would wrap
 // past 2^32 - 1 pairs): a grid-stride sum per thread, one atomic per workgroup.
-// The largest count too, which picks how the lists are sorted.
+// The largest count too, which picks how the lists are sorted, and behind it how many exceed
+// `limit`.
 __global__ __launch_bounds__(256) void k_sum_counts(int n, const uint32_t* __restrict__ in,
                                                     unsigned long long* __restrict__ out,
-                                                    uint32_t* __restrict__ max_out) {
+                                                    uint32_t* __restrict__ max_out,
+                                                    uint32_t limit) {
     __shared__ unsigned long long ss[4];
-    __shared__ uint32_t sm[4];
+    __shared__ uint32_t sm[4], sl[4];
     unsigned long long s = 0;
-    uint32_t mx = 0;
+    uint32_t mx = 0, over = 0;
     for (int i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256) {
         s += in[i];
         mx = max(mx, in[i]);
+        over += in[i] > limit ? 1 : 0;
     }
     for (int d = 32; d >= 1; d >>= 1) {
         s += (unsigned long long)__shfl_xor((long long)s, d);
         mx = max(mx, (uint32_t)__shfl_xor((int)mx, d));
+        over += (uint32_t)__shfl_xor((int)over, d);
     }
     if ((threadIdx.x & 63) == 0) {
         ss[threadIdx.x >> 6] = s;
+        sl[threadIdx.x >> 6] = over;
         sm[threadIdx.x >> 6] = mx;
     }
     __syncthreads();
@@ -380,8 +385,10 @@ __global__ __launch_bounds__(256) void k_sum_counts(int n, const uint32_t* __res
     for (int k = 1; k < 4; ++k) {
         s += ss[k];
         mx = max(mx, sm[k]);
+        over += sl[k];
     }
     if (s) atomicAdd(out, s);
+    if (over) atomicAdd(max_out + 1, over);
     if (mx) atomicMax(max_out, mx);
 }
 
@@ -395,8 +402,13 @@ __device__ __forceinline__ float h_as_bound(double h) {
 // A lane per query, 64 consecutive queries per wave, on walk_spheres: a query meets its neighbours
 // in slot order, which is its list's order. The first launch counts them and keeps the first
 // kNgbRow in a row per query, so that a list is found, counted and ordered in one walk; only
-// queries with longer lists are walked again (FILL), straight into their place in the CSR.
+// queries with longer lists are walked again, straight into their place in the CSR: by a wave each
+// (k_ngb_long) while they are few, else as they were walked first (FILL).
 constexpr int kNgbRow = 64;
+// A wave each up to one query in this many. 1M queries, ms a search with a wave each / walked as
+// first, by the share of long lists: Hernquist .0015 1.50 / 1.77, .05 2.04 / 2.25, .11 2.50 / 2.55,
+// .20 3.10 / 2.86; halo + disk .008 1.59 / 1.96, .07 2.30 / 2.54, .13 2.83 / 2.86, .22 3.52 / 3.17.
+constexpr int kNgbFew = 8;
 constexpr size_t kNgbRowsMax = size_t(1) << 30; // bytes of rows beyond which every list is walked twice
 
 struct NgbFwd {
@@ -456,8 +468,46 @@ __global__ __launch_bounds__(64) void k_ngb_fwd(NgbFwd a) {
     if (!FILL && mine) a.count[q] = n;
 }
 
-// The rows into their places: half a wave per query, those with longer lists left to the FILL
-// launch.
+// The queries with lists longer than a row, in any order (one atomic per wave that has some).
+__global__ __launch_bounds__(256) void k_ngb_longs(int nq, const size_t* __restrict__ start,
+                                                   uint32_t* __restrict__ longs,
+                                                   uint32_t* __restrict__ n_longs) {
+    const int q = blockIdx.x * 256 + threadIdx.x;
+    const bool is = q < nq && start[q + 1] - start[q] > (size_t)kNgbRow;
+    const uint64_t m = __ballot(is);
+    if (m == 0) return;
+    int at = 0;
+    if ((threadIdx.x & 63) == 0) at = (int)atomicAdd(n_longs, (uint32_t)__builtin_popcountll(m));
+    at = __builtin_amdgcn_readfirstlane(at);
+    if (is) longs[at + lanes_under(m)] = (uint32_t)q;
+}
+
+// A wave per listed query. They lie among shorter ones: with a lane each, the waves that held one
+// or two of them tested every particle of the largest sphere in a lane, and the longest lists' waves
+// set the time.
+template <bool PACKED>
+__global__ __launch_bounds__(64) void k_ngb_long(NgbFwd a, const uint32_t* __restrict__ longs,
+                                                 int n_longs) {
+    __shared__ int stk[kSphStack], lpre[64], lplo[64];
+    for (int i = blockIdx.x; i < n_longs; i += gridDim.x) {
+        const uint32_t c = longs[i];
+        const double qx = a.cx[c], qy = a.cy[c], qz = a.cz[c], r = a.radius[c];
+        const double r2 = r * r;
+        size_t at = a.start[c];
+        walk_sphere<PACKED>(a.nodes, qx, qy, qz, r, stk, lpre, lplo,
+                            [&](bool some, int slot, const double4& p) {
+            const double ex = p.x - qx, ey = p.y - qy, ez = p.z - qz;
+            const bool in = some && ex * ex + ey * ey + ez * ez < r2;
+            const uint64_t im = __ballot(in);
+            if (in) a.found[at + lanes_under(im)] = a.orderbuf[slot];
+            at += __builtin_popcountll(im);
+            return true;
+        });
+    }
+}
+
+// The rows into their places: half a wave per query, those with longer lists left to the launches
+// above.
 __global__ __launch_bounds__(256) void k_ngb_rows(int nq, const size_t* __restrict__ start,
                                                   const uint32_t* __restrict__ rows,
                                                   uint32_t* __restrict__ found) {
@@ -672,7 +722,7 @@ static gz_status ngb_run(gz_ctx* ctx, const gz_tree* tree, const double* cx, con
     GZ_TRY(fill_zero_u32(count, n_q + 1, st));
     unsigned long long* total64 = reinterpret_cast<unsigned long long*>(misc + 4);
     uint32_t* max_count = reinterpret_cast<uint32_t*>(misc + 6);
-    GZ_TRY(fill_zero_u32(reinterpret_cast<uint32_t*>(total64), 3, st));
+    GZ_TRY(fill_zero_u32(reinterpret_cast<uint32_t*>(total64), 4, st));
     NgbFwd f{};
     const unsigned fgrid = (unsigned)a.ngroups;
     if (rev) {
@@ -695,7 +745,7 @@ static gz_status ngb_run(gz_ctx* ctx, const gz_tree* tree, const double* cx, con
         GZ_HIP(hipGetLastError());
     }
     k_sum_counts<<<(unsigned)std::min<size_t>(256, (n_q + 255) / 256), 256, 0, st>>>(
-        (int)n_q, count, total64, max_count);
+        (int)n_q, count, total64, max_count, (uint32_t)kNgbRow);
     GZ_HIP(hipGetLastError());
     // offsets: exclusive scan of the counts (count[n_q] = 0 gives the total at start[n_q])
     uint32_t tot32 = 0;
@@ -712,14 +762,15 @@ static gz_status ngb_run(gz_ctx* ctx, const gz_tree* tree, const double* cx, con
     }
     int h_status = 0;
     unsigned long long h_total = 0;
-    uint32_t h_max = 0;
-    GZ_HIP(hipMemcpyAsync(&h_max, max_count, sizeof h_max, hipMemcpyDeviceToHost, st));
+    uint32_t h_most[2] = {0, 0}; // the longest list, the lists longer than a row
+    GZ_HIP(hipMemcpyAsync(h_most, max_count, sizeof h_most, hipMemcpyDeviceToHost, st));
     GZ_HIP(hipMemcpyAsync(&h_status, a.status, sizeof h_status, hipMemcpyDeviceToHost, st));
     GZ_HIP(hipMemcpyAsync(&h_total, total64, sizeof h_total, hipMemcpyDeviceToHost, st));
     GZ_HIP(hipStreamSynchronize(st));
     if (h_status & 1)
         return fail(GZ_ERR_INTERNAL, "%s: a search stack outgrew %d entries", who,
                     stack_cap);
+    const uint32_t h_max = h_most[0], h_long = h_most[1];
     if (h_total > 0xFFFFFFFFull)
         return fail(GZ_ERR_UNSUPPORTED,
                     "%s: %llu neighbour pairs exceed the 2^32 - 1 one call can return; split the "
@@ -732,7 +783,15 @@ static gz_status ngb_run(gz_ctx* ctx, const gz_tree* tree, const double* cx, con
                 (int)n_q, start, f.rows, found);
             GZ_HIP(hipGetLastError());
         }
-        if (!rows || h_max > (uint32_t)kNgbRow) {
+        if (rows && h_long > 0 && h_long <= n_q / kNgbFew) {
+            // (the counts are in the offsets: their array takes the list)
+            k_ngb_longs<<<(unsigned)((n_q + 255) / 256), 256, 0, st>>>(
+                (int)n_q, start, count, reinterpret_cast<uint32_t*>(misc + 2));
+            const unsigned grid = (unsigned)std::min<size_t>(h_long, (size_t)waves);
+            if (packed) k_ngb_long<true><<<grid, 64, 0, st>>>(f, count, (int)h_long);
+            else k_ngb_long<false><<<grid, 64, 0, st>>>(f, count, (int)h_long);
+            GZ_HIP(hipGetLastError());
+        } else if (!rows || h_long > 0) {
             k_ngb_fwd<true><<<fgrid, 64, 0, st>>>(f);
             GZ_HIP(hipGetLastError());
         }

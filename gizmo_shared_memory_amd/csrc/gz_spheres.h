@@ -227,6 +227,99 @@ __device__ __forceinline__ void walk_spheres(const SphereNodes& a, bool mine, do
     }
 }
 
+// Walks the tree for one sphere with the whole wave: up to 64 nodes at a time under the reference's
+// own node test, on a stack kept as walk_spheres keeps its. take(have, slot, q) is called by every
+// lane on the particles of the admitted leaves, in slot order over the calls and their lanes; the
+// walk ends when it returns false. PACKED: a.srec is there.
+template <bool PACKED, class Take>
+__device__ __forceinline__ void walk_sphere(const SphereNodes& a, double qx, double qy, double qz,
+                                            double h, int* stk, int* lpre, int* lplo,
+                                            Take&& take) {
+    const int lane = threadIdx.x & 63;
+    int r_next = (a.nclusters > 1) ? 0 : a.root;
+    const int r_end = (a.nclusters > 1) ? a.nclusters : a.root + 1;
+    int sp = 0;
+    for (;;) {
+        __syncthreads();
+        if (sp == 0) {
+            if (r_next == r_end) break;
+            sp = min(64, r_end - r_next);
+            if (lane < sp) stk[sp - 1 - lane] = r_next + lane;
+            r_next += sp;
+            __syncthreads();
+        }
+        // (the stack, its window and its bound are walk_spheres')
+        const int w = min(sp, max(1, min(64, (kSphStack - kSphSpare - sp) / 7)));
+        int ent = 0;
+        if (lane < w) ent = stk[sp - 1 - lane];
+        const uint64_t leaf_m = __ballot(lane < w && ent < 0);
+        const int run = (~leaf_m == 0) ? 64 : (int)__builtin_ctzll(~leaf_m);
+        if (run < kSphRun && run < w) {
+            int n = 0, link = 0;
+            if (lane < w && ent < 0) {
+                n = 1;
+            } else if (lane < w) {
+                const SRec r = PACKED ? a.srec[ent] : a.at(ent);
+                double dist = h + (double)r.half + (double)r.xpad;
+                if (a.tau > 0) dist += (double)r.vmax * a.tau;
+                const double dx = (double)r.cx - qx, dy = (double)r.cy - qy,
+                             dz = (double)r.cz - qz;
+                const double ds = dist + 0.7320508075688772 * (double)r.half;
+                if (!(dx > dist || -dx > dist) && !(dy > dist || -dy > dist) &&
+                    !(dz > dist || -dz > dist) && !(dx * dx + dy * dy + dz * dz > ds * ds)) {
+                    link = r.link;
+                    n = (link < 0) ? 1 : r.span;
+                    if (link < 0) ent = ~ent;
+                }
+            }
+            int total;
+            const int off = wave_excl_scan(n, total);
+            const int top = sp - w + total - 1;
+            __syncthreads();
+            if (n > 0 && ent < 0) {
+                stk[top - off] = ent;
+            } else {
+                for (int j = 0; j < n; ++j) stk[top - off - j] = link + j;
+            }
+            sp = top + 1;
+            continue;
+        }
+        sp -= run;
+        int plo = 0, cnt = 0;
+        if (lane < run) {
+            const SRec r = PACKED ? a.srec[~ent] : a.at(~ent);
+            plo = ~r.link;
+            cnt = r.span - plo;
+        }
+        const uint64_t some = __ballot(cnt > 0);
+        int total;
+        const int off = wave_excl_scan(cnt, total);
+        if (cnt > 0) {
+            const int li = lanes_under(some);
+            lpre[li] = off;
+            lplo[li] = plo;
+        }
+        __syncthreads();
+        const int nleaf = __builtin_popcountll(some);
+        for (int g0 = 0; g0 < total; g0 += 64) {
+            const int g = g0 + lane;
+            int slot = 0;
+            double4 q = make_double4(0.0, 0.0, 0.0, 0.0);
+            if (g < total) {
+                int lo_ = 0, hi_ = nleaf; // the last leaf li with lpre[li] <= g
+                while (hi_ - lo_ > 1) {
+                    const int mid = (lo_ + hi_) >> 1;
+                    if (lpre[mid] <= g) lo_ = mid;
+                    else hi_ = mid;
+                }
+                slot = lplo[lo_] + (g - lpre[lo_]);
+                q = a.src[slot];
+            }
+            if (!take(g < total, slot, q)) return;
+        }
+    }
+}
+
 // t's nodes for a walk; with srec (room for t's nodes) and moved (zero before), packed.
 gz_status launch_sphere_nodes(const gz_tree* t, double tau, SRec* srec, int* moved,
                               SphereNodes* out, hipStream_t st);

@@ -50,6 +50,38 @@ def test_lists_around_a_rows_length(gz, nq, aged):
         assert np.array_equal(mine, every[np.argsort(rank[every])]), q
 
 
+@pytest.mark.parametrize("nq,n_long", [(8, 1), (64, 8), (300, 1), (300, 37), (5000, 625),
+                                       (5000, 626)])
+@pytest.mark.parametrize("aged", [False, True])
+def test_few_long_lists(gz, nq, n_long, aged):
+    """Up to one query in eight with a list longer than a row: a wave each, as far as one whose
+    sphere holds every particle."""
+    rng = np.random.default_rng(nq + n_long)
+    pos = rng.normal(size=(3, N))
+    v = 0.1 * rng.normal(size=(3, N))
+    tau = 0.05 if aged else 0.0
+    m, soft = np.full(N, 1.0 / N), np.full(N, 0.01)
+    T = gz.build(gz.Particles(*pos, m, soft), vel=v)
+    now = pos + tau * v
+    T.update_sources(gz.Particles(*now, m, soft))
+    rank = T.download()["rank"].astype(np.int64)
+    c = now[:, rng.choice(N, nq, replace=False)].T
+    r = np.zeros(nq)
+    longs = np.sort(rng.choice(nq, n_long, replace=False))
+    want = rng.choice([65, 128, 129, 1000], n_long)
+    want[0] = N
+    for q, k in zip(longs, want):
+        d = np.sort(((c[q] - now.T) ** 2).sum(1))
+        r[q] = np.sqrt(0.5 * (d[k - 1] + (d[k] if k < N else 4 * d[k - 1])))
+    print(f"[ngb rows] nq={nq} long={n_long} aged={aged}", flush=True)
+    start, found = gz.ngb_search(T, c, r, tau)
+    start, found = start.cpu().numpy(), found.cpu().view(torch.int32).numpy()
+    assert np.array_equal(np.diff(start)[longs], want) and start[-1] == want.sum()
+    for q in longs:
+        every = np.nonzero(((c[q] - now.T) ** 2).sum(1) < r[q] * r[q])[0]
+        assert np.array_equal(found[start[q]:start[q + 1]], every[np.argsort(rank[every])]), q
+
+
 def test_buffers_that_do_not_hold_the_lists(gz):
     """The C call with no buffer, one too small, one exactly large enough and one with room for
     long lists: the same total, and the lists where they fit."""
