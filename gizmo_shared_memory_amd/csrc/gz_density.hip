@@ -570,7 +570,7 @@ __global__ __launch_bounds__(64) void k_density_far(DensArgs a) {
 // end. The wave collects its target's candidates once, out to kNearMargin times the radius, up to
 // 64 nodes in depth-first order at a time, and keeps them in registers (candidate 64 k + lane), in
 // slot order: a step is then a distance test and the terms of those inside, without the tree, until
-// the radius outgrows the collection. (Targets that run to the 100-iteration cap, whose walks one
+// the radius outgrows the collection (one of a radius above zero). (Targets that run to the 100-iteration cap, whose walks one
 // node at a time set the launch's time, took 39 us a step before, and 2-3 us now.) When some
 // particle has left its cell the candidates are collected for each step at its own radius, under
 // the reference's node tests. A sphere of more than kNearMax candidates is left to k_density_far
@@ -636,7 +636,7 @@ __global__ __launch_bounds__(64, 3) void k_density_near(DensArgs a) {
                     nb[k] = neighbour_at(a, slot);
                 }
             }
-            have = fresh;
+            have = fresh && st.h > 0; // (a negative radius's next step may be larger in size)
         }
         const double r2 = st.h * st.h;
         Kernel kern;
