@@ -72,8 +72,12 @@ __device__ __forceinline__ double ball_vol(double h, int dim) {
 // the hardware's estimate or a rounded reciprocal, refined with fused multiply-adds until the last
 // correction is a rounding of the exact remainder (P. Markstein, IBM J. Res. Dev. 34 (1990) 111).
 // Outside the ranges where every intermediate is exact the general operation is used.
-__device__ __forceinline__ double sqrt_rn(double x) {
-    if ((x > 0.0 && x < 1e-250) || !(x <= 1e250)) return sqrt(x);
+// most: a bound on the root, applied only outside the range.
+__device__ __forceinline__ double sqrt_rn(double x, double most) {
+    if ((x > 0.0 && x < 1e-250) || !(x <= 1e250)) {
+        const double r = sqrt(x);
+        return r > most ? most : r;
+    }
     const double y = __builtin_amdgcn_rsq(x);
     double g = x * y, h = 0.5 * y;
     const double e = __builtin_fma(-h, g, 0.5);
@@ -96,6 +100,12 @@ struct Kernel {
         norm2 = norm * 2.0;
         c1 = -((double)dim / h) * norm;
         general = !(h > 1e-120 && h < 1e120);
+    }
+    // The distance of a square. Where the short quotient serves, distances end at 1e187, far outside
+    // any kernel: the quotient of a larger one (a particle that has moved to infinity since the
+    // tree took its position) could be infinite, and its correction NaN.
+    __device__ __forceinline__ double distance(double x) const {
+        return sqrt_rn(x, general ? __builtin_inf() : 1e187);
     }
     // a / h (a of a size where a quotient that underflows changes no sum it enters)
     __device__ __forceinline__ double over_h(double a) const {
@@ -233,7 +243,7 @@ __device__ __forceinline__ bool density_terms(const Neighbour& nb, double p0, do
                                               const Kernel& kern, double* v, bool* inside) {
     if (!nb.gas) return false; // gas neighbours only
     const double d0 = nb.x - p0, d1 = nb.y - p1, d2 = nb.z - p2;
-    const double r = sqrt_rn(d0 * d0 + d1 * d1 + d2 * d2);
+    const double r = kern.distance(d0 * d0 + d1 * d1 + d2 * d2);
     double w;
     kern.at(r, &w, &v[1]);
     v[0] = w;

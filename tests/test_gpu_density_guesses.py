@@ -1,6 +1,6 @@
 """The density solve from first guesses and positions at the edges of what it accepts: radii that
-are negative or zero, for which the reference's node tests decide what a step finds, against the
-oracle."""
+are negative or zero, for which the reference's node tests decide what a step finds, and particles
+that have since moved beyond any radius, against the oracle."""
 import numpy as np
 import pytest
 
@@ -46,4 +46,27 @@ def test_negative_and_zero_guesses(gz, oracle, dims, scale):
     dev, ora = _both(gz, oracle, case, case, tg, h0, des_ngb={3: 32.0, 2: 20.0, 1: 6.0}[dims],
                      ngb_tol=1.0, n_dims=dims)
     assert np.count_nonzero(ora[3] == 100) > tg.shape[0] // 2  # they do not leave the sign
+    _compare(dev, ora)
+
+
+@pytest.mark.parametrize("x", [1e154, 1e200, np.inf])
+def test_live_positions_beyond_any_radius(gz, oracle, x):
+    """Particles that have moved so far since the tree's copy of the positions was taken that r / h
+    overflows add nothing (W = 0 beyond the kernel), in the wave's kernel and in the rounds. A
+    jittered lattice, whose inner particles' corrections (which their infinite moments would switch
+    off) do not apply."""
+    k = 22
+    rng = np.random.default_rng(4)
+    g = (np.stack(np.meshgrid(*[np.arange(k)] * 3, indexing="ij"), -1).reshape(-1, 3) + 0.5 +
+         rng.uniform(-0.1, 0.1, (k ** 3, 3))) / k
+    case = [np.ascontiguousarray(g[:, d]) for d in range(3)]
+    case += [np.full(k ** 3, 1.0 / k ** 3), np.full(k ** 3, 0.01)]
+    live = [a.copy() for a in case]
+    gone = rng.choice(k ** 3, 40, replace=False)
+    live[0][gone] = x
+    inner = np.flatnonzero((np.abs(g - 0.5) < 0.2).all(1))
+    tg = np.setdiff1d(inner, gone).astype(np.uint32)
+    h0 = np.full(tg.shape[0], 0.2)
+    print(f"[density guesses] live x={x}", flush=True)
+    dev, ora = _both(gz, oracle, case, live, tg, h0, des_ngb=40.0, ngb_tol=0.5)
     _compare(dev, ora)
