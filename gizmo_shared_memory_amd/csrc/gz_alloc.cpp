@@ -1,0 +1,131 @@
+// The library's error text and the device memory that it keeps between calls (gz_alloc.h).
+#include "gz_alloc.h"
+
+#include <algorithm>
+#include <cstdarg>
+#include <cstdio>
+#include <string>
+
+namespace gz {
+
+// ---- errors ----------------------------------------------------------------------------------
+static thread_local std::string g_last_error;
+
+void set_error(const char* fmt, ...) {
+    char buf[1024];
+    va_list ap;
+    va_start(ap, fmt);
+    vsnprintf(buf, sizeof buf, fmt, ap);
+    va_end(ap);
+    g_last_error = buf;
+}
+
+gz_status fail(gz_status s, const char* fmt, ...) {
+    char buf[1024];
+    va_list ap;
+    va_start(ap, fmt);
+    vsnprintf(buf, sizeof buf, fmt, ap);
+    va_end(ap);
+    g_last_error = buf;
+    return s;
+}
+
+gz_status hip_fail(hipError_t e, const char* what, const char* file, int line) {
+    set_error("%s failed: %s (%s:%d)", what, hipGetErrorString(e), file, line);
+    return (e == hipErrorOutOfMemory) ? GZ_ERR_NOMEM : GZ_ERR_HIP;
+}
+
+const char* last_error_cstr() { return g_last_error.c_str(); }
+void clear_error() { g_last_error.clear(); }
+
+// ---- device memory ---------------------------------------------------------------------------
+gz_status DevMem::reserve(size_t want) {
+    if (want <= bytes && p) return GZ_OK;
+    if (p) {
+        // work already queued may still read the old buffer
+        GZ_HIP(hipDeviceSynchronize());
+        GZ_HIP(hipFree(p));
+        p = nullptr;
+        bytes = 0;
+    }
+    const size_t b = std::max<size_t>(want, 256);
+    GZ_HIP(hipMalloc(&p, b));
+    bytes = b;
+    return GZ_OK;
+}
+
+void DevMem::release() {
+    if (p) (void)hipFree(p);
+    p = nullptr;
+    bytes = 0;
+}
+
+gz_status BlockCache::get(size_t bytes, DevBlock* out) {
+    const size_t want = (std::max<size_t>(bytes, 1) + 4095) & ~size_t(4095);
+    {
+        std::lock_guard<std::mutex> lock(mu_);
+        int best = -1;
+        for (int i = 0; i < n_; ++i)
+            if (kept_[i].bytes >= want && kept_[i].bytes - want <= want / 4 &&
+                (best < 0 || kept_[i].bytes < kept_[best].bytes))
+                best = i;
+        if (best >= 0) {
+            *out = kept_[best];
+            held_ -= out->bytes;
+            kept_[best] = kept_[--n_];
+            return GZ_OK;
+        }
+    }
+    *out = {nullptr, 0};
+    hipError_t e = hipMalloc(&out->p, want);
+    if (e == hipErrorOutOfMemory) {
+        (void)hipGetLastError();
+        drain();
+        e = hipMalloc(&out->p, want);
+    }
+    if (e != hipSuccess) {
+        out->p = nullptr;
+        return hip_fail(e, "hipMalloc", __FILE__, __LINE__);
+    }
+    out->bytes = want;
+    return GZ_OK;
+}
+
+void BlockCache::put(DevBlock b) {
+    {
+        std::lock_guard<std::mutex> lock(mu_);
+        if (open_ && n_ < kBlocks && held_ + b.bytes <= kBytes) {
+            kept_[n_++] = b;
+            held_ += b.bytes;
+            return;
+        }
+    }
+    (void)hipFree(b.p);
+}
+
+void BlockCache::retire(const DevBlock* b, int n) {
+    if (n <= 0) return;
+    const bool idle = hipDeviceSynchronize() == hipSuccess;
+    for (int i = 0; i < n; ++i) {
+        if (idle) put(b[i]);
+        else (void)hipFree(b[i].p);
+    }
+    if (!idle) (void)hipGetLastError(); // (the next launch's check is not to find it)
+}
+
+void BlockCache::drain() {
+    std::lock_guard<std::mutex> lock(mu_);
+    for (int i = 0; i < n_; ++i) (void)hipFree(kept_[i].p);
+    n_ = 0;
+    held_ = 0;
+}
+
+void BlockCache::close() {
+    {
+        std::lock_guard<std::mutex> lock(mu_);
+        open_ = false;
+    }
+    drain();
+}
+
+} // namespace gz

@@ -474,7 +474,7 @@ gz_status gz_tree_build(gz_ctx* ctx, const gz_particles* p, const gz_build_opts*
     t->blocks = ctx->blocks;
     gz_status s = gz::build_tree(ctx, p, opts, t);
     if (s != GZ_OK) {
-        (void)hipDeviceSynchronize();
+        (void)hipStreamSynchronize(ctx->stream); // (the caller's arrays are in use until then)
         gz::tree_release(t);
         delete t;
         return s;
@@ -485,9 +485,7 @@ gz_status gz_tree_build(gz_ctx* ctx, const gz_particles* p, const gz_build_opts*
 
 gz_status gz_tree_free(gz_tree* tree) {
     if (!tree) return GZ_OK;
-    // every stream, as freeing the blocks would wait for: another may still read the tree
     (void)hipSetDevice(tree->device);
-    (void)hipDeviceSynchronize();
     gz::tree_release(tree);
     delete tree;
     return GZ_OK;

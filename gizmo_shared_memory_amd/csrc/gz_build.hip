@@ -753,8 +753,8 @@ static gz_status tree_alloc(gz_tree* t, void** p, size_t bytes) {
     *p = nullptr;
     if (t->nblocks == gz_tree::kMaxBlocks)
         return fail(GZ_ERR_INTERNAL, "gz_tree_build: more device blocks than a tree has");
-    gz_tree::Block b{};
-    GZ_TRY(t->blocks->get(bytes, &b.p, &b.bytes));
+    DevBlock b{};
+    GZ_TRY(t->blocks->get(bytes, &b));
     t->block[t->nblocks++] = b;
     *p = b.p;
     return GZ_OK;
@@ -764,7 +764,7 @@ static gz_status tree_alloc(gz_tree* t, void** p, size_t bytes) {
 static void tree_drop(gz_tree* t, void* p) {
     for (int i = 0; i < t->nblocks; ++i)
         if (t->block[i].p == p) {
-            t->blocks->put(p, t->block[i].bytes);
+            t->blocks->put(t->block[i]);
             t->block[i] = t->block[--t->nblocks];
             return;
         }
@@ -823,9 +823,9 @@ static gz_status alloc_reuse(gz_tree* t, int nn, bool vel) {
     return GZ_OK;
 }
 
-// The caller has waited for the device: the blocks may be handed to the next build at once.
+// Work on any stream may still use the blocks (the cache waits for it).
 void tree_release(gz_tree* t) {
-    for (int i = 0; i < t->nblocks; ++i) t->blocks->put(t->block[i].p, t->block[i].bytes);
+    t->blocks->retire(t->block, t->nblocks);
     t->nblocks = 0;
     if (t->hmax) (void)hipFree(t->hmax);
 }

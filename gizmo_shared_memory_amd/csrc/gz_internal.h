@@ -6,11 +6,11 @@
 #include <cfloat>
 #include <cstdint>
 #include <memory>
-#include <mutex>
 #include <string>
 #include <utility>
 #include <vector>
 
+#include "gz_alloc.h"
 #include "gz_grav.h"
 
 namespace gz {
@@ -137,58 +137,6 @@ struct PtArgs {
     double *ax, *ay, *az;    // potential: ax only
 };
 
-// ---- errors ---------------------------------------------------------------------------------
-void set_error(const char* fmt, ...);
-gz_status fail(gz_status s, const char* fmt, ...);
-gz_status hip_fail(hipError_t e, const char* what, const char* file, int line);
-
-#define GZ_HIP(call)                                                          \
-    do {                                                                      \
-        hipError_t gz_e_ = (call);                                            \
-        if (gz_e_ != hipSuccess) return ::gz::hip_fail(gz_e_, #call, __FILE__, __LINE__); \
-    } while (0)
-
-#define GZ_TRY(expr)                       \
-    do {                                   \
-        gz_status gz_s_ = (expr);          \
-        if (gz_s_ != GZ_OK) return gz_s_;  \
-    } while (0)
-
-// Grow-only device allocation.
-struct DevMem {
-    void* p = nullptr;
-    size_t bytes = 0;
-    gz_status reserve(size_t want);
-    void release();
-    template <class T> T* as() const { return static_cast<T*>(p); }
-};
-
-// Device blocks that freed trees leave for the next build on their context: a tree is some 25
-// arrays, and at 4M particles freeing and allocating them took 4.6 of a rebuild's 5.3 ms. It
-// holds at most kBytes and kBlocks (beyond that blocks go back to the device), and gives
-// everything back when its context is destroyed or an allocation here finds no memory. Trees may
-// be freed by another thread than the one that builds (the list is locked), and after their
-// context (they share the cache's ownership; it then keeps nothing).
-class BlockCache {
-public:
-    static constexpr size_t kBytes = size_t(2) << 30;
-    static constexpr int kBlocks = 64;
-    // A block of at least `bytes` (*got of them): a kept one if it is not much larger.
-    gz_status get(size_t bytes, void** p, size_t* got);
-    // A block that nothing on the device uses any more.
-    void put(void* p, size_t bytes);
-    void drain();
-    void close(); // drain, and keep nothing from now on
-
-private:
-    std::mutex mu_;
-    void* ptr_[kBlocks];
-    size_t size_[kBlocks];
-    int n_ = 0;
-    size_t held_ = 0;
-    bool open_ = true;
-};
-
 // ---- device-wide primitives (gz_prims.hip) --------------------------------------------------
 // Exclusive scan of n uint32 values (in may equal out). total_dev, when non-null, receives the
 // sum (device). tmp must hold scan_tmp_bytes(n).
@@ -206,9 +154,6 @@ gz_status radix_sort_pairs(uint64_t*& keys, uint32_t*& vals, uint64_t*& keys_alt
 
 // Zero n uint32 words with a kernel (no memset node, so the call is safe under stream capture).
 gz_status fill_zero_u32(uint32_t* a, size_t n, hipStream_t st);
-
-const char* last_error_cstr();
-void clear_error();
 
 // ---- walks (gz_walk.hip) ------------------------------------------------------------------------
 gz_status launch_group_prep(const uint32_t* targets, size_t nt, const uint32_t* rank,
@@ -352,12 +297,8 @@ struct gz_tree {
     int device = 0;
     // every device block of the tree but hmax, and the context's cache they come from
     std::shared_ptr<gz::BlockCache> blocks;
-    struct Block {
-        void* p;
-        size_t bytes;
-    };
     static constexpr int kMaxBlocks = 32;
-    Block block[kMaxBlocks];
+    gz::DevBlock block[kMaxBlocks];
     int nblocks = 0;
     size_t n = 0, n_live = 0;
     int nnodes = 0, nleaves = 0, depth = 0, arena_grows = 0, root = 0;

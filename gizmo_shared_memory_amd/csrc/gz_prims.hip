@@ -2,127 +2,11 @@
 // (64-bit key, 32-bit value) pairs. Both are memory-bound at the sizes of large trees (>= 1M
 // keys), where one launch has a thousand workgroups, and bound by their launches below that.
 #include <algorithm>
-#include <cstdarg>
-#include <cstdio>
-#include <cstring>
 
 #include "gz_internal.h"
 #include "gz_wave.h"
 
 namespace gz {
-
-// ---- errors ----------------------------------------------------------------------------------
-static thread_local std::string g_last_error;
-
-void set_error(const char* fmt, ...) {
-    char buf[1024];
-    va_list ap;
-    va_start(ap, fmt);
-    vsnprintf(buf, sizeof buf, fmt, ap);
-    va_end(ap);
-    g_last_error = buf;
-}
-
-gz_status fail(gz_status s, const char* fmt, ...) {
-    char buf[1024];
-    va_list ap;
-    va_start(ap, fmt);
-    vsnprintf(buf, sizeof buf, fmt, ap);
-    va_end(ap);
-    g_last_error = buf;
-    return s;
-}
-
-gz_status hip_fail(hipError_t e, const char* what, const char* file, int line) {
-    set_error("%s failed: %s (%s:%d)", what, hipGetErrorString(e), file, line);
-    return (e == hipErrorOutOfMemory) ? GZ_ERR_NOMEM : GZ_ERR_HIP;
-}
-
-const char* last_error_cstr() { return g_last_error.c_str(); }
-void clear_error() { g_last_error.clear(); }
-
-gz_status DevMem::reserve(size_t want) {
-    if (want <= bytes && p) return GZ_OK;
-    if (p) {
-        // work already queued may still read the old buffer
-        GZ_HIP(hipDeviceSynchronize());
-        GZ_HIP(hipFree(p));
-        p = nullptr;
-        bytes = 0;
-    }
-    const size_t b = std::max<size_t>(want, 256);
-    GZ_HIP(hipMalloc(&p, b));
-    bytes = b;
-    return GZ_OK;
-}
-
-void DevMem::release() {
-    if (p) (void)hipFree(p);
-    p = nullptr;
-    bytes = 0;
-}
-
-gz_status BlockCache::get(size_t bytes, void** p, size_t* got) {
-    const size_t want = (std::max<size_t>(bytes, 1) + 4095) & ~size_t(4095);
-    {
-        std::lock_guard<std::mutex> lock(mu_);
-        int best = -1;
-        for (int i = 0; i < n_; ++i)
-            if (size_[i] >= want && size_[i] - want <= want / 4 &&
-                (best < 0 || size_[i] < size_[best]))
-                best = i;
-        if (best >= 0) {
-            *p = ptr_[best];
-            *got = size_[best];
-            held_ -= size_[best];
-            --n_;
-            ptr_[best] = ptr_[n_];
-            size_[best] = size_[n_];
-            return GZ_OK;
-        }
-    }
-    hipError_t e = hipMalloc(p, want);
-    if (e == hipErrorOutOfMemory) {
-        (void)hipGetLastError();
-        drain();
-        e = hipMalloc(p, want);
-    }
-    if (e != hipSuccess) {
-        *p = nullptr;
-        return hip_fail(e, "hipMalloc", __FILE__, __LINE__);
-    }
-    *got = want;
-    return GZ_OK;
-}
-
-void BlockCache::put(void* p, size_t bytes) {
-    {
-        std::lock_guard<std::mutex> lock(mu_);
-        if (open_ && n_ < kBlocks && held_ + bytes <= kBytes) {
-            ptr_[n_] = p;
-            size_[n_] = bytes;
-            ++n_;
-            held_ += bytes;
-            return;
-        }
-    }
-    (void)hipFree(p);
-}
-
-void BlockCache::drain() {
-    std::lock_guard<std::mutex> lock(mu_);
-    for (int i = 0; i < n_; ++i) (void)hipFree(ptr_[i]);
-    n_ = 0;
-    held_ = 0;
-}
-
-void BlockCache::close() {
-    {
-        std::lock_guard<std::mutex> lock(mu_);
-        open_ = false;
-    }
-    drain();
-}
 
 // ---- wave / block scans ----------------------------------------------------------------------
 __device__ __forceinline__ uint32_t wave_inclusive_scan(uint32_t x) {
