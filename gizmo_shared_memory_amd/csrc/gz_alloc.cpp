@@ -60,8 +60,15 @@ void DevMem::release() {
     bytes = 0;
 }
 
+// The block size that serves `bytes`: up to an eighth more, in whole pages.
+static size_t block_size(size_t bytes) {
+    size_t step = 4096;
+    while (bytes > 16 * step) step *= 2;
+    return (std::max<size_t>(bytes, 1) + step - 1) / step * step;
+}
+
 gz_status BlockCache::get(size_t bytes, DevBlock* out) {
-    const size_t want = (std::max<size_t>(bytes, 1) + 4095) & ~size_t(4095);
+    const size_t want = block_size(bytes);
     {
         std::lock_guard<std::mutex> lock(mu_);
         int best = -1;
@@ -72,7 +79,8 @@ gz_status BlockCache::get(size_t bytes, DevBlock* out) {
         if (best >= 0) {
             *out = kept_[best];
             held_ -= out->bytes;
-            kept_[best] = kept_[--n_];
+            std::copy(kept_ + best + 1, kept_ + n_, kept_ + best);
+            --n_;
             return GZ_OK;
         }
     }
@@ -94,7 +102,12 @@ gz_status BlockCache::get(size_t bytes, DevBlock* out) {
 void BlockCache::put(DevBlock b) {
     {
         std::lock_guard<std::mutex> lock(mu_);
-        if (open_ && n_ < kBlocks && held_ + b.bytes <= kBytes) {
+        if (open_ && b.bytes <= kBytes) {
+            int old = (n_ == kBlocks) ? 1 : 0;
+            size_t held = held_;
+            for (int i = 0; i < old; ++i) held -= kept_[i].bytes;
+            while (held + b.bytes > kBytes) held -= kept_[old++].bytes;
+            evict(old);
             kept_[n_++] = b;
             held_ += b.bytes;
             return;
@@ -113,11 +126,18 @@ void BlockCache::retire(const DevBlock* b, int n) {
     if (!idle) (void)hipGetLastError(); // (the next launch's check is not to find it)
 }
 
+void BlockCache::evict(int n) {
+    for (int i = 0; i < n; ++i) {
+        (void)hipFree(kept_[i].p);
+        held_ -= kept_[i].bytes;
+    }
+    std::copy(kept_ + n, kept_ + n_, kept_);
+    n_ -= n;
+}
+
 void BlockCache::drain() {
     std::lock_guard<std::mutex> lock(mu_);
-    for (int i = 0; i < n_; ++i) (void)hipFree(kept_[i].p);
-    n_ = 0;
-    held_ = 0;
+    evict(n_);
 }
 
 void BlockCache::close() {

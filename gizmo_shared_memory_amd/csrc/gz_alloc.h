@@ -45,11 +45,14 @@ struct DevBlock {
 };
 
 // Device blocks that freed trees leave for the next build on their context: a tree is some 25
-// arrays, and at 4M particles freeing and allocating them took 4.6 of a rebuild's 5.3 ms. It
-// holds at most kBytes and kBlocks (beyond that blocks go back to the device), and gives
-// everything back when its context is destroyed or an allocation here finds no memory. Trees may
-// be freed by another thread than the one that builds (the list is locked), and after their
-// context (they share the cache's ownership; it then keeps nothing).
+// arrays, and at 4M particles freeing and allocating them took 4.6 of a rebuild's 5.3 ms. Blocks
+// come in sizes an eighth of a power of two apart, so that a tree that grows a little from one
+// rebuild to the next finds its blocks again (exact sizes left each tree's blocks useless to the
+// next: a rebuild of a 4M tree that grows by 0.1% a time took 6.6 to 27 ms once the cache was full
+// of them, now 2.6). It holds at most kBytes and kBlocks; beyond that the blocks put longest ago go back to
+// the device, and everything does when its context is destroyed or an allocation here finds no
+// memory. Trees may be freed by another thread than the one that builds (the list is locked), and
+// after their context (they share the cache's ownership; it then keeps nothing).
 class BlockCache {
 public:
     static constexpr size_t kBytes = size_t(2) << 30;
@@ -66,8 +69,9 @@ public:
     void close(); // drain, and keep nothing from now on
 
 private:
+    void evict(int n); // the n put longest ago (the list is locked)
     std::mutex mu_;
-    DevBlock kept_[kBlocks];
+    DevBlock kept_[kBlocks]; // in the order they were put
     int n_ = 0;
     size_t held_ = 0;
     bool open_ = true;

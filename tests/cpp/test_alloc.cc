@@ -95,8 +95,84 @@ static void refused_wait() {
     CHECK(dev.live.size() == 3); // those refused, which the device kept
 }
 
+// The blocks of a tree of n particles, as a build takes them.
+static std::vector<DevBlock> tree(BlockCache& c, size_t n, double cells = 0.375) {
+    const size_t nodes = (size_t)(cells * n) + 1024;
+    const size_t sizes[] = {4 * n, 4 * n, 4 * n, 8 * n, 4 * n, 32 * n, 8 * n, 64 * nodes, 4 * nodes,
+                            4 * nodes, 4 * nodes, 4 * nodes, 8 * nodes, 8 * nodes, 8 * nodes,
+                            8 * nodes, 8 * nodes, 8 * nodes, 96, 6 * nodes, 8};
+    std::vector<DevBlock> t;
+    for (size_t s : sizes) {
+        DevBlock b;
+        CHECK(c.get(s, &b) == GZ_OK && b.bytes >= s);
+        CHECK(4 * b.bytes <= 5 * (s + s / 8 + 4096)); // a kept one may be a quarter larger
+        for (auto& o : t) CHECK(o.p != b.p);
+        t.push_back(b);
+    }
+    return t;
+}
+
+static size_t held(const std::vector<DevBlock>& t) {
+    size_t s = 0;
+    for (auto& b : t) s += b.bytes;
+    return s;
+}
+
+// A tree that grows a little from rebuild to rebuild keeps finding its blocks, and so does one that
+// follows trees of quite other sizes.
+static void growing_trees() {
+    for (double n0 : {5e4, 1e6, 4e6}) {
+        BlockCache c;
+        long first = 0;
+        for (int i = 0; i < 400; ++i) {
+            const std::vector<DevBlock> t = tree(c, (size_t)(n0 * (1.0 + 1e-3 * i)));
+            c.retire(t.data(), (int)t.size());
+            CHECK(dev.used() <= BlockCache::kBytes && dev.live.size() <= BlockCache::kBlocks);
+            if (i == 0) first = dev.mallocs;
+        }
+        // 1.4 times as large: some four steps of the sizes for each array
+        CHECK(dev.mallocs - first <= 6 * first);
+        for (double f : {2.0, 3.1, 0.4, 0.3, 5.0}) {
+            const std::vector<DevBlock> t = tree(c, (size_t)(f * n0));
+            c.retire(t.data(), (int)t.size());
+        }
+        std::vector<DevBlock> t = tree(c, (size_t)n0);
+        c.retire(t.data(), (int)t.size());
+        const long before = dev.mallocs;
+        t = tree(c, (size_t)(1.0001 * n0));
+        CHECK(dev.mallocs - before <= 2);
+        c.retire(t.data(), (int)t.size());
+        c.close();
+        CHECK(dev.live.empty());
+        dev.mallocs = 0;
+    }
+}
+
+// A tree larger than what is kept: most of its blocks are.
+static void large_tree() {
+    BlockCache c;
+    std::vector<DevBlock> t = tree(c, 20000000);
+    CHECK(held(t) > BlockCache::kBytes);
+    for (int i = 0; i < 5; ++i) {
+        const long before = dev.mallocs;
+        if (i) t = tree(c, 20000000);
+        CHECK(i == 0 || dev.mallocs - before <= (long)t.size() / 2);
+        c.retire(t.data(), (int)t.size());
+        CHECK(dev.used() <= BlockCache::kBytes);
+    }
+    DevBlock b;
+    CHECK(c.get(BlockCache::kBytes + 1, &b) == GZ_OK);
+    const size_t kept = dev.live.size() - 1;
+    c.retire(&b, 1); // larger than all that may be kept: straight back, the others stay
+    CHECK(dev.live.size() == kept);
+    c.close();
+    CHECK(dev.live.empty());
+}
+
 int main(int argc, char** argv) {
-    const std::map<std::string, void (*)()> checks = {{"refused_wait", refused_wait}};
+    const std::map<std::string, void (*)()> checks = {{"refused_wait", refused_wait},
+                                                         {"growing_trees", growing_trees},
+                                                         {"large_tree", large_tree}};
     CHECK(argc == 2 && checks.count(argv[1]));
     checks.at(argv[1])();
     std::printf("ok\n");
