@@ -39,6 +39,19 @@ const char* last_error_cstr() { return g_last_error.c_str(); }
 void clear_error() { g_last_error.clear(); }
 
 // ---- device memory ---------------------------------------------------------------------------
+gz_status device_alloc(BlockCache* cache, void** p, size_t bytes) {
+    hipError_t e = hipMalloc(p, bytes);
+    if (e == hipErrorOutOfMemory && cache) {
+        (void)hipGetLastError();
+        cache->drain();
+        e = hipMalloc(p, bytes);
+    }
+    if (e == hipSuccess) return GZ_OK;
+    (void)hipGetLastError(); // (reported here; the next launch's check is not to find it)
+    *p = nullptr;
+    return hip_fail(e, "hipMalloc", __FILE__, __LINE__);
+}
+
 gz_status DevMem::reserve(size_t want) {
     if (want <= bytes && p) return GZ_OK;
     if (p) {
@@ -49,7 +62,7 @@ gz_status DevMem::reserve(size_t want) {
         bytes = 0;
     }
     const size_t b = std::max<size_t>(want, 256);
-    GZ_HIP(hipMalloc(&p, b));
+    GZ_TRY(device_alloc(cache, &p, b));
     bytes = b;
     return GZ_OK;
 }
@@ -84,17 +97,7 @@ gz_status BlockCache::get(size_t bytes, DevBlock* out) {
             return GZ_OK;
         }
     }
-    *out = {nullptr, 0};
-    hipError_t e = hipMalloc(&out->p, want);
-    if (e == hipErrorOutOfMemory) {
-        (void)hipGetLastError();
-        drain();
-        e = hipMalloc(&out->p, want);
-    }
-    if (e != hipSuccess) {
-        out->p = nullptr;
-        return hip_fail(e, "hipMalloc", __FILE__, __LINE__);
-    }
+    GZ_TRY(device_alloc(this, &out->p, want));
     out->bytes = want;
     return GZ_OK;
 }

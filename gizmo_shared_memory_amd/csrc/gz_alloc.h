@@ -30,10 +30,17 @@ void clear_error();
     } while (0)
 
 // ---- device memory --------------------------------------------------------------------------
+class BlockCache;
+
+// Device memory for a context whose freed trees left their blocks in cache: on out of memory those
+// are given back and the allocation is tried again.
+gz_status device_alloc(BlockCache* cache, void** p, size_t bytes);
+
 // Grow-only device allocation.
 struct DevMem {
     void* p = nullptr;
     size_t bytes = 0;
+    BlockCache* cache = nullptr; // the context's
     gz_status reserve(size_t want);
     void release();
     template <class T> T* as() const { return static_cast<T*>(p); }
@@ -50,8 +57,8 @@ struct DevBlock {
 // rebuild to the next finds its blocks again (exact sizes left each tree's blocks useless to the
 // next: a rebuild of a 4M tree that grows by 0.1% a time took 6.6 to 27 ms once the cache was full
 // of them, now 2.6). It holds at most kBytes and kBlocks; beyond that the blocks put longest ago go back to
-// the device, and everything does when its context is destroyed or an allocation here finds no
-// memory. Trees may be freed by another thread than the one that builds (the list is locked), and
+// the device, and everything does when its context is destroyed or an allocation of the context
+// finds no memory. Trees may be freed by another thread than the one that builds (the list is locked), and
 // after their context (they share the cache's ownership; it then keeps nothing).
 class BlockCache {
 public:

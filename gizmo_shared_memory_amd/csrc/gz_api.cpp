@@ -419,6 +419,7 @@ gz_status gz_ctx_create(int device, void* stream, gz_ctx** out) {
         delete c;
         return fail(GZ_ERR_NOMEM, "gz_ctx_create: out of host memory");
     }
+    for (auto& m : c->scratch) m.cache = c->blocks.get();
     if (stream) {
         c->stream = static_cast<hipStream_t>(stream);
     } else {
@@ -1041,10 +1042,10 @@ gz_status gz_walk_plan_create(gz_ctx* ctx, const gz_tree* tree, const gz_particl
                  o_rl = c.add<int>(n_t + 1), o_seg = c.add<uint32_t>(n_seg + 2),
                  o_sc = c.add<float>(model ? n_t : 1), o_ts = c.add<int>(n_t),
                  o_stk = c.add<int>((size_t)P->retry_waves * P->gstack_cap);
-    hipError_t e = hipMalloc(&P->mem, c.used);
-    if (e != hipSuccess) {
+    const gz_status m = gz::device_alloc(ctx->blocks.get(), &P->mem, c.used);
+    if (m != GZ_OK) {
         delete P;
-        return gz::hip_fail(e, "hipMalloc", __FILE__, __LINE__);
+        return m;
     }
     uint8_t* b = static_cast<uint8_t*>(P->mem);
     P->gstart = reinterpret_cast<int*>(b + o_gs);
@@ -1084,8 +1085,7 @@ gz_status gz_walk_plan_create(gz_ctx* ctx, const gz_tree* tree, const gz_particl
     }
     if (s == GZ_OK && model && P->ngroups > 0) {
         void* f = nullptr;
-        if (hipMalloc(&f, (size_t)P->ngroups * sizeof(gz::GroupStats)) != hipSuccess)
-            s = fail(GZ_ERR_NOMEM, "gz_walk_plan_create: no device memory for group features");
+        s = gz::device_alloc(ctx->blocks.get(), &f, (size_t)P->ngroups * sizeof(gz::GroupStats));
         P->stats = static_cast<gz::GroupStats*>(f);
     }
     if (s != GZ_OK) {
@@ -1240,10 +1240,10 @@ gz_status gz_model_create(gz_ctx* ctx, const float* host_params, gz_model** out)
     const size_t nf = (size_t)gz::kMlpParams;
     const size_t bytes = 4 * nf * sizeof(float) + 256 + 4 * gz::kMlpIn * sizeof(float) +
                          nf * sizeof(uint16_t) + 1024;
-    hipError_t e = hipMalloc(&M->mem, bytes);
-    if (e != hipSuccess) {
+    const gz_status a = gz::device_alloc(ctx->blocks.get(), &M->mem, bytes);
+    if (a != GZ_OK) {
         delete M;
-        return gz::hip_fail(e, "hipMalloc", __FILE__, __LINE__);
+        return a;
     }
     float* f = static_cast<float*>(M->mem);
     M->theta = f;

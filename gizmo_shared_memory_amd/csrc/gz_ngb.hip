@@ -872,7 +872,7 @@ extern "C" gz_status gz_tree_init_hmax(gz_ctx* ctx, gz_tree* tree, const double*
     if (nn <= 0) return GZ_OK;
     if (!tree->hmax) {
         void* p = nullptr;
-        GZ_HIP(hipMalloc(&p, (size_t)nn * sizeof(float)));
+        GZ_TRY(device_alloc(tree->blocks.get(), &p, (size_t)nn * sizeof(float)));
         tree->hmax = static_cast<float*>(p);
     }
     GZ_TRY(fill_zero_u32(reinterpret_cast<uint32_t*>(tree->hmax), (size_t)nn, st));

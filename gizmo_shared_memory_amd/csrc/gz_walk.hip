@@ -1241,7 +1241,7 @@ gz_status ctx_spill(gz_ctx* ctx, int** spill, int* cap) {
         int waves = 0;
         GZ_TRY(persistent_waves(&waves));
         void* p = nullptr;
-        GZ_HIP(hipMalloc(&p, (size_t)waves * kSpillCap * sizeof(int)));
+        GZ_TRY(device_alloc(ctx->blocks.get(), &p, (size_t)waves * kSpillCap * sizeof(int)));
         ctx->spill = static_cast<int*>(p);
         ctx->spill_cap = kSpillCap;
     }

@@ -169,10 +169,37 @@ static void large_tree() {
     CHECK(dev.live.empty());
 }
 
+// Kept blocks make way for every other allocation of their context, which fails only when the device
+// is full without them, and leaves no error behind for the next call's check.
+static void room_for_others() {
+    BlockCache c;
+    std::vector<DevBlock> t = tree(c, 4000000);
+    c.retire(t.data(), (int)t.size());
+    const size_t kept = dev.used();
+    CHECK(kept > size_t(300) << 20);
+    dev.room = kept + (size_t(64) << 20);
+    gz::DevMem m;
+    m.cache = &c;
+    CHECK(m.reserve(size_t(32) << 20) == GZ_OK && dev.used() == kept + m.bytes);
+    CHECK(m.reserve(kept) == GZ_OK && m.bytes == kept && dev.used() == kept);
+    CHECK(hipGetLastError() == hipSuccess);
+    CHECK(m.reserve(dev.room + 1) == GZ_ERR_NOMEM && m.p == nullptr && m.bytes == 0);
+    CHECK(hipGetLastError() == hipSuccess);
+    CHECK(m.reserve(kept) == GZ_OK);
+    m.release();
+    t = tree(c, 4000000);
+    c.retire(t.data(), (int)t.size());
+    void* p = nullptr;
+    CHECK(gz::device_alloc(&c, &p, kept) == GZ_OK && dev.used() == kept);
+    CHECK(gz::device_alloc(nullptr, &p, dev.room) == GZ_ERR_NOMEM && p == nullptr);
+    c.close();
+}
+
 int main(int argc, char** argv) {
     const std::map<std::string, void (*)()> checks = {{"refused_wait", refused_wait},
                                                          {"growing_trees", growing_trees},
-                                                         {"large_tree", large_tree}};
+                                                         {"large_tree", large_tree},
+                                                         {"room_for_others", room_for_others}};
     CHECK(argc == 2 && checks.count(argv[1]));
     checks.at(argv[1])();
     std::printf("ok\n");
