@@ -67,6 +67,12 @@ gz_status DevMem::reserve(size_t want) {
     return GZ_OK;
 }
 
+bool DevMem::offer(size_t want) {
+    if (reserve(want) == GZ_OK) return true;
+    clear_error();
+    return false;
+}
+
 void DevMem::release() {
     if (p) (void)hipFree(p);
     p = nullptr;
@@ -138,15 +144,25 @@ void BlockCache::evict(int n) {
     n_ -= n;
 }
 
+void BlockCache::lend(DevMem* m) {
+    if (n_lent_ < (int)(sizeof lent_ / sizeof *lent_)) lent_[n_lent_++] = m;
+}
+
 void BlockCache::drain() {
     std::lock_guard<std::mutex> lock(mu_);
     evict(n_);
+    for (int i = 0; i < n_lent_; ++i) {
+        DevMem& m = *lent_[i];
+        // (queued work may still read it)
+        if (m.p && !m.in_use && hipDeviceSynchronize() == hipSuccess) m.release();
+    }
 }
 
 void BlockCache::close() {
     {
         std::lock_guard<std::mutex> lock(mu_);
         open_ = false;
+        n_lent_ = 0; // (the context frees its scratch)
     }
     drain();
 }

@@ -32,8 +32,8 @@ void clear_error();
 // ---- device memory --------------------------------------------------------------------------
 class BlockCache;
 
-// Device memory for a context whose freed trees left their blocks in cache: on out of memory those
-// are given back and the allocation is tried again.
+// Device memory for a context whose freed trees left their blocks in cache: on out of memory those,
+// and scratch lent to it, are given back and the allocation is tried again.
 gz_status device_alloc(BlockCache* cache, void** p, size_t bytes);
 
 // Grow-only device allocation.
@@ -41,9 +41,20 @@ struct DevMem {
     void* p = nullptr;
     size_t bytes = 0;
     BlockCache* cache = nullptr; // the context's
+    bool in_use = false;         // a call has its contents there (ScratchUse)
     gz_status reserve(size_t want);
+    // The same for memory that a call can do without: false when there is not enough (what was
+    // here is gone then).
+    bool offer(size_t want);
     void release();
     template <class T> T* as() const { return static_cast<T*>(p); }
+};
+
+struct ScratchUse {
+    DevMem& m;
+    explicit ScratchUse(DevMem& mem) : m(mem) { m.in_use = true; }
+    ~ScratchUse() { m.in_use = false; }
+    ScratchUse(const ScratchUse&) = delete;
 };
 
 struct DevBlock {
@@ -72,6 +83,9 @@ public:
     // be waited for (some stream of the process is being captured) they go back to the device
     // instead, whose own free waits, or refuses.
     void retire(const DevBlock* b, int n);
+    // Scratch of the context that drain gives back too when no call has its contents there: what is
+    // large, kept for speed alone, and no captured graph reads.
+    void lend(DevMem* m);
     void drain();
     void close(); // drain, and keep nothing from now on
 
@@ -82,6 +96,8 @@ private:
     int n_ = 0;
     size_t held_ = 0;
     bool open_ = true;
+    DevMem* lent_[4];
+    int n_lent_ = 0;
 };
 
 } // namespace gz

@@ -420,6 +420,8 @@ gz_status gz_ctx_create(int device, void* stream, gz_ctx** out) {
         return fail(GZ_ERR_NOMEM, "gz_ctx_create: out of host memory");
     }
     for (auto& m : c->scratch) m.cache = c->blocks.get();
+    // sort buffers and packed particles, levels, the search's, the density solve's
+    for (int k : {2, 4, 10, 13}) c->blocks->lend(&c->scratch[k]);
     if (stream) {
         c->stream = static_cast<hipStream_t>(stream);
     } else {

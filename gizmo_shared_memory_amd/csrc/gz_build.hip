@@ -330,14 +330,15 @@ __global__ __launch_bounds__(kThreads) void k_gather_sorted(
 }
 
 // grow: the records' memory may be allocated (else they are used only if there is room already).
+// A line per particle is much to ask for late in a large build: without it the arrays are read.
 static gz_status gather_sources(const gz_particles* p, const uint32_t* orderbuf, size_t nl,
                                 double4* src, double* src_soft, DevMem& mem, bool grow,
                                 hipStream_t st) {
     if (nl == 0) return GZ_OK;
     const size_t rec_bytes = p->n * sizeof(PRec);
     // (packing the dead particles of a set that is mostly dead would cost more than it saves)
-    if (nl >= kPackRec && nl >= p->n / 2 && (grow || mem.bytes >= rec_bytes)) {
-        GZ_TRY(mem.reserve(rec_bytes));
+    if (nl >= kPackRec && nl >= p->n / 2 &&
+        (grow ? mem.offer(rec_bytes) : mem.bytes >= rec_bytes)) {
         k_pack_rec<<<grid_for(p->n), kThreads, 0, st>>>(p->n, p->x, p->y, p->z, p->m, p->soft,
                                                         mem.as<PRec>());
         k_gather_rec<<<grid_for(nl), kThreads, 0, st>>>(orderbuf, nl, mem.as<PRec>(), src,
@@ -904,6 +905,7 @@ gz_status build_tree(gz_ctx* ctx, const gz_particles* p, const gz_build_opts* op
     const size_t nalloc = std::max<size_t>(n, 1);
     // order / keys ping-pong buffers
     DevMem& s2 = ctx->scratch[2];
+    ScratchUse s2_use(s2);
     GZ_TRY(s2.reserve(nalloc * (2 * sizeof(uint64_t) + 2 * sizeof(uint32_t)) + 256));
     uint64_t* k0 = s2.as<uint64_t>();
     uint64_t* k1 = k0 + nalloc;
@@ -977,6 +979,7 @@ gz_status build_tree(gz_ctx* ctx, const gz_particles* p, const gz_build_opts* op
         GZ_HIP(hipGetLastError());
     }
     GZ_TRY(gather_sources(p, t->orderbuf, nl, t->src, t->src_soft, ctx->scratch[2], true, st));
+    s2.in_use = false;
     GZ_HIP(hipEventRecord(ev[4], st));
 
     // --- topology, level by level
@@ -1012,14 +1015,23 @@ gz_status build_tree(gz_ctx* ctx, const gz_particles* p, const gz_build_opts* op
         GZ_HIP(hipGetLastError());
     }
     DevMem& s4 = ctx->scratch[4];
+    ScratchUse s4_use(s4);
     // Levels are enqueued in batches, a read-back of the table after each: as many as a tree of nl
     // particles has unless it is deeply clustered, then four at a time.
     int level = 0, batch = 5;
     for (size_t k = nl / (size_t)nc; k > 8; k >>= 3) ++batch;
     for (bool done = false; !done;) {
-        // a level holds at most cap nodes
-        const size_t per = (size_t)cap, sums = (per + kLevelChunk - 1) / kLevelChunk;
-        GZ_TRY(s4.reserve((per * 9 + sums) * sizeof(int) + 768));
+        // a level holds at most cap nodes; when there is no memory for that many, the next level
+        // alone, whose size is known
+        auto bytes = [](size_t nodes) {
+            return (nodes * 9 + (nodes + kLevelChunk - 1) / kLevelChunk) * sizeof(int) + 768;
+        };
+        size_t per = (size_t)cap;
+        if (!s4.offer(bytes(per))) {
+            per = (size_t)(t->level_begin[level + 1] - t->level_begin[level]);
+            batch = 1;
+            GZ_TRY(s4.reserve(bytes(per)));
+        }
         int* oct = s4.as<int>();
         uint32_t* nk = reinterpret_cast<uint32_t*>(oct + 8 * per);
         uint32_t* csum = nk + per;
@@ -1075,6 +1087,7 @@ gz_status build_tree(gz_ctx* ctx, const gz_particles* p, const gz_build_opts* op
         }
         batch = 4;
     }
+    s4.in_use = false;
     const int nnodes = t->level_begin.back();
     t->nnodes = nnodes;
     t->depth = (int)t->level_begin.size() - 2;

@@ -928,7 +928,7 @@ extern "C" gz_status gz_tree_density(gz_ctx* ctx, const gz_tree* tree, const gz_
     // Many targets: the particles' live values are put in slot order first, where the targets of a
     // wave find their neighbours together (a neighbour's four values cost four scattered reads
     // otherwise, several times a call)
-    const bool by_slot = n_t >= tree->n_live / 8;
+    bool by_slot = n_t >= tree->n_live / 8;
     const size_t o_lo = take(n_t * 8), o_hi = take(n_t * 8), o_iter = take(n_t * 4),
                  o_act = take(n_t * 4), o_nxt = take(n_t * 4), o_keep = take((n_t + 1) * 4),
                  o_scan = take((n_t + 1) * 4), o_kept = take((n_t + 1) * 4),
@@ -936,11 +936,13 @@ extern "C" gz_status gz_tree_density(gz_ctx* ctx, const gz_tree* tree, const gz_
                  o_v0 = take(n_t * 4), o_v1 = take(n_t * 4), o_far = take(n_t * 4),
                  o_fact = take(n_t * 4), o_fkeep = take(n_t * 4),
                  o_srec = take((size_t)std::max(tree->nnodes, 1) * sizeof(SRec)),
+                 o_misc = take(256), o_tmp = take(scan_tmp_bytes(n_t + 1)), need = off,
                  o_live = take(by_slot ? tree->n_live * sizeof(double4) : 0),
-                 o_gas = take(by_slot && p->type ? tree->n_live : 0),
-                 o_misc = take(256), o_tmp = take(scan_tmp_bytes(n_t + 1));
+                 o_gas = take(by_slot && p->type ? tree->n_live : 0);
     DevMem& mem = ctx->scratch[13];
-    GZ_TRY(mem.reserve(off));
+    ScratchUse mem_use(mem);
+    by_slot = by_slot && mem.offer(off); // (without the memory for it: through orderbuf)
+    GZ_TRY(mem.reserve(need));
     uint8_t* base = mem.as<uint8_t>();
     double* d_lo = reinterpret_cast<double*>(base + o_lo);
     double* d_hi = reinterpret_cast<double*>(base + o_hi);

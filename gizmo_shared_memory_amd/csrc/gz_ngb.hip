@@ -685,16 +685,23 @@ static gz_status ngb_run(gz_ctx* ctx, const gz_tree* tree, const double* cx, con
         waves = std::max(1, ncu) * 16; // the spill arena holds this many slices
     }
     DevMem& s = ctx->scratch[10];
+    ScratchUse s_use(s);
     const size_t cnt_bytes = ((n_q + 1) * sizeof(uint32_t) + 255) & ~size_t(255);
     const size_t tmp_bytes = (256 + scan_tmp_bytes(n_q + 1) + 255) & ~size_t(255);
     // forward: the search nodes, and a row per query unless the caller has room for longer lists
     // (packing reads the whole tree, 75 us at 4M particles: for a few queries it would be most of
     // the search)
-    const bool packed = !rev && n_q >= tree->n_live / 16;
-    const size_t srec_bytes = packed ? (size_t)tree->nnodes * sizeof(SRec) : 0;
+    bool packed = !rev && n_q >= tree->n_live / 16;
+    size_t srec_bytes = packed ? (size_t)tree->nnodes * sizeof(SRec) : 0;
     const size_t row_bytes = n_q * kNgbRow * sizeof(uint32_t);
-    const bool rows = !rev && found && cap / kNgbRow <= n_q && row_bytes <= kNgbRowsMax;
-    GZ_TRY(s.reserve(cnt_bytes + tmp_bytes + srec_bytes + (rows ? row_bytes : 0)));
+    bool rows = !rev && found && cap / kNgbRow <= n_q && row_bytes <= kNgbRowsMax;
+    // (both only when there is memory for them)
+    rows = rows && s.offer(cnt_bytes + tmp_bytes + srec_bytes + row_bytes);
+    if (packed && !rows && !s.offer(cnt_bytes + tmp_bytes + srec_bytes)) {
+        packed = false;
+        srec_bytes = 0;
+    }
+    GZ_TRY(s.reserve(cnt_bytes + tmp_bytes));
     uint8_t* b = s.as<uint8_t>();
     uint32_t* count = reinterpret_cast<uint32_t*>(b);
     int* misc = reinterpret_cast<int*>(b + cnt_bytes);
@@ -872,7 +879,7 @@ extern "C" gz_status gz_tree_init_hmax(gz_ctx* ctx, gz_tree* tree, const double*
     if (nn <= 0) return GZ_OK;
     if (!tree->hmax) {
         void* p = nullptr;
-        GZ_TRY(device_alloc(tree->blocks.get(), &p, (size_t)nn * sizeof(float)));
+        GZ_TRY(device_alloc(ctx->blocks.get(), &p, (size_t)nn * sizeof(float)));
         tree->hmax = static_cast<float*>(p);
     }
     GZ_TRY(fill_zero_u32(reinterpret_cast<uint32_t*>(tree->hmax), (size_t)nn, st));

@@ -195,11 +195,41 @@ static void room_for_others() {
     c.close();
 }
 
+// So does scratch that no call is using; a call can do without what it only offers to take.
+static void lent_scratch() {
+    BlockCache c;
+    gz::DevMem a, b;
+    a.cache = b.cache = &c;
+    c.lend(&a);
+    c.lend(&b);
+    dev.room = size_t(300) << 20;
+    CHECK(a.reserve(size_t(200) << 20) == GZ_OK);
+    {
+        gz::ScratchUse use(a);
+        CHECK(!b.offer(size_t(150) << 20) && b.p == nullptr && a.p != nullptr);
+        CHECK(*gz::last_error_cstr() == 0);
+        CHECK(b.offer(size_t(50) << 20));
+        CHECK(b.offer(size_t(50) << 20) && b.bytes == size_t(50) << 20);
+    }
+    DevBlock t;
+    CHECK(c.get(size_t(250) << 20, &t) == GZ_OK && !a.p && !b.p && dev.waits > 0);
+    dev.refuse = true; // nothing is given back that may still be read
+    c.put(t);
+    CHECK(a.reserve(size_t(1) << 20) == GZ_OK);
+    CHECK(b.reserve(size_t(300) << 20) == GZ_ERR_NOMEM && a.p);
+    dev.refuse = false;
+    c.close();
+    DevBlock u;
+    CHECK(c.get(size_t(290) << 20, &u) == GZ_ERR_NOMEM && a.p); // the context frees its scratch
+    a.release();
+}
+
 int main(int argc, char** argv) {
     const std::map<std::string, void (*)()> checks = {{"refused_wait", refused_wait},
                                                          {"growing_trees", growing_trees},
                                                          {"large_tree", large_tree},
-                                                         {"room_for_others", room_for_others}};
+                                                         {"room_for_others", room_for_others},
+                                                         {"lent_scratch", lent_scratch}};
     CHECK(argc == 2 && checks.count(argv[1]));
     checks.at(argv[1])();
     std::printf("ok\n");

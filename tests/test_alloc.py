@@ -22,7 +22,8 @@ def program(tmp_path_factory):
     return out
 
 
-@pytest.mark.parametrize("check", ["refused_wait", "growing_trees", "large_tree", "room_for_others"])
+@pytest.mark.parametrize("check", ["refused_wait", "growing_trees", "large_tree", "room_for_others",
+                                   "lent_scratch"])
 def test_kept_device_memory(program, check):
     r = subprocess.run([program, check], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0 and r.stdout == "ok\n", r.stdout + r.stderr
