@@ -15,12 +15,12 @@
 //     column of an LDS buffer; whenever some column is nearly full, and at the end, the lanes add
 //     their neighbours' terms. The targets that are done leave the active list (a stable
 //     compaction, so the waves keep their Morton locality).
-//   * k_density_near, for the last kLoopTargets: a wave per target, iterated to the end on
+//   * k_density_near, for the last kLastTargets: a wave per target, iterated to the end on
 //     candidates collected once.
 //   * k_density_far, a wave per target on the tree, for spheres that hold many particles: in a
 //     round, targets whose radius exceeds kFarLeaf times their leaf's side (one of them would make
 //     its wave of 64 walk a large part of the tree), and among the last, those with more than
-//     kNearMax candidates.
+//     kNearMax candidates, or all when that many neighbours are wanted.
 //
 // What bounds a round: at 4.2M targets (Hernquist, 3% from converged) 38,500 VALU instructions a
 // wave, busy 4.4 of 7.0 ms, the rest latency at 2.5 waves per SIMD (LDS): about 14 instructions for
@@ -46,14 +46,36 @@ namespace {
 
 constexpr double kPi = 3.14159265358979323846;
 constexpr int kMaxIter = 100; // hydro.cc:201
-constexpr int kWavesWanted = 2048; // a round's targets are spread thinner below this many waves
 constexpr int kNbBuf = 32;          // neighbours each lane holds before their terms are added
-constexpr double kFarLeaf = 4.0;    // radius over leaf side beyond which a target takes the lists
-// Active targets few enough to iterate in one launch. Rounds are cheaper per target while a wave's
-// targets are neighbours; the fewer are left, the further apart they lie and the more launches and
-// read-backs they cost: on 4.2M targets the solve took 22.8 ms with 131,072, 22.3 with 524,288 and
-// 23.9 with 1,048,576; on 300k 4.7, 3.55 and 3.54, on 1M 8.4, 8.8 and 13.7.
-constexpr uint32_t kLoopTargets = 393216;
+constexpr double kFarLeaf = 4.0;    // radius over leaf side beyond which a target takes a wave
+// The last active targets iterate to the end in one launch. Rounds are cheaper per target while a
+// wave's targets are neighbours; the fewer are left, the further apart they lie and the more
+// launches and read-backs they cost. How many are the last, and which kernel takes them, depends on
+// how well a converged target's candidates (wanted neighbours times the volume of kNearMargin) fit
+// the 256 that k_density_near holds. ms a solve, guesses 2% off, by the limit and the kernel:
+//
+//   neighbours (candidates)      32 (49)   64 (97)   128 (195)  150 (228)  200 (304)  300 (456)
+//   300k Hernquist, 131,072 near    2.26      2.22      3.60       4.08       5.51       8.50
+//                   393,216 near    2.40      2.37      4.00       6.21      16.0       24.3
+//                   131,072 far     4.27      2.39      3.60       4.09       5.29       7.86
+//   300k halo+disk, 131,072 near    2.72      3.27      5.80       6.80       9.56      13.9
+//                   393,216 near    2.65      2.79      5.08       7.17      15.4       24.3
+//                   131,072 far     5.25      3.28      5.84       6.90       9.11      13.3
+//   60k Hernquist,  131,072 near     .73       .71      1.15       1.71       3.71       5.35
+//                   131,072 far     2.71      1.54      2.46       2.74       3.34       4.63
+//   1M Hernquist,   131,072 near    7.19      5.68      9.34      10.7       13.6       20.5
+//                   393,216 near    7.17      5.69      9.39      10.7       13.6       23.3
+//                   131,072 far     8.42      5.78      9.77      11.3       14.8       20.5
+//   4.2M Hernquist, 131,072 near   23.0                35.5                  53.5       73.2
+//                   393,216 near   22.6                35.5                  51.0       73.2
+//
+// So near to 310 candidates, of which up to 393,216 targets to 200 candidates, else 131,072.
+constexpr uint32_t kLastTargets = 393216, kLastTargetsFull = 131072;
+constexpr double kCollectMost = 200.0, kCollectMax = 310.0;
+// Up to this many targets the launch's time is its slowest target's, and one that starts from a
+// radius far too large takes that long twice in two kernels: 1,000 targets of 1M from rough guesses
+// .83 ms in two, .52 in one; from good ones .43 and .45, and 6% more for 8,000.
+constexpr uint32_t kNearFar = 2048;
 
 // kernel_norm, ball_vol, kernel_w, kernel_dwdh (hydro.h:29-65): cubic spline of support h in dim
 // dimensions, operand for operand.
@@ -184,7 +206,6 @@ __device__ __forceinline__ T ld_const(const T* p) {
 struct DensArgs {
     const uint32_t* act; // active targets (positions in the target list), in slot order
     int n_act;
-    int tpw;             // targets per wavefront (a power of two, at most 64)
     const uint32_t* targets;
     const double *x, *y, *z, *m;
     const uint8_t* type; // null: all gas
@@ -385,213 +406,227 @@ __device__ __forceinline__ double add_terms(const double (*s_v)[65], int lane, i
     return acc;
 }
 
-// One step for each of its targets (a.act[e] for block e), one wavefront per target walking that
-// target's own search depth first. The lanes test a node's children together (a forest's roots up
-// to 64 at a time), so the wave takes one step per admitted interior node; the admitted leaves
-// among a node's children up to its next admitted interior child are taken together, their
-// particles (contiguous slot ranges) spread over the lanes in slot order, tested against the
-// sphere, and the neighbours' terms computed into LDS in that order. Lane c (c < 12) then adds
-// term c of each, in order, so every sum is the round's, term by term. For the targets whose
-// spheres reach far beyond their leaf; with LOOP, the wave repeats its target's steps until the
-// target is done.
+// A step's sums for one target by a whole wave on the tree, the search walked depth first. The lanes
+// test a node's children together (a forest's roots up to 64 at a time), so the wave takes one step
+// per admitted interior node; the admitted leaves among a node's children up to its next admitted
+// interior child are taken together, their particles (contiguous slot ranges) spread over the
+// lanes in slot order, tested against the sphere, and the neighbours' terms computed into s_v in
+// that order. Lane c (c < 12) then adds term c of each, in order, so every sum is the round's, term
+// by term.
+__device__ __forceinline__ void far_sums(const DensArgs& a, double qx, double qy, double qz, double h,
+                                         double (*s_v)[65], DensSums* out) {
+    const int lane = threadIdx.x;
+    const int r_first = (a.nodes.nclusters > 1) ? 0 : a.nodes.root;
+    const int r_count = (a.nodes.nclusters > 1) ? a.nodes.nclusters : 1;
+    const double r2 = h * h; // the search's radius_sq (hydro.cc:50)
+    Kernel kern;
+    kern.set(h, a.n_dims);
+    // the node test of the forward search (hydro.cc:55-72), as the rounds evaluate it
+    auto admits = [&](const SRec& nr) -> bool {
+        double dist = h + (double)nr.half + (double)nr.xpad;
+        if (a.nodes.tau > 0) dist += (double)nr.vmax * a.nodes.tau;
+        const double dx = (double)nr.cx - qx, dy = (double)nr.cy - qy,
+                     dz = (double)nr.cz - qz;
+        if ((dx > dist || -dx > dist) || (dy > dist || -dy > dist) ||
+            (dz > dist || -dz > dist))
+            return false;
+        const double ds = dist + 0.7320508075688772 * (double)nr.half;
+        return !(dx * dx + dy * dy + dz * dz > ds * ds);
+    };
+    double acc = 0.0; // lane c < 12: term c's sum
+    int n_in = 0;     // the count inside h (the same in every lane)
+    int nbuf = 0;     // neighbours waiting in s_v (the same in every lane)
+    auto flush = [&]() {
+        __syncthreads();
+        acc = add_terms(s_v, lane, nbuf, acc);
+        __syncthreads();
+        nbuf = 0;
+    };
+    // one particle per lane (slot s, or none for s < 0): a neighbour when within the radius
+    // (the tree's copy of the position, as the search tests it), its terms packed into s_v
+    // in lane order
+    auto take = [&](int s) {
+        double v[kTerms];
+        bool inside = false, ok = false;
+        if (s >= 0) {
+            const double4 q = a.src[s];
+            const double ex = q.x - qx, ey = q.y - qy, ez = q.z - qz;
+            if (ex * ex + ey * ey + ez * ez < r2)
+                ok = density_terms(neighbour_at(a, s), qx, qy, qz, kern, v, &inside);
+        }
+        const uint64_t om = __ballot(ok);
+        if (om == 0) return;
+        const int n_ok = __builtin_popcountll(om);
+        if (nbuf + n_ok > 64) flush();
+        if (ok) {
+            const int pos = nbuf + lanes_under(om);
+#pragma unroll
+            for (int c = 0; c < kTerms; ++c) s_v[c][pos] = v[c];
+        }
+        n_in += __builtin_popcountll(__ballot(ok && inside));
+        nbuf += n_ok;
+    };
+    // the admitted leaves run (bit j: child cf + j), their particles in slot order
+    auto leaves = [&](int cf, uint64_t run) {
+        int plo = 0, cnt = 0, off = 0, total = 0;
+        if ((run >> lane) & 1ull) {
+            const SRec c = a.nodes.srec[cf + lane];
+            plo = ~c.link;
+            cnt = c.span - plo;
+        }
+        for (uint64_t r = run; r != 0; r &= r - 1) {
+            const int j = (int)__builtin_ctzll(r);
+            if (lane == j) off = total;
+            total += __builtin_amdgcn_readlane(cnt, j);
+        }
+        for (int g0 = 0; g0 < total; g0 += 64) {
+            const int g = g0 + lane;
+            int s = -1;
+            for (uint64_t r = run; r != 0; r &= r - 1) {
+                const int j = (int)__builtin_ctzll(r);
+                const int o = __builtin_amdgcn_readlane(off, j);
+                if (g >= o && g < o + __builtin_amdgcn_readlane(cnt, j))
+                    s = __builtin_amdgcn_readlane(plo, j) + (g - o);
+            }
+            take(s);
+        }
+    };
+    // A node whose box (its centre and half side as the node test reads them, so the cells
+    // below it too) lies inside the sphere, by a margin above the float rounding of node
+    // centres: every node below it is admitted, so the walk would test each of its particles
+    // in slot order. They are a contiguous slot range, taken 64 at a time instead.
+    auto inside_sphere = [&](const SRec& nr) -> bool {
+        const double hf = (double)nr.half;
+        const double ax = fabs((double)nr.cx - qx) + hf, ay = fabs((double)nr.cy - qy) + hf,
+                     az = fabs((double)nr.cz - qz) + hf;
+        const double m = 1e-6 * (fabs((double)nr.cx) + fabs((double)nr.cy) +
+                                 fabs((double)nr.cz));
+        const double hm = h * (1.0 - 1e-12) - m;
+        return hm > 0 && ax * ax + ay * ay + az * az < hm * hm;
+    };
+    for (int r0 = 0; r0 < r_count; r0 += 64) {
+        // the children of the node being walked (first index; lane masks of those admitted
+        // and not yet visited, and of those that are leaves) and the stack of the same above
+        // it, entry d in lane d
+        int cf = r_first + r0;
+        uint64_t cm, lm;
+        {
+            bool hit = false, leaf = false;
+            if (lane < min(64, r_count - r0)) {
+                const SRec c = a.nodes.srec[cf + lane];
+                hit = admits(c);
+                leaf = c.link < 0;
+            }
+            cm = __ballot(hit);
+            lm = __ballot(hit && leaf);
+        }
+        int sp = 0, stf = 0, sml = 0, smh = 0, sll = 0, slh = 0;
+        for (;;) {
+            if (cm == 0) {
+                if (sp == 0) break;
+                --sp;
+                cf = __builtin_amdgcn_readlane(stf, sp);
+                cm = ((uint64_t)(uint32_t)__builtin_amdgcn_readlane(smh, sp) << 32) |
+                     (uint64_t)(uint32_t)__builtin_amdgcn_readlane(sml, sp);
+                lm = ((uint64_t)(uint32_t)__builtin_amdgcn_readlane(slh, sp) << 32) |
+                     (uint64_t)(uint32_t)__builtin_amdgcn_readlane(sll, sp);
+                continue;
+            }
+            const uint64_t inner = cm & ~lm;
+            if ((cm & (0 - cm) & lm) != 0) {
+                // the next child is a leaf: it and the leaves after it up to the next
+                // interior child
+                const uint64_t run = inner ? (cm & ((inner & (0 - inner)) - 1)) : cm;
+                cm &= ~run;
+                leaves(cf, run);
+                continue;
+            }
+            // an interior child: its admitted children are walked before its remaining
+            // siblings, which wait on the stack
+            const int node = cf + (int)__builtin_ctzll(cm);
+            cm &= cm - 1;
+            const SRec nr = ld_const(a.nodes.srec + node);
+            if (inside_sphere(nr)) {
+                const WNode w = ld_const(a.wn + node);
+                for (int s0 = w.plo; s0 < w.phi; s0 += 64)
+                    take(s0 + lane < w.phi ? s0 + lane : -1);
+                continue;
+            }
+            bool hit = false, leaf = false;
+            if (lane < nr.span) {
+                const SRec c = a.nodes.srec[nr.link + lane];
+                hit = admits(c);
+                leaf = c.link < 0;
+            }
+            const uint64_t om = __ballot(hit);
+            if (om == 0) continue;
+            if (cm != 0) {
+                const bool top = lane == sp;
+                stf = top ? cf : stf;
+                sml = top ? (int)(uint32_t)cm : sml;
+                smh = top ? (int)(uint32_t)(cm >> 32) : smh;
+                sll = top ? (int)(uint32_t)lm : sll;
+                slh = top ? (int)(uint32_t)(lm >> 32) : slh;
+                ++sp;
+            }
+            cf = nr.link;
+            cm = om;
+            lm = __ballot(hit && leaf);
+        }
+    }
+    flush();
+#pragma unroll
+    for (int c = 0; c < kTerms; ++c) out->s[c] = __shfl(acc, c);
+    out->n_inside = n_in;
+}
+
+// Targets whose spheres reach far beyond their leaf, a wave each (a.act[e] for block e): one step, or
+// with LOOP their steps to the end.
 template <bool LOOP>
 __global__ __launch_bounds__(64) void k_density_far(DensArgs a) {
     __shared__ double s_v[kTerms][65]; // rows padded so the 12 adding lanes hit distinct banks
-    const int lane = threadIdx.x;
     const int e = blockIdx.x;
-    const int dim = a.n_dims;
     const uint32_t t = a.act[e];
     const uint32_t p = a.targets[t];
     const double qx = a.x[p], qy = a.y[p], qz = a.z[p];
-    const int r_first = (a.nodes.nclusters > 1) ? 0 : a.nodes.root;
-    const int r_count = (a.nodes.nclusters > 1) ? a.nodes.nclusters : 1;
     for (;;) {
         const double h = a.h[t];
         const int it = a.iter[t];
-        const double r2 = h * h; // the search's radius_sq (hydro.cc:50)
-        Kernel kern;
-        kern.set(h, dim);
-        // the node test of the forward search (hydro.cc:55-72), as the rounds evaluate it
-        auto admits = [&](const SRec& nr) -> bool {
-            double dist = h + (double)nr.half + (double)nr.xpad;
-            if (a.nodes.tau > 0) dist += (double)nr.vmax * a.nodes.tau;
-            const double dx = (double)nr.cx - qx, dy = (double)nr.cy - qy,
-                         dz = (double)nr.cz - qz;
-            if ((dx > dist || -dx > dist) || (dy > dist || -dy > dist) ||
-                (dz > dist || -dz > dist))
-                return false;
-            const double ds = dist + 0.7320508075688772 * (double)nr.half;
-            return !(dx * dx + dy * dy + dz * dz > ds * ds);
-        };
-        double acc = 0.0; // lane c < 12: term c's sum
-        int n_in = 0;     // the count inside h (the same in every lane)
-        int nbuf = 0;     // neighbours waiting in s_v (the same in every lane)
-        auto flush = [&]() {
-            __syncthreads();
-            acc = add_terms(s_v, lane, nbuf, acc);
-            __syncthreads();
-            nbuf = 0;
-        };
-        // one particle per lane (slot s, or none for s < 0): a neighbour when within the radius
-        // (the tree's copy of the position, as the search tests it), its terms packed into s_v
-        // in lane order
-        auto take = [&](int s) {
-            double v[kTerms];
-            bool inside = false, ok = false;
-            if (s >= 0) {
-                const double4 q = a.src[s];
-                const double ex = q.x - qx, ey = q.y - qy, ez = q.z - qz;
-                if (ex * ex + ey * ey + ez * ez < r2)
-                    ok = density_terms(neighbour_at(a, s), qx, qy, qz, kern, v, &inside);
-            }
-            const uint64_t om = __ballot(ok);
-            if (om == 0) return;
-            const int n_ok = __builtin_popcountll(om);
-            if (nbuf + n_ok > 64) flush();
-            if (ok) {
-                const int pos = nbuf + lanes_under(om);
-#pragma unroll
-                for (int c = 0; c < kTerms; ++c) s_v[c][pos] = v[c];
-            }
-            n_in += __builtin_popcountll(__ballot(ok && inside));
-            nbuf += n_ok;
-        };
-        // the admitted leaves run (bit j: child cf + j), their particles in slot order
-        auto leaves = [&](int cf, uint64_t run) {
-            int plo = 0, cnt = 0, off = 0, total = 0;
-            if ((run >> lane) & 1ull) {
-                const SRec c = a.nodes.srec[cf + lane];
-                plo = ~c.link;
-                cnt = c.span - plo;
-            }
-            for (uint64_t r = run; r != 0; r &= r - 1) {
-                const int j = (int)__builtin_ctzll(r);
-                if (lane == j) off = total;
-                total += __builtin_amdgcn_readlane(cnt, j);
-            }
-            for (int g0 = 0; g0 < total; g0 += 64) {
-                const int g = g0 + lane;
-                int s = -1;
-                for (uint64_t r = run; r != 0; r &= r - 1) {
-                    const int j = (int)__builtin_ctzll(r);
-                    const int o = __builtin_amdgcn_readlane(off, j);
-                    if (g >= o && g < o + __builtin_amdgcn_readlane(cnt, j))
-                        s = __builtin_amdgcn_readlane(plo, j) + (g - o);
-                }
-                take(s);
-            }
-        };
-        // A node whose box (its centre and half side as the node test reads them, so the cells
-        // below it too) lies inside the sphere, by a margin above the float rounding of node
-        // centres: every node below it is admitted, so the walk would test each of its particles
-        // in slot order. They are a contiguous slot range, taken 64 at a time instead.
-        auto inside_sphere = [&](const SRec& nr) -> bool {
-            const double hf = (double)nr.half;
-            const double ax = fabs((double)nr.cx - qx) + hf, ay = fabs((double)nr.cy - qy) + hf,
-                         az = fabs((double)nr.cz - qz) + hf;
-            const double m = 1e-6 * (fabs((double)nr.cx) + fabs((double)nr.cy) +
-                                     fabs((double)nr.cz));
-            const double hm = h * (1.0 - 1e-12) - m;
-            return hm > 0 && ax * ax + ay * ay + az * az < hm * hm;
-        };
-        for (int r0 = 0; r0 < r_count; r0 += 64) {
-            // the children of the node being walked (first index; lane masks of those admitted
-            // and not yet visited, and of those that are leaves) and the stack of the same above
-            // it, entry d in lane d
-            int cf = r_first + r0;
-            uint64_t cm, lm;
-            {
-                bool hit = false, leaf = false;
-                if (lane < min(64, r_count - r0)) {
-                    const SRec c = a.nodes.srec[cf + lane];
-                    hit = admits(c);
-                    leaf = c.link < 0;
-                }
-                cm = __ballot(hit);
-                lm = __ballot(hit && leaf);
-            }
-            int sp = 0, stf = 0, sml = 0, smh = 0, sll = 0, slh = 0;
-            for (;;) {
-                if (cm == 0) {
-                    if (sp == 0) break;
-                    --sp;
-                    cf = __builtin_amdgcn_readlane(stf, sp);
-                    cm = ((uint64_t)(uint32_t)__builtin_amdgcn_readlane(smh, sp) << 32) |
-                         (uint64_t)(uint32_t)__builtin_amdgcn_readlane(sml, sp);
-                    lm = ((uint64_t)(uint32_t)__builtin_amdgcn_readlane(slh, sp) << 32) |
-                         (uint64_t)(uint32_t)__builtin_amdgcn_readlane(sll, sp);
-                    continue;
-                }
-                const uint64_t inner = cm & ~lm;
-                if ((cm & (0 - cm) & lm) != 0) {
-                    // the next child is a leaf: it and the leaves after it up to the next
-                    // interior child
-                    const uint64_t run = inner ? (cm & ((inner & (0 - inner)) - 1)) : cm;
-                    cm &= ~run;
-                    leaves(cf, run);
-                    continue;
-                }
-                // an interior child: its admitted children are walked before its remaining
-                // siblings, which wait on the stack
-                const int node = cf + (int)__builtin_ctzll(cm);
-                cm &= cm - 1;
-                const SRec nr = ld_const(a.nodes.srec + node);
-                if (inside_sphere(nr)) {
-                    const WNode w = ld_const(a.wn + node);
-                    for (int s0 = w.plo; s0 < w.phi; s0 += 64)
-                        take(s0 + lane < w.phi ? s0 + lane : -1);
-                    continue;
-                }
-                bool hit = false, leaf = false;
-                if (lane < nr.span) {
-                    const SRec c = a.nodes.srec[nr.link + lane];
-                    hit = admits(c);
-                    leaf = c.link < 0;
-                }
-                const uint64_t om = __ballot(hit);
-                if (om == 0) continue;
-                if (cm != 0) {
-                    const bool top = lane == sp;
-                    stf = top ? cf : stf;
-                    sml = top ? (int)(uint32_t)cm : sml;
-                    smh = top ? (int)(uint32_t)(cm >> 32) : smh;
-                    sll = top ? (int)(uint32_t)lm : sll;
-                    slh = top ? (int)(uint32_t)(lm >> 32) : slh;
-                    ++sp;
-                }
-                cf = nr.link;
-                cm = om;
-                lm = __ballot(hit && leaf);
-            }
-        }
-        flush();
         DensSums S;
-#pragma unroll
-        for (int c = 0; c < kTerms; ++c) S.s[c] = __shfl(acc, c);
-        S.n_inside = n_in;
-        if (lane == 0) density_update(a, e, t, p, h, it, S);
+        far_sums(a, qx, qy, qz, h, s_v, &S);
+        if (threadIdx.x == 0) density_update(a, e, t, p, h, it, S);
         if (!LOOP) break;
         __syncthreads(); // the update's state, written by lane 0, for every lane
         if (a.keep[e] == 0) break;
     }
 }
 
-// The last kLoopTargets targets, a wavefront each (target a.act[e] for block e), iterated to the
-// end. The wave collects its target's candidates once, out to kNearMargin times the radius, up to
-// 64 nodes in depth-first order at a time, and keeps them in registers (candidate 64 k + lane), in
-// slot order: a step is then a distance test and the terms of those inside, without the tree, until
-// the radius outgrows the collection (one of a radius above zero). (Targets that run to the 100-iteration cap, whose walks one
-// node at a time set the launch's time, took 39 us a step before, and 2-3 us now.) When some
-// particle has left its cell the candidates are collected for each step at its own radius, under
-// the reference's node tests. A sphere of more than kNearMax candidates is left to k_density_far
-// (appended to far_list, its state in memory).
+// The last targets, a wavefront each (target a.act[e] for block e), iterated to the end. The wave
+// collects its target's candidates once, out to kNearMargin times the radius, up to 64 nodes in
+// depth-first order at a time, and keeps them in registers (candidate 64 k + lane), in slot order: a
+// step is then a distance test and the terms of those inside, without the tree, until the radius
+// outgrows the collection (one of a radius above zero). (Targets that run to the 100-iteration cap,
+// whose walks one node at a time set the launch's time, took 39 us a step before, and 2-3 us now.)
+// When some particle has left its cell the candidates are collected for each step at its own radius,
+// under the reference's node tests.
+//
+// A sphere of more than kNearMax candidates is left to k_density_far (appended to far_list, its state
+// in memory), or with FAR takes its steps from far_sums here until it has shrunk: a launch less, but
+// more registers. Whether it will be one is then told in advance, since a collection that overflows
+// is thrown away: at first by the leaf's side, as in the rounds, then from the step before, whose
+// neighbours fill the next sphere in proportion to its volume.
 constexpr int kNearSlots = 4; // candidates a lane holds
 constexpr int kNearMax = 64 * kNearSlots;
 constexpr double kNearMargin = 1.15;
+__host__ __device__ __forceinline__ double near_volume(double g, int dim) { // relative, of g times the radius
+    g *= kNearMargin;
+    return (dim == 3) ? g * g * g : (dim == 2 ? g * g : g);
+}
+template <bool FAR>
 __global__ __launch_bounds__(64, 3) void k_density_near(DensArgs a) {
     // the collection's stack and leaf runs, then a step's packed terms
     __shared__ union {
-        double v[kTerms][65];
+        double v[kTerms][65]; // rows padded so the 12 adding lanes hit distinct banks
         struct {
             int stk[kSphStack], lpre[64], lplo[64];
         } w;
@@ -609,9 +644,14 @@ __global__ __launch_bounds__(64, 3) void k_density_near(DensArgs a) {
     int nc = 0;
     double hc = 0.0;   // the radius the candidates reach
     bool have = false; // they can serve another step
+    bool full = false; // FAR: this step by far_sums
+    if (FAR) {
+        const int ts = a.tslot[t];
+        full = ts >= 0 && st.h > kFarLeaf * a.size[a.slot_leaf[ts]];
+    }
 
     for (;;) {
-        if (!have || !(st.h <= hc)) {
+        if (!full && !(have && st.h <= hc)) {
             // collect: the search at radius hc, its particles tested against the sphere
             hc = (fresh && st.h > 0) ? st.h * kNearMargin : st.h;
             const double c2 = hc * hc;
@@ -626,76 +666,90 @@ __global__ __launch_bounds__(64, 3) void k_density_near(DensArgs a) {
                 nc += __builtin_popcountll(im);
                 return nc <= kNearMax;
             });
-            if (nc > kNearMax) {
+            if (!FAR && nc > kNearMax) {
                 if (lane == 0) {
                     a.h[t] = st.h;
                     a.h_lo[t] = st.lo;
                     a.h_hi[t] = st.hi;
                     a.iter[t] = st.it;
-                    a.keep[e] = 0; // k_density_far takes it to the end
                     a.far_list[atomicAdd(a.n_far, 1u)] = (uint32_t)e;
                 }
                 return;
             }
+            full = nc > kNearMax;
+            have = fresh && st.h > 0; // (a negative radius's next step may be larger in size)
+            __syncthreads();
 #pragma unroll
             for (int k = 0; k < kNearSlots; ++k) {
-                if (64 * k + lane < nc) {
+                if (FAR) {
+                    cx[k] = cy[k] = cz[k] = 0.0;
+                    nb[k] = Neighbour{};
+                }
+                if (!full && 64 * k + lane < nc) {
                     const uint32_t slot = s_cand[64 * k + lane];
                     const double4 q = a.src[slot];
                     cx[k] = q.x; cy[k] = q.y; cz[k] = q.z;
                     nb[k] = neighbour_at(a, slot);
                 }
             }
-            have = fresh && st.h > 0; // (a negative radius's next step may be larger in size)
         }
-        const double r2 = st.h * st.h;
-        Kernel kern;
-        kern.set(st.h, a.n_dims);
-        double acc = 0.0;
-        int n_in = 0, nbuf = 0;
+        DensSums S;
+        if (FAR && full) {
+            have = false;
+            far_sums(a, qx, qy, qz, st.h, s.v, &S);
 #pragma unroll
-        for (int k = 0; k < kNearSlots; ++k) {
-            if (64 * k >= nc) break;
-            double v[kTerms];
-            bool inside = false, ok = false;
-            if (64 * k + lane < nc) {
-                const double ex = cx[k] - qx, ey = cy[k] - qy, ez = cz[k] - qz;
-                if (ex * ex + ey * ey + ez * ez < r2)
-                    ok = density_terms(nb[k], qx, qy, qz, kern, v, &inside);
+            for (int k = 0; k < kNearSlots; ++k) { // (held in no register while far_sums runs)
+                cx[k] = cy[k] = cz[k] = 0.0;
+                nb[k] = Neighbour{};
             }
-            const uint64_t om = __ballot(ok);
-            const int n_ok = __builtin_popcountll(om);
-            if (nbuf + n_ok > 64) {
+        } else {
+            const double r2 = st.h * st.h;
+            Kernel kern;
+            kern.set(st.h, a.n_dims);
+            double acc = 0.0;
+            int n_in = 0, nbuf = 0;
+#pragma unroll
+            for (int k = 0; k < kNearSlots; ++k) {
+                if (64 * k >= nc) break;
+                double v[kTerms];
+                bool inside = false, ok = false;
+                if (64 * k + lane < nc) {
+                    const double ex = cx[k] - qx, ey = cy[k] - qy, ez = cz[k] - qz;
+                    if (ex * ex + ey * ey + ez * ez < r2)
+                        ok = density_terms(nb[k], qx, qy, qz, kern, v, &inside);
+                }
+                const uint64_t om = __ballot(ok);
+                const int n_ok = __builtin_popcountll(om);
+                if (nbuf + n_ok > 64) {
+                    __syncthreads();
+                    acc = add_terms(s.v, lane, nbuf, acc);
+                    nbuf = 0;
+                }
                 __syncthreads();
-                acc = add_terms(s.v, lane, nbuf, acc);
-                nbuf = 0;
+                if (ok) {
+                    const int pos = nbuf + lanes_under(om);
+#pragma unroll
+                    for (int c = 0; c < kTerms; ++c) s.v[c][pos] = v[c];
+                }
+                n_in += __builtin_popcountll(__ballot(ok && inside));
+                nbuf += n_ok;
             }
             __syncthreads();
-            if (ok) {
-                const int pos = nbuf + lanes_under(om);
+            acc = add_terms(s.v, lane, nbuf, acc);
+            __syncthreads();
 #pragma unroll
-                for (int c = 0; c < kTerms; ++c) s.v[c][pos] = v[c];
-            }
-            n_in += __builtin_popcountll(__ballot(ok && inside));
-            nbuf += n_ok;
+            for (int c = 0; c < kTerms; ++c) S.s[c] = __shfl(acc, c);
+            S.n_inside = n_in;
         }
-        __syncthreads();
-        acc = add_terms(s.v, lane, nbuf, acc);
-        __syncthreads();
-        DensSums S;
-#pragma unroll
-        for (int c = 0; c < kTerms; ++c) S.s[c] = __shfl(acc, c);
-        S.n_inside = n_in;
+        const double h = st.h;
         if (density_step(a, t, p, st, S, lane == 0)) break;
+        if (FAR) full = S.n_inside * near_volume(st.h / h, a.n_dims) > (double)kNearMax;
     }
-    if (lane == 0) {
-        a.h[t] = st.h;
-        a.keep[e] = 0;
-    }
+    if (lane == 0) a.h[t] = st.h;
 }
 
-// One step for every active target (see the top of the file): tpw targets per wavefront, lane l
-// holding active entry wave * tpw + l. A target whose radius reaches far beyond its own leaf would
+// One step for every active target (see the top of the file): lane l of wave w holds active entry
+// 64 w + l. A target whose radius reaches far beyond its own leaf would
 // make its wave walk a large part of the tree one node at a time; it is queued for a wave of its
 // own (k_density_far) and takes no part here.
 __global__ __launch_bounds__(64, 3) void k_density_round(DensArgs a) {
@@ -704,8 +758,8 @@ __global__ __launch_bounds__(64, 3) void k_density_round(DensArgs a) {
     const int b = blockIdx.x, nb = gridDim.x;
     const int xcd = b & 7, per = nb >> 3, rem = nb & 7;
     const int wv = xcd * per + min(xcd, rem) + (b >> 3);
-    const int k = wv * a.tpw + lane;
-    const bool live = lane < a.tpw && k < a.n_act;
+    const int k = wv * 64 + lane;
+    const bool live = k < a.n_act;
     const int dim = a.n_dims;
     uint32_t t = 0, p = 0;
     double qx = 0, qy = 0, qz = 0, h = 0;
@@ -820,7 +874,7 @@ __global__ __launch_bounds__(256) void k_density_init(int nt, const uint32_t* __
     act[t] = (uint32_t)t;
 }
 
-// The far targets' entries in the active list: their target positions, for the list path.
+// The far targets' entries in the active list: their target positions.
 __global__ __launch_bounds__(256) void k_density_far_act(int nf, const uint32_t* __restrict__ far,
                                                          const uint32_t* __restrict__ act,
                                                          uint32_t* __restrict__ far_act) {
@@ -828,7 +882,7 @@ __global__ __launch_bounds__(256) void k_density_far_act(int nf, const uint32_t*
     if (j < nf) far_act[j] = act[far[j]];
 }
 
-// The list path's keep flags back into the active list's.
+// The far targets' keep flags back into the active list's.
 __global__ __launch_bounds__(256) void k_density_far_keep(int nf, const uint32_t* __restrict__ far,
                                                           const uint32_t* __restrict__ far_keep,
                                                           uint32_t* __restrict__ keep) {
@@ -1055,24 +1109,24 @@ extern "C" gz_status gz_tree_density(gz_ctx* ctx, const gz_tree* tree, const gz_
     a.src = tree->src;
     a.orderbuf = tree->orderbuf;
 
+    const double cand = des_ngb * near_volume(1.0, n_dims); // a converged target's candidates
+    const bool collect = cand <= kCollectMax;
+    const uint32_t last = (cand <= kCollectMost) ? kLastTargets : kLastTargetsFull;
     // rounds: a target takes at most 100 steps and one last search
     uint32_t n_act = (uint32_t)n_t;
     for (int round = 0; n_act > 0; ++round) {
         if (round > kMaxIter + 1)
             return fail(GZ_ERR_INTERNAL, "gz_tree_density: the solve did not end");
-        // 64 targets per wave while that gives enough waves; fewer (down to one) when the active
-        // targets are too few to occupy the GPU that way (and often far apart, as the last
-        // unconverged targets are). The last few iterate to the end in one launch.
-        int tpw = 64;
-        while (tpw > 1 && (n_act + tpw - 1) / tpw < (uint32_t)kWavesWanted) tpw >>= 1;
         a.act = d_act;
         a.n_act = (int)n_act;
-        a.tpw = tpw;
-        const bool loop = n_act <= kLoopTargets;
+        const bool loop = n_act <= last; // to the end in one launch
         GZ_TRY(fill_zero_u32(d_nfar, 1, st));
-        if (loop) k_density_near<<<n_act, 64, 0, st>>>(a);
-        else k_density_round<<<(n_act + tpw - 1) / tpw, 64, 0, st>>>(a);
+        if (!loop) k_density_round<<<(n_act + 63) / 64, 64, 0, st>>>(a);
+        else if (!collect) k_density_far<true><<<n_act, 64, 0, st>>>(a);
+        else if (n_act <= kNearFar) k_density_near<true><<<n_act, 64, 0, st>>>(a);
+        else k_density_near<false><<<n_act, 64, 0, st>>>(a);
         GZ_HIP(hipGetLastError());
+        if (loop && (!collect || n_act <= kNearFar)) break;
         uint32_t n_far = 0;
         GZ_HIP(hipMemcpyAsync(&n_far, d_nfar, sizeof n_far, hipMemcpyDeviceToHost, st));
         GZ_HIP(hipStreamSynchronize(st));
@@ -1089,10 +1143,11 @@ extern "C" gz_status gz_tree_density(gz_ctx* ctx, const gz_tree* tree, const gz_
             if (loop) k_density_far<true><<<n_far, 64, 0, st>>>(f);
             else k_density_far<false><<<n_far, 64, 0, st>>>(f);
             GZ_HIP(hipGetLastError());
+            if (loop) break; // every target is done
             k_density_far_keep<<<gf, 256, 0, st>>>((int)n_far, d_far, d_fkeep, d_keep);
             GZ_HIP(hipGetLastError());
         }
-        if (loop) break; // every target is done
+        if (loop) break;
         // the targets still active, in their order: kept positions, then their target indices
         GZ_TRY(exclusive_scan_u32(d_keep, d_scan, n_act, d_total, base + o_tmp, st, d_kept));
         uint32_t n_next = 0;
