@@ -404,7 +404,14 @@ __device__ __forceinline__ float h_as_bound(double h) {
 // kNgbRow in a row per query, so that a list is found, counted and ordered in one walk; only
 // queries with longer lists are walked again, straight into their place in the CSR: by a wave each
 // (k_ngb_long) while they are few, else as they were walked first (FILL).
+//
+// A lane gives up a list that reaches kNgbLane entries per query of its wave, and a wave of its own
+// counts and fills it (k_ngb_count, k_ngb_long): alone in its wave, one lane tests a particle at a
+// time. With few queries, one to a wave, each takes the whole wave from the start. ms of 1M Hernquist,
+// by lanes throughout / so: 300 queries of 133,000 neighbours each 742 / 314, of 27 .22 / .18; 30,000
+// of 3,773 715 / 337, of 420 4.2 / 2.8.
 constexpr int kNgbRow = 64;
+constexpr uint32_t kNgbLane = 64;
 // A wave each up to one query in this many. 1M queries, ms a search with a wave each / walked as
 // first, by the share of long lists: Hernquist .0015 1.50 / 1.77, .05 2.04 / 2.25, .11 2.50 / 2.55,
 // .20 3.10 / 2.86; halo + disk .008 1.59 / 1.96, .07 2.30 / 2.54, .13 2.83 / 2.86, .22 3.52 / 3.17.
@@ -420,6 +427,8 @@ struct NgbFwd {
     uint32_t* rows; // kNgbRow per query, or NULL
     const size_t* start;
     uint32_t* found;
+    uint32_t lane_max; // entries from which on a list is a wave's ...
+    uint32_t *big, *n_big; // ... and the queries of these
 };
 
 template <bool FILL>
@@ -434,9 +443,9 @@ __global__ __launch_bounds__(64) void k_ngb_fwd(NgbFwd a) {
     uint32_t* out = nullptr;
     if (FILL) {
         if (mine) {
-            const size_t s = a.start[q];
+            const size_t s = a.start[q], n = a.start[q + 1] - s;
             out = a.found + s;
-            mine = a.start[q + 1] - s > (size_t)(a.rows ? kNgbRow : 0);
+            mine = n > (size_t)(a.rows ? kNgbRow : 0) && n < (size_t)a.lane_max;
         }
         if (__ballot(mine) == 0) return;
     } else if (a.rows && mine) {
@@ -447,7 +456,8 @@ __global__ __launch_bounds__(64) void k_ngb_fwd(NgbFwd a) {
         qx = a.cx[q]; qy = a.cy[q]; qz = a.cz[q];
         r = a.radius[q];
     }
-    const double r2 = mine ? r * r : -1.0;
+    double r2 = mine ? r * r : -1.0;
+    const bool asked = mine;
     const uint32_t room = FILL ? 0xFFFFFFFFu : (a.rows ? (uint32_t)kNgbRow : 0u);
     uint32_t n = 0;
     walk_spheres(a.nodes, mine, qx, qy, qz, r, lds, a.orderbuf, [&](int np, auto allowed) {
@@ -464,8 +474,43 @@ __global__ __launch_bounds__(64) void k_ngb_fwd(NgbFwd a) {
         };
         if (allowed.all) test([](int) { return true; });
         else test(allowed);
+        if (!FILL && n >= a.lane_max) {
+            mine = false;
+            r2 = -1.0;
+        }
     });
-    if (!FILL && mine) a.count[q] = n;
+    if (!FILL && asked) {
+        a.count[q] = n; // (of a list given up: lane_max or more)
+        if (!mine) a.big[atomicAdd(a.n_big, 1u)] = (uint32_t)q;
+    }
+}
+
+// A wave per query, of a list of them (*n_list) or all (NULL): its count, and its row if there are.
+template <bool PACKED>
+__global__ __launch_bounds__(64) void k_ngb_count(NgbFwd a, const uint32_t* __restrict__ list,
+                                                  const uint32_t* __restrict__ n_list) {
+    __shared__ int stk[kSphStack], lpre[64], lplo[64];
+    const int n = list ? (int)*n_list : a.nq;
+    for (int i = blockIdx.x; i < n; i += gridDim.x) {
+        const uint32_t c = list ? list[i] : (uint32_t)i;
+        const double qx = a.cx[c], qy = a.cy[c], qz = a.cz[c], r = a.radius[c];
+        const double r2 = r * r;
+        uint32_t* const row = a.rows ? a.rows + (size_t)c * kNgbRow : nullptr;
+        uint32_t found = 0;
+        walk_sphere<PACKED>(a.nodes, qx, qy, qz, r, stk, lpre, lplo,
+                            [&](bool some, int slot, const double4& p) {
+            const double ex = p.x - qx, ey = p.y - qy, ez = p.z - qz;
+            const bool in = some && ex * ex + ey * ey + ez * ez < r2;
+            const uint64_t im = __ballot(in);
+            if (row && found < (uint32_t)kNgbRow) {
+                const uint32_t at = found + (uint32_t)lanes_under(im);
+                if (in && at < (uint32_t)kNgbRow) row[at] = a.orderbuf[slot];
+            }
+            found += (uint32_t)__builtin_popcountll(im);
+            return true;
+        });
+        if (threadIdx.x == 0) a.count[c] = found;
+    }
 }
 
 // The queries with lists longer than a row, in any order. One atomic per 1,024 queries (an atomic on
@@ -489,15 +534,17 @@ __global__ __launch_bounds__(1024) void k_ngb_longs(int nq, const size_t* __rest
     if (is) longs[s_at + at + lanes_under(m)] = (uint32_t)q;
 }
 
-// A wave per listed query. They lie among shorter ones: with a lane each, the waves that held one
-// or two of them tested every particle of the largest sphere in a lane, and the longest lists' waves
-// set the time.
+// A wave per listed query (of *n_list; NULL: all whose list is no row). They lie among shorter ones:
+// with a lane each, the waves that held one or two of them tested every particle of the largest
+// sphere in a lane, and the longest lists' waves set the time.
 template <bool PACKED>
-__global__ __launch_bounds__(64) void k_ngb_long(NgbFwd a, const uint32_t* __restrict__ longs,
-                                                 int n_longs) {
+__global__ __launch_bounds__(64) void k_ngb_long(NgbFwd a, const uint32_t* __restrict__ list,
+                                                 const uint32_t* __restrict__ n_list) {
     __shared__ int stk[kSphStack], lpre[64], lplo[64];
-    for (int i = blockIdx.x; i < n_longs; i += gridDim.x) {
-        const uint32_t c = longs[i];
+    const int n = list ? (int)*n_list : a.nq;
+    for (int i = blockIdx.x; i < n; i += gridDim.x) {
+        const uint32_t c = list ? list[i] : (uint32_t)i;
+        if (a.start[c + 1] - a.start[c] <= (size_t)(a.rows ? kNgbRow : 0)) continue;
         const double qx = a.cx[c], qy = a.cy[c], qz = a.cz[c], r = a.radius[c];
         const double r2 = r * r;
         size_t at = a.start[c];
@@ -687,6 +734,7 @@ static gz_status ngb_run(gz_ctx* ctx, const gz_tree* tree, const double* cx, con
     DevMem& s = ctx->scratch[10];
     ScratchUse s_use(s);
     const size_t cnt_bytes = ((n_q + 1) * sizeof(uint32_t) + 255) & ~size_t(255);
+    const size_t big_bytes = rev ? 0 : cnt_bytes;
     const size_t tmp_bytes = (256 + scan_tmp_bytes(n_q + 1) + 255) & ~size_t(255);
     // forward: the search nodes, and a row per query unless the caller has room for longer lists
     // (packing reads the whole tree, 75 us at 4M particles: for a few queries it would be most of
@@ -695,13 +743,14 @@ static gz_status ngb_run(gz_ctx* ctx, const gz_tree* tree, const double* cx, con
     size_t srec_bytes = packed ? (size_t)tree->nnodes * sizeof(SRec) : 0;
     const size_t row_bytes = n_q * kNgbRow * sizeof(uint32_t);
     bool rows = !rev && found && cap / kNgbRow <= n_q && row_bytes <= kNgbRowsMax;
+    const size_t need = cnt_bytes + tmp_bytes + big_bytes;
     // (both only when there is memory for them)
-    rows = rows && s.offer(cnt_bytes + tmp_bytes + srec_bytes + row_bytes);
-    if (packed && !rows && !s.offer(cnt_bytes + tmp_bytes + srec_bytes)) {
+    rows = rows && s.offer(need + srec_bytes + row_bytes);
+    if (packed && !rows && !s.offer(need + srec_bytes)) {
         packed = false;
         srec_bytes = 0;
     }
-    GZ_TRY(s.reserve(cnt_bytes + tmp_bytes));
+    GZ_TRY(s.reserve(need));
     uint8_t* b = s.as<uint8_t>();
     uint32_t* count = reinterpret_cast<uint32_t*>(b);
     int* misc = reinterpret_cast<int*>(b + cnt_bytes);
@@ -739,31 +788,45 @@ static gz_status ngb_run(gz_ctx* ctx, const gz_tree* tree, const double* cx, con
     GZ_TRY(fill_zero_u32(reinterpret_cast<uint32_t*>(total64), 4, st));
     NgbFwd f{};
     const unsigned fgrid = (unsigned)a.ngroups;
+    const bool wave_each = a.qpw == 1;
+    auto count_by_waves = [&](const uint32_t* list) -> gz_status {
+        const unsigned grid = (unsigned)std::min<size_t>(n_q, (size_t)waves);
+        if (packed) k_ngb_count<true><<<grid, 64, 0, st>>>(f, list, f.n_big);
+        else k_ngb_count<false><<<grid, 64, 0, st>>>(f, list, f.n_big);
+        GZ_HIP(hipGetLastError());
+        return GZ_OK;
+    };
     if (rev) {
         GZ_TRY(ngb_rev_pass(a, false, waves, st));
     } else {
         GZ_TRY(fill_zero_u32(reinterpret_cast<uint32_t*>(misc), 9, st));
         GZ_TRY(launch_sphere_nodes(
-            tree, tau, packed ? reinterpret_cast<SRec*>(b + cnt_bytes + tmp_bytes) : nullptr,
+            tree, tau, packed ? reinterpret_cast<SRec*>(b + need) : nullptr,
             packed ? misc + 8 : nullptr, &f.nodes, st));
         f.cx = cx; f.cy = cy; f.cz = cz; f.radius = radius;
         f.orderbuf = tree->orderbuf;
         f.nq = a.nq;
         f.qpw = a.qpw;
         f.count = count;
-        f.rows = rows ? reinterpret_cast<uint32_t*>(b + cnt_bytes + tmp_bytes + srec_bytes)
-                      : nullptr;
+        f.rows = rows ? reinterpret_cast<uint32_t*>(b + need + srec_bytes) : nullptr;
         f.start = start;
         f.found = found;
-        k_ngb_fwd<false><<<fgrid, 64, 0, st>>>(f);
+        f.lane_max = kNgbLane * (uint32_t)a.qpw;
+        f.big = reinterpret_cast<uint32_t*>(b + cnt_bytes + tmp_bytes);
+        f.n_big = reinterpret_cast<uint32_t*>(misc + 3);
+        if (wave_each) GZ_TRY(count_by_waves(nullptr));
+        else k_ngb_fwd<false><<<fgrid, 64, 0, st>>>(f);
         GZ_HIP(hipGetLastError());
     }
-    k_sum_counts<<<(unsigned)std::min<size_t>(256, (n_q + 255) / 256), 256, 0, st>>>(
-        (int)n_q, count, total64, max_count, (uint32_t)kNgbRow);
-    GZ_HIP(hipGetLastError());
-    // offsets: exclusive scan of the counts (count[n_q] = 0 gives the total at start[n_q])
     uint32_t tot32 = 0;
-    {
+    int h_status = 0;
+    unsigned long long h_total = 0;
+    uint32_t h_most[2] = {0, 0}; // the longest list, the lists longer than a row
+    auto offsets = [&]() -> gz_status {
+        k_sum_counts<<<(unsigned)std::min<size_t>(256, (n_q + 255) / 256), 256, 0, st>>>(
+            (int)n_q, count, total64, max_count, (uint32_t)kNgbRow);
+        GZ_HIP(hipGetLastError());
+        // exclusive scan of the counts (count[n_q] = 0 gives the total at start[n_q])
         DevMem& o = ctx->scratch[11];
         GZ_TRY(o.reserve((n_q + 1) * sizeof(uint32_t)));
         GZ_TRY(exclusive_scan_u32(count, o.as<uint32_t>(), n_q + 1, nullptr,
@@ -773,14 +836,18 @@ static gz_status ngb_run(gz_ctx* ctx, const gz_tree* tree, const double* cx, con
         GZ_HIP(hipGetLastError());
         GZ_HIP(hipMemcpyAsync(&tot32, o.as<uint32_t>() + n_q, sizeof tot32,
                               hipMemcpyDeviceToHost, st));
+        GZ_HIP(hipMemcpyAsync(h_most, max_count, sizeof h_most, hipMemcpyDeviceToHost, st));
+        GZ_HIP(hipMemcpyAsync(&h_status, a.status, sizeof h_status, hipMemcpyDeviceToHost, st));
+        GZ_HIP(hipMemcpyAsync(&h_total, total64, sizeof h_total, hipMemcpyDeviceToHost, st));
+        GZ_HIP(hipStreamSynchronize(st));
+        return GZ_OK;
+    };
+    GZ_TRY(offsets());
+    if (!rev && !wave_each && h_most[0] >= f.lane_max) { // some were given up
+        GZ_TRY(count_by_waves(f.big));
+        GZ_TRY(fill_zero_u32(reinterpret_cast<uint32_t*>(total64), 4, st));
+        GZ_TRY(offsets());
     }
-    int h_status = 0;
-    unsigned long long h_total = 0;
-    uint32_t h_most[2] = {0, 0}; // the longest list, the lists longer than a row
-    GZ_HIP(hipMemcpyAsync(h_most, max_count, sizeof h_most, hipMemcpyDeviceToHost, st));
-    GZ_HIP(hipMemcpyAsync(&h_status, a.status, sizeof h_status, hipMemcpyDeviceToHost, st));
-    GZ_HIP(hipMemcpyAsync(&h_total, total64, sizeof h_total, hipMemcpyDeviceToHost, st));
-    GZ_HIP(hipStreamSynchronize(st));
     if (h_status & 1)
         return fail(GZ_ERR_INTERNAL, "%s: a search stack outgrew %d entries", who,
                     stack_cap);
@@ -797,18 +864,24 @@ static gz_status ngb_run(gz_ctx* ctx, const gz_tree* tree, const double* cx, con
                 (int)n_q, start, f.rows, found);
             GZ_HIP(hipGetLastError());
         }
-        if (rows && h_long > 0 && h_long <= n_q / kNgbFew) {
+        auto by_waves = [&](const uint32_t* list, const uint32_t* n_list, size_t most) {
+            const unsigned grid = (unsigned)std::min<size_t>(most, (size_t)waves);
+            if (packed) k_ngb_long<true><<<grid, 64, 0, st>>>(f, list, n_list);
+            else k_ngb_long<false><<<grid, 64, 0, st>>>(f, list, n_list);
+        };
+        if (wave_each) {
+            if (!rows || h_long > 0) by_waves(nullptr, nullptr, n_q);
+        } else if (rows && h_long > 0 && h_long <= n_q / kNgbFew) {
             // (the counts are in the offsets: their array takes the list)
-            k_ngb_longs<<<(unsigned)((n_q + 1023) / 1024), 1024, 0, st>>>(
-                (int)n_q, start, count, reinterpret_cast<uint32_t*>(misc + 2));
-            const unsigned grid = (unsigned)std::min<size_t>(h_long, (size_t)waves);
-            if (packed) k_ngb_long<true><<<grid, 64, 0, st>>>(f, count, (int)h_long);
-            else k_ngb_long<false><<<grid, 64, 0, st>>>(f, count, (int)h_long);
-            GZ_HIP(hipGetLastError());
+            uint32_t* n_longs = reinterpret_cast<uint32_t*>(misc + 2);
+            k_ngb_longs<<<(unsigned)((n_q + 1023) / 1024), 1024, 0, st>>>((int)n_q, start, count,
+                                                                          n_longs);
+            by_waves(count, n_longs, h_long);
         } else if (!rows || h_long > 0) {
             k_ngb_fwd<true><<<fgrid, 64, 0, st>>>(f);
-            GZ_HIP(hipGetLastError());
+            if (h_max >= f.lane_max) by_waves(f.big, f.n_big, n_q);
         }
+        GZ_HIP(hipGetLastError());
         GZ_HIP(hipStreamSynchronize(st));
         return GZ_OK;
     }

@@ -84,9 +84,10 @@ struct SphereAllowed {
 
 // Walks the tree once for the spheres (qx, qy, qz, h) of the lanes with `mine`, and calls
 // chunk(np, allowed) on the particles of the leaves that some sphere may reach, in slot order, up
-// to 64 at a time in s.p and s.id (their slots, or ids[slot]). Every lane of the wave calls it.
+// to 64 at a time in s.p and s.id (their slots, or ids[slot]). Every lane of the wave calls it; chunk
+// may clear a lane's `mine`, whose sphere then keeps no node.
 template <class Chunk>
-__device__ __forceinline__ void walk_spheres(const SphereNodes& a, bool mine, double qx, double qy,
+__device__ __forceinline__ void walk_spheres(const SphereNodes& a, bool& mine, double qx, double qy,
                                              double qz, double h, SphereLds& s,
                                              const uint32_t* ids, Chunk&& chunk) {
     const int lane = threadIdx.x & 63;
