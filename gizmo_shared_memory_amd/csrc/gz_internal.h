@@ -306,7 +306,8 @@ struct gz_tree {
     double root_box[4] = {0, 0, 0, 0};
     double root_com[3] = {0, 0, 0}, root_mass = 0; // the root node's moments
     std::vector<int> level_begin; // node ids of level L are [level_begin[L], level_begin[L+1])
-    int* level_begin_dev = nullptr; // the same table on the device (kMaxLevel + 2 entries)
+    // the same table on the device (any level to kMaxLevel + 1; two entries more are the build's)
+    int* level_begin_dev = nullptr;
     int n_clusters = 1;             // independent trees (a forest); their roots are nodes 0..nc-1
     uint32_t* cluster_start_dev = nullptr; // forest: particle offsets of the clusters (nc + 1)
     gz_build_times times = {};

@@ -321,8 +321,6 @@ __global__ __launch_bounds__(64) void k_ngb_finish(int nq, const size_t* __restr
     }
 }
 
-
-
 // Some lists too long for the LDS sort: every list sorted at once by a device radix sort of
 // (query << 32 | slot) keys, which keeps each query's range of the CSR and does not slow down on
 // long lists (lists that all fit the LDS sort are faster in k_ngb_finish; past kFinishLds it
@@ -416,7 +414,9 @@ constexpr uint32_t kNgbLane = 64;
 // first, by the share of long lists: Hernquist .0015 1.50 / 1.77, .05 2.04 / 2.25, .11 2.50 / 2.55,
 // .20 3.10 / 2.86; halo + disk .008 1.59 / 1.96, .07 2.30 / 2.54, .13 2.83 / 2.86, .22 3.52 / 3.17.
 constexpr int kNgbFew = 8;
-constexpr size_t kNgbRowsMax = size_t(1) << 30; // bytes of rows beyond which every list is walked twice
+// Rows take at most so many bytes (4,194,304 queries), beyond which every list is walked twice: of 6M
+// Hernquist, that many queries take 4.1 ms and one more 6.6 (10.3 for 4.3M with the separate sort).
+constexpr size_t kNgbRowsMax = size_t(1) << 30;
 
 struct NgbFwd {
     SphereNodes nodes;
@@ -736,9 +736,10 @@ static gz_status ngb_run(gz_ctx* ctx, const gz_tree* tree, const double* cx, con
     const size_t cnt_bytes = ((n_q + 1) * sizeof(uint32_t) + 255) & ~size_t(255);
     const size_t big_bytes = rev ? 0 : cnt_bytes;
     const size_t tmp_bytes = (256 + scan_tmp_bytes(n_q + 1) + 255) & ~size_t(255);
-    // forward: the search nodes, and a row per query unless the caller has room for longer lists
-    // (packing reads the whole tree, 75 us at 4M particles: for a few queries it would be most of
-    // the search)
+    // forward: the search nodes, and a row per query unless the caller has room for more than a row
+    // each (such lists would nearly all be walked again; a caller with more room than its lists
+    // need walks twice too: 1M of 27 entries 2.2 ms instead of 1.3) (packing reads the whole tree,
+    // 75 us at 4M particles: for a few queries it would be most of the search)
     bool packed = !rev && n_q >= tree->n_live / 16;
     size_t srec_bytes = packed ? (size_t)tree->nnodes * sizeof(SRec) : 0;
     const size_t row_bytes = n_q * kNgbRow * sizeof(uint32_t);

@@ -1,5 +1,5 @@
-// Device-wide primitives used by the tree build: an exclusive scan and a stable LSD radix sort of
-// (64-bit key, 32-bit value) pairs. Both are memory-bound at the sizes of large trees (>= 1M
+// Device-wide primitives: an exclusive scan and a stable LSD radix sort of (64-bit key, 32-bit value)
+// pairs. Both are memory-bound at the sizes of large trees (>= 1M
 // keys), where one launch has a thousand workgroups, and bound by their launches below that.
 #include <algorithm>
 

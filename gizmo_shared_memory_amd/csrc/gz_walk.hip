@@ -1270,13 +1270,20 @@ gz_status launch_walk(const WalkArgs& a, bool fp64, bool count, hipStream_t st) 
     } else if (count) {
         k_walk<false, true, false><<<grid, 64, 0, st>>>(a);
     } else if (a.persistent && a.waves_per_cu == 0) {
-        // Waves per group: the fewer groups there are for the GPU's 5,120 waves, the more. All
-        // targets of n particles, ms a force call (tree build included) with 1 | 2 | 4 | 8 waves:
-        // 4,000 .86 | .77 | .72 | .69; 30,000 2.42 | 1.94 | 1.60 | 1.42 (650 groups); 65,536 2.98 |
-        // 2.37 | 1.98 | 1.83; 131,072 1.06 | .98 | 1.00 | 1.13; 262,147 1.20 | 1.20 | 1.29 | 1.54;
-        // 1M (walk only) .84 | .99 | 1.40 | 2.26. Of 1M particles 64 targets .50 | .45 | .41 |
-        // .40; 4,099 .65 | .54 | .47 | .46; 30,000 .70 | .59 | .59 | .70; 200,000 .83 | .84 | .99 |
-        // 1.35. Eight up to a tenth of the waves, four up to 0.4, two up to their number.
+        // Waves per group: the fewer groups there are for the GPU's 5,120 waves, the more. ms with
+        // 1 | 2 | 4 | 8 waves of force calls (tree build included) with every particle a target:
+        //   Hernquist    4,000    .86 |  .77 |  .72 |  .69   (some 90 groups)
+        //   Hernquist   30,000   2.42 | 1.94 | 1.60 | 1.42   (650 groups, one of them meets all)
+        //   halo + disk 65,536   2.98 | 2.37 | 1.98 | 1.83   (1,400 groups, the same)
+        //   Hernquist  131,072   1.06 |  .98 | 1.00 | 1.13
+        //   Hernquist  262,147   1.20 | 1.20 | 1.29 | 1.54
+        // and of substeps of a 1M halo + disk with so many targets:
+        //          64 .50 | .45 | .41 | .40      4,099 .65 | .54 | .47 | .46
+        //      30,000 .70 | .59 | .59 | .70    200,000 .83 | .84 | .99 | 1.35
+        // (all 1M, the walk alone: .84 | .99 | 1.40 | 2.26). A launch's time is its slowest group's or
+        // its work's; the count of groups tells the second only, and the lines are set by the
+        // substeps, where it is the work's: eight up to a tenth of the waves, four up to 0.4, two
+        // up to their number. A caller that sets waves_per_cu keeps one wave a group.
         int waves = 0;
         GZ_TRY(persistent_waves(&waves));
         const long long n = a.groups_expected;
