@@ -67,12 +67,12 @@ struct DevBlock {
 // come in sizes an eighth of a power of two apart, so that a tree that grows a little from one
 // rebuild to the next finds its blocks again (exact sizes left each tree's blocks useless to the
 // next: a rebuild of a 4M tree that grows by 0.1% a time took 6.6 to 27 ms once the cache was full
-// of them, now 2.6). It holds at most kBytes and kBlocks (nothing outside the library can ask for
-// them back; a rebuild of 16.8M particles, whose blocks are more, loses .1 of 5.1 ms to the bound,
-// of 33.6M 1.7 of 11.4); beyond that the blocks put longest ago go back to
-// the device, and everything does when its context is destroyed or an allocation of the context
-// finds no memory. Trees may be freed by another thread than the one that builds (the list is locked), and
-// after their context (they share the cache's ownership; it then keeps nothing).
+// of them, now 2.6). It holds at most kBytes and kBlocks, since nothing outside the library can ask
+// for them back (a rebuild of 16.8M particles, whose blocks are more, loses .1 of 5.1 ms to the
+// bound, of 33.6M 1.7 of 11.4); beyond that the blocks put longest ago go back to the device, and
+// everything does when its context is destroyed or an allocation of the context finds no memory.
+// Trees may be freed by another thread than the one that builds (the list is locked), and after
+// their context (they share the cache's ownership; it then keeps nothing).
 class BlockCache {
 public:
     static constexpr size_t kBytes = size_t(2) << 30;

@@ -618,7 +618,8 @@ __global__ __launch_bounds__(64) void k_density_far(DensArgs a) {
 constexpr int kNearSlots = 4; // candidates a lane holds
 constexpr int kNearMax = 64 * kNearSlots;
 constexpr double kNearMargin = 1.15;
-__host__ __device__ __forceinline__ double near_volume(double g, int dim) { // relative, of g times the radius
+// The volume out to which candidates are collected for a sphere of g times the radius, over this one's.
+__host__ __device__ __forceinline__ double near_volume(double g, int dim) {
     g *= kNearMargin;
     return (dim == 3) ? g * g * g : (dim == 2 ? g * g : g);
 }

@@ -111,7 +111,7 @@ def test_density_without_room_for_its_copy(gz, P):
 
 
 def test_search_without_room_for_rows_or_nodes(gz, P):
-    """732 MB of rows, some 30 MB of nodes."""
+    """732 MB of rows, some 22 MB of nodes."""
     def prepare(c):
         T = gz.build(P, ctx=c)
         at = T.device_orderbuf().view(torch.int32).long()
@@ -119,4 +119,4 @@ def test_search_without_room_for_rows_or_nodes(gz, P):
         r = torch.full((N,), 0.01, dtype=torch.float64, device="cuda")
         return lambda: [v.view(torch.int32 if v.dtype == torch.uint32 else v.dtype).cpu().numpy()
                         for v in gz.ngb_search(T, q, r)]
-    _limited(gz, prepare, (400 * MB, 748 * MB))
+    _limited(gz, prepare, (400 * MB, 742 * MB))
